@@ -239,6 +239,8 @@ struct pdk_spec_s
     bool uploaded = false, built = false, inited = false;
     bool lattice_rows = false; // device order is lattice rows (else Morton)
     int32_t unroll = -1;       // force-pass variant (tuning knob): -1 default, 0 row windows, 1/2/4/8 gathers
+    bool coords_plain = false; // every coordinate is zero or within [2^-100, 2^100)
+    bool vols_plain = false;   // every volume is within [2^-150, 2^150)
     bool vol_uniform = false;  // every particle has volume vol_value
     double vol_value = 0.0;
     bool any_nofail = false;
@@ -345,6 +347,33 @@ struct pdk_spec_s
         return step_graph[c];
     }
 
+    // Whether the FP64 row passes may take the shared-reciprocal arithmetic
+    // (rootRecip, divBy): with lattice vectors within [2^-60, 2^60], volumes,
+    // c V and the LPS coefficients as tested here, u, x and T zero or within
+    // [2^-100, 2^100) and lpsA, lpsB zero or within [2^-200, 2^200), a bond's
+    // nonzero terms satisfy |s| >= 2^-54 (2^-266 with a thermal strain),
+    // |r_k| >= 2^-205, coeff >= 2^-570, so every quotient and remainder is
+    // above 2^-930 and, with |coeff| <= 2^600, below 2^930.
+    bool plainRange() const
+    {
+        auto within = []( double a, double lo, double hi ) { return std::fabs( a ) >= lo && std::fabs( a ) < hi; };
+        auto zeroOr = [&]( double a, double lo, double hi ) { return a == 0.0 || within( a, lo, hi ); };
+        if ( !coords_plain || !vols_plain || slot.slots <= 0 )
+            return false;
+        for ( int dd = 0; dd < 3; dd++ )
+            if ( !within( lat_h[dd], 0x1p-60, 0x1p60 ) && lat_dims[dd] > 1 )
+                return false;
+        if ( !within( d.horizon, 0x1p-60, 0x1p60 ) )
+            return false;
+        bool ok = lps() || within( k.c, 0x1p-150, 0x1p150 );
+        ok = ok && zeroOr( k.theta_coeff, 0x1p-150, 0x1p150 ) && zeroOr( k.s_coeff, 0x1p-150, 0x1p150 );
+        ok = ok && zeroOr( d.alpha, 0x1p-60, 0x1p60 ) && zeroOr( d.temp0, 0x1p-100, 0x1p100 );
+        ok = ok && zeroOr( k.thermal_coeff, 0x1p-150, 0x1p150 );
+        for ( int t = 0; pair_tables && t < 16; t++ )
+            ok = ok && zeroOr( mat_c[t], 0x1p-150, 0x1p150 );
+        return ok;
+    }
+
     void pushArgs()
     {
         dropGraphs();
@@ -357,6 +386,7 @@ struct pdk_spec_s
         h.f = f.as<double>();
         h.vol = vol.as<double>();
         h.rho = rho.as<double>();
+        h.plain_range = plainRange() ? 1 : 0;
         h.nofail = nofail.as<uint8_t>();
         h.bcflag = bcflag.as<uint8_t>();
         h.body = body ? body.as<double>() : nullptr;
@@ -968,12 +998,24 @@ int pdk_spec_upload( pdk_spec s, const double* x, const double* u, const double*
         // particle spacing (cube root of the mean volume).
         double lo[3] = { x[0], x[1], x[2] };
         double vsum = 0.0;
+        // magnitudes, for the FP64 row passes' arithmetic (plainRange)
+        double cmin = 1.0, cmax = 1.0, vmin = vol[0], vmax = vol[0];
         for ( int64_t i = 0; i < n; i++ )
         {
             for ( int dd = 0; dd < 3; dd++ )
-                lo[dd] = std::min( lo[dd], x[3 * i + dd] );
+            {
+                const double c = x[3 * i + dd];
+                lo[dd] = std::min( lo[dd], c );
+                const double a = c == 0.0 ? 1.0 : std::fabs( c );
+                cmin = std::min( cmin, a );
+                cmax = std::max( cmax, a );
+            }
             vsum += vol[i];
+            vmin = std::min( vmin, vol[i] );
+            vmax = std::max( vmax, vol[i] );
         }
+        s->coords_plain = cmin >= 0x1p-100 && cmax < 0x1p100;
+        s->vols_plain = vmin >= 0x1p-150 && vmax < 0x1p150;
         double h = std::cbrt( vsum / n );
         if ( !( h > 0 ) || !std::isfinite( h ) )
             h = 1.0;

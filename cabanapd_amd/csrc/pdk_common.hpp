@@ -137,6 +137,10 @@ struct PDArgs
     const uint32_t* rowstart; // bit q set: slot q starts a row (9 words), or null
     int32_t nrows;          // 0: no row table
     int32_t lat_n[3];       // lattice extent (stencil-slot form)
+    // FP64 row passes: positions, volumes and constants are within the ranges
+    // for which the shared-reciprocal bond arithmetic gives the general
+    // code's bits (the rows test displacements themselves)
+    int32_t plain_range;
     // Multi-material specimens (FP64 gather passes): material of each
     // particle (null: one material), the PMB coefficient and the critical
     // stretch coefficient of each material pair [4 a + b], and each

@@ -276,6 +276,112 @@ __device__ __forceinline__ void linearized32g( double xi0, double xi1, double xi
     linearized32( gx, gy, gz, g2 * xinv, xinv, ui0, ui1, ui2, uj0, uj1, uj2, b );
 }
 
+// ---------------------------------------------------------------------------
+// The FP64 bond arithmetic without the range handling of the compiler's
+// square root and division (the row-window passes).  A bond takes two roots
+// and four divisions by them; the compiler's forms scale each operand into
+// range, iterate and fix up the special cases, every division from a
+// reciprocal of its own (117 VALU instructions per slot of the PMB pass).
+// Here one reciprocal square root starts both the root and the reciprocal of
+// the root (Goldschmidt's iteration, then Newton's), and the divisions by one
+// divisor share it, each corrected by its exact remainder (Markstein):
+// the same iterations, so the results are the correctly rounded ones, the
+// same bits.  That holds
+//   - for operands whose intermediate values neither overflow nor lose bits
+//     to underflow: PDArgs::plain_range (lattice, constants) and the rows'
+//     own test of the staged values (kPlainExp) see to that, together with
+//     the coefficient's bound plainLimit;
+//   - for roots that are neither zero, infinite nor NaN: those make the
+//     stretch NaN, and with it the coefficient;
+//   - for divisors other than 2^k (2 - 2^-52), the one mantissa whose
+//     reciprocal Newton's iteration misses by an ulp: lastBits finds every
+//     divisor whose low word is all ones.
+// A row in which a lane fails one of them is evaluated again by the general
+// code, from the sums as they were before the row.
+// (checked on the GPU against IEEE results: 1e8 roots and quotients, half of
+// them with mantissas within 16 ulp of a power of two, no difference but for
+// the excluded divisors.  The PMB fracture slot takes 75 VALU instructions;
+// 25 steps of the 1.44M-particle plate with their download 28.2 -> 23.6 ms,
+// 50 steps of a 41^3 cube 4.23 -> 3.52 ms, with the LPS model 8.50 -> 7.48.)
+// ---------------------------------------------------------------------------
+constexpr int kPlainExp = 100;   // staged u, x and T: zero or 2^-100 <= |.| < 2^100
+constexpr int kPlainExpAB = 200; // staged lpsA, lpsB: zero or 2^-200 <= |.| < 2^200
+
+struct Root64
+{
+    double r, y; // correctly rounded sqrt(a), and 1 / r to within an ulp
+};
+__device__ __forceinline__ Root64 rootRecip( double a )
+{
+#pragma clang fp contract( off )
+    const double y0 = __builtin_amdgcn_rsq( a );
+    const double g0 = a * y0;
+    const double h0 = 0.5 * y0;
+    const double e = fma( -h0, g0, 0.5 );
+    const double g1 = fma( g0, e, g0 );
+    const double h1 = fma( h0, e, h0 );
+    const double g2 = fma( fma( -g1, g1, a ), h1, g1 );
+    Root64 o;
+    o.r = fma( fma( -g2, g2, a ), h1, g2 );
+    const double y = h1 + h1;
+    o.y = fma( y, fma( -o.r, y, 1.0 ), y );
+    return o;
+}
+// The reciprocal of a divisor that is no root (a particle's m).
+__device__ __forceinline__ double recip64( double b )
+{
+    double y = __builtin_amdgcn_rcp( b );
+    y = fma( y, fma( -b, y, 1.0 ), y );
+    return fma( y, fma( -b, y, 1.0 ), y );
+}
+// a / b, y = 1 / b to within an ulp
+__device__ __forceinline__ double divBy( double a, double b, double y )
+{
+#pragma clang fp contract( off )
+    const double q = a * y;
+    return fma( fma( -b, q, a ), y, q );
+}
+__device__ __forceinline__ uint32_t lowWord( double a )
+{
+    return static_cast<uint32_t>( __builtin_bit_cast( uint64_t, a ) );
+}
+// Every finite nonzero argument has magnitude in [2^-(lim+1), 2^lim) (infinities and
+// NaN pass: they reach the coefficient as NaN).
+__device__ __forceinline__ void expRange( double a, int& lo, int& hi )
+{
+    const int e = __builtin_amdgcn_frexp_exp( a );
+    lo = min( lo, e );
+    hi = max( hi, e );
+}
+
+struct Fast64
+{
+    double xi, r, s, rx, ry, rz, yxi, yr;
+};
+// getDistance64 with shared reciprocals.
+__device__ __forceinline__ void getDistanceFast( double xi0, double xi1, double xi2, double ui0, double ui1,
+                                                 double ui2, double xj0, double xj1, double xj2, double uj0,
+                                                 double uj1, double uj2, Fast64& b )
+{
+#pragma clang fp contract( off )
+    const double xi_x = xj0 - xi0;
+    const double eta_u = uj0 - ui0;
+    const double xi_y = xj1 - xi1;
+    const double eta_v = uj1 - ui1;
+    const double xi_z = xj2 - xi2;
+    const double eta_w = uj2 - ui2;
+    b.rx = xi_x + eta_u;
+    b.ry = xi_y + eta_v;
+    b.rz = xi_z + eta_w;
+    const Root64 r = rootRecip( b.rx * b.rx + b.ry * b.ry + b.rz * b.rz );
+    const Root64 x = rootRecip( xi_x * xi_x + xi_y * xi_y + xi_z * xi_z );
+    b.r = r.r;
+    b.yr = r.y;
+    b.xi = x.r;
+    b.yxi = x.y;
+    b.s = divBy( b.r - b.xi, b.xi, b.yxi );
+}
+
 // Uniform per-wave access to the spec of this wave's slice.
 struct WaveCtx
 {
@@ -911,6 +1017,7 @@ kForceRows( const PDArgs* __restrict__ specs,
     // in FP64 from the slot's FP64 stencil offset xi; the windows hold u only
     constexpr bool XV = ( PREC == kMixed ) && !kIsLin<MODEL>;
     constexpr int NAB = kIsLps<MODEL> ? 2 : 0;  // staged lpsA, lpsB
+    constexpr bool FAST = ( PREC == kF64 ) && !kIsLin<MODEL>; // shared reciprocals where they give the same bits
     constexpr int KV = 3 + NX + NAB;                // staged vol (GEN)
     constexpr int KNF = KV + 1;                     // staged no-fail flag (GEN)
     constexpr int NC = KV + ( GEN ? 2 : 0 );
@@ -962,6 +1069,7 @@ kForceRows( const PDArgs* __restrict__ specs,
     const double c = A.c;
     const double bcc = A.bcc;
     const float c32 = static_cast<float>( A.c );
+    const double s0near = A.s0 - 0x1p-30 * ( 1.0 + A.s0 );
     const double volu = A.vol_value;
     const float s0f = A.s0f;
     const float bandK = A.bandK;
@@ -1047,6 +1155,39 @@ kForceRows( const PDArgs* __restrict__ specs,
             loadHalf( v1, g + kSlice );
     };
 
+    // FAST: the range test of a row's staged values and of particle i's own
+    const bool plain = FAST && scalarLoad( &A.plain_range ) != 0;
+    int own_lo = 0, own_hi = 0;
+    if constexpr ( FAST )
+    {
+        expRange( ui0, own_lo, own_hi );
+        expRange( ui1, own_lo, own_hi );
+        expRange( ui2, own_lo, own_hi );
+    }
+    auto rowPlain = [&]() {
+        int lo = own_lo, hi = own_hi;
+#pragma unroll
+        for ( int q = 0; q < 3; q++ )
+        {
+            expRange( v0[q], lo, hi );
+            expRange( v1[q], lo, hi );
+        }
+        bool out = lo < -kPlainExp || hi > kPlainExp;
+        if constexpr ( NAB )
+        {
+            int la = 0, ha = 0;
+#pragma unroll
+            for ( int q = 3 + NX; q < 5 + NX; q++ )
+            {
+                expRange( v0[q], la, ha );
+                expRange( v1[q], la, ha );
+            }
+            expRange( Ai, la, ha );
+            expRange( Bi, la, ha );
+            out = out || la < -kPlainExpAB || ha > kPlainExpAB;
+        }
+        return __ballot( out ) == 0;
+    };
     const int nrows = scalarLoad( &A.nrows );
     loadRow( 0 );
     for ( int r = 0; r < nrows; r++ )
@@ -1060,6 +1201,9 @@ kForceRows( const PDArgs* __restrict__ specs,
             if ( PAD || lane < R.y - 1 )
                 wb[k * kWS + kSlice + lane] = v1[k];
         }
+        // a tiny (or huge) displacement in the row: only bonds without force
+        // may take the shared reciprocals
+        const double limit = FAST && rowPlain() ? 0x1p600 : 0.0;
         // LDS operations of one wavefront complete in order; the fences keep
         // the compiler from moving the window reads above the stores.
         __builtin_amdgcn_fence( __ATOMIC_RELEASE, "wavefront" );
@@ -1257,6 +1401,61 @@ kForceRows( const PDArgs* __restrict__ specs,
                 }
             }
         };
+        // FP64 with shared reciprocals: the lanes whose bond the general code
+        // has to evaluate (nothing of such a lane is kept; a bond that breaks
+        // in another lane is recorded, and breaks again if the row is
+        // evaluated again).
+        auto slotFast = [&]( const int t, const double lim ) __attribute__( ( always_inline ) ) {
+            const uint64_t ww = scalarLoad( mw_r + t );
+            const double* __restrict__ wr = wb + lane + t;
+            bool brk = false, gen = false;
+            if ( __builtin_amdgcn_inverse_ballot_w64( ww ) )
+            {
+                const double vj = GEN ? wr[KV * kWS] : volu;
+                Fast64 b;
+                getDistanceFast( xi0, xi1, xi2, ui0, ui1, ui2, wr[3 * kWS], wr[4 * kWS], wr[5 * kWS], wr[0], wr[kWS],
+                                 wr[2 * kWS], b );
+                if constexpr ( FRAC )
+                {
+                    // a bond below s0 by more than rounding cannot break: the
+                    // reference's test runs only in a wave with a stretch near
+                    // s0 or above it
+                    if ( __ballot( b.s >= s0near ) )
+                    {
+                        bool ok = !nf_i;
+                        if constexpr ( !kIsLps<MODEL> && GEN )
+                            ok = ok && wr[KNF * kWS] == 0.0;
+                        brk = criticalStretch64( b.r, b.xi, bcc ) && ok;
+                    }
+                }
+                double coeff;
+                if constexpr ( !kIsLps<MODEL> )
+                    coeff = c * b.s * vj;
+                else
+                {
+                    const double infl = infl1 ? 1.0 / b.xi : 1.0;
+                    coeff = ( Ai + wr[( 3 + NX ) * kWS] + b.s * ( Bi + wr[( 4 + NX ) * kWS] ) ) * infl * b.xi * vj;
+                }
+                gen = !( fabs( coeff ) <= lim ) || max( lowWord( b.r ), lowWord( b.xi ) ) == 0xffffffffu;
+                brk = brk && !gen;
+                if ( !brk )
+                {
+                    fx += divBy( coeff * b.rx, b.r, b.yr );
+                    fy += divBy( coeff * b.ry, b.r, b.yr );
+                    fz += divBy( coeff * b.rz, b.r, b.yr );
+                }
+            }
+            if constexpr ( FRAC )
+            {
+                const uint64_t brkm = __ballot( brk );
+                if ( __builtin_expect( brkm != 0, 0 ) )
+                {
+                    if ( lane == 0 )
+                        bits_r[t] = ww & ~brkm;
+                }
+            }
+            return __ballot( gen );
+        };
         // Mixed forms: the slots of a row (at most kRowMaxSlots) unrolled, so
         // the window reads take immediate offsets and the PMB pass fits 70
         // VGPRs without spills (7 % faster on the fracture plate, 2 % on the
@@ -1270,6 +1469,21 @@ kForceRows( const PDArgs* __restrict__ specs,
         }
         else
         {
+            if constexpr ( FAST )
+            {
+                if ( plain )
+                {
+                    const double fx0 = fx, fy0 = fy, fz0 = fz;
+                    uint64_t bad = 0;
+                    for ( int t = 0; t < R.y; t++ )
+                        bad |= slotFast( t, limit );
+                    if ( __builtin_expect( bad == 0, 1 ) )
+                        continue;
+                    fx = fx0;
+                    fy = fy0;
+                    fz = fz0;
+                }
+            }
             for ( int t = 0; t < R.y; t++ )
                 slot( t, loadK( t ) );
         }
@@ -1468,6 +1682,46 @@ __global__ __launch_bounds__( kBlock ) __attribute__( ( amdgpu_waves_per_eu( ( P
             loadHalf( v1, g + kSlice );
     };
 
+    // FP64: rows of ordinary values take the shared reciprocals (see kForceRows)
+    constexpr bool FAST = ( PREC == kF64 );
+    const bool plain = FAST && scalarLoad( &A.plain_range ) != 0;
+    int own_lo = 0, own_hi = 0;
+    if constexpr ( FAST )
+    {
+        expRange( ui0, own_lo, own_hi );
+        expRange( ui1, own_lo, own_hi );
+        expRange( ui2, own_lo, own_hi );
+        expRange( Ti, own_lo, own_hi );
+    }
+    auto rowPlain = [&]() {
+        int lo = own_lo, hi = own_hi;
+#pragma unroll
+        for ( int q = 0; q < 3; q++ )
+        {
+            expRange( v0[q], lo, hi );
+            expRange( v1[q], lo, hi );
+        }
+        if constexpr ( TH )
+        {
+            expRange( v0[KH], lo, hi );
+            expRange( v1[KH], lo, hi );
+        }
+        bool out = lo < -kPlainExp || hi > kPlainExp;
+        if constexpr ( NAB )
+        {
+            int la = 0, ha = 0;
+#pragma unroll
+            for ( int q = 3 + NX; q < 5 + NX; q++ )
+            {
+                expRange( v0[q], la, ha );
+                expRange( v1[q], la, ha );
+            }
+            expRange( Ai, la, ha );
+            expRange( Bi, la, ha );
+            out = out || la < -kPlainExpAB || ha > kPlainExpAB;
+        }
+        return __ballot( out ) == 0;
+    };
     double* __restrict__ wb = &win[wv][0][0];
     const int nrows = scalarLoad( &A.nrows );
     loadRow( 0 );
@@ -1486,6 +1740,7 @@ __global__ __launch_bounds__( kBlock ) __attribute__( ( amdgpu_waves_per_eu( ( P
             if ( lane < R.y - 1 )
                 wb[k * kW + kSlice + lane] = v1[k];
         }
+        const double limit = FAST && rowPlain() ? 0x1p600 : 0.0;
         __builtin_amdgcn_fence( __ATOMIC_RELEASE, "wavefront" );
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence( __ATOMIC_ACQUIRE, "wavefront" );
@@ -1659,6 +1914,80 @@ __global__ __launch_bounds__( kBlock ) __attribute__( ( amdgpu_waves_per_eu( ( P
                 }
             }
         };
+        // FP64 with shared reciprocals: the lanes the general code has to
+        // evaluate (a plastic stretch is updated only where s is final, and
+        // updating it again with the same s changes nothing)
+        auto slotFast = [&]( const int t, const double lim ) __attribute__( ( always_inline ) ) {
+            const int32_t q = R.x + t;
+            const uint64_t ww = scalarLoad( mwords + q );
+            const double* __restrict__ wr = wb + lane + t;
+            double spv = 0.0;
+            if constexpr ( EP )
+                spv = spl[q * kSlice];
+            bool brk = false, gen = false;
+            if ( __builtin_amdgcn_inverse_ballot_w64( ww ) )
+            {
+                int mj = 0;
+                bool nf_j = false;
+                if constexpr ( TAG )
+                {
+                    const int tag = static_cast<int>( wr[KT * kW] );
+                    mj = tag >> 1;
+                    nf_j = ( tag & 1 ) != 0;
+                }
+                if constexpr ( kIsLps<MODEL> )
+                    nf_j = nf_i;
+                const double vj = wr[KV * kW];
+                Fast64 b;
+                getDistanceFast( xi0, xi1, xi2, ui0, ui1, ui2, wr[3 * kW], wr[4 * kW], wr[5 * kW], wr[0], wr[kW],
+                                 wr[2 * kW], b );
+                double temp_avg = 0.0;
+                if constexpr ( TH )
+                {
+                    temp_avg = thermalAvg( A, Ti, wr[KH * kW] );
+                    b.s = b.s - ( A.alpha * temp_avg );
+                }
+                gen = !( fabs( b.s ) <= 0x1p600 ) || max( lowWord( b.r ), lowWord( b.xi ) ) == 0xffffffffu;
+                if constexpr ( FRAC )
+                {
+                    const double bcc_ij = TH ? thermalBcc( A, temp_avg ) : ( MT ? tab_bcc[ti4 + mj] : bcc );
+                    brk = !gen && criticalStretch64( b.r, b.xi, bcc_ij ) && !nf_i && !nf_j;
+                }
+                if ( !brk )
+                {
+                    double coeff;
+                    if constexpr ( !kIsLps<MODEL> )
+                    {
+                        double sd = b.s;
+                        if constexpr ( EP )
+                        {
+                            if ( !gen )
+                                sd = plasticStretchAt( spl + q * kSlice, spv, b.s, A.sY );
+                        }
+                        coeff = ( MT ? tab_c[ti4 + mj] : c ) * sd * vj;
+                    }
+                    else
+                    {
+                        const double infl = infl1 ? 1.0 / b.xi : 1.0;
+                        coeff = ( Ai + wr[( 3 + NX ) * kW] + b.s * ( Bi + wr[( 4 + NX ) * kW] ) ) * infl * b.xi * vj;
+                    }
+                    gen = gen || !( fabs( coeff ) <= lim );
+                    fx += divBy( coeff * b.rx, b.r, b.yr );
+                    fy += divBy( coeff * b.ry, b.r, b.yr );
+                    fz += divBy( coeff * b.rz, b.r, b.yr );
+                }
+            }
+            if constexpr ( FRAC )
+            {
+                const uint64_t brkm = __ballot( brk );
+                if ( __builtin_expect( brkm != 0, 0 ) )
+                {
+                    if ( lane == 0 )
+                        bits[q] = ww & ~brkm;
+                }
+            }
+            return __ballot( gen );
+        };
         if constexpr ( PREC == kMixed )
         {
 #pragma unroll
@@ -1668,6 +1997,18 @@ __global__ __launch_bounds__( kBlock ) __attribute__( ( amdgpu_waves_per_eu( ( P
         }
         else
         {
+            if ( plain )
+            {
+                const double fx0 = fx, fy0 = fy, fz0 = fz;
+                uint64_t bad = 0;
+                for ( int t = 0; t < R.y; t++ )
+                    bad |= slotFast( t, limit );
+                if ( __builtin_expect( bad == 0, 1 ) )
+                    continue;
+                fx = fx0;
+                fy = fy0;
+                fz = fz0;
+            }
             for ( int t = 0; t < R.y; t++ )
                 slot( t );
         }
@@ -1919,8 +2260,11 @@ __global__ __launch_bounds__( kBlock ) void kLpsStateRows( const PDArgs* __restr
             loadHalf( v1, g + kSlice );
     };
     // Walk every bond slot in slot order; bond(live, wr, q) gets the window
-    // position of the neighbor's staged values.
-    auto walk = [&]( auto&& bond ) {
+    // position of the neighbor's staged values.  FP64: a row goes through
+    // fast first where plain; rows with a lane for which it returns true are
+    // evaluated again by bond, from the sums as save left them.
+    const bool plain = PREC == kF64 && scalarLoad( &A.plain_range ) != 0;
+    auto walk = [&]( auto&& bond, auto&& fast, double& sum ) {
         const int nrows = scalarLoad( &A.nrows );
         loadRow( 0 );
         for ( int r = 0; r < nrows; r++ )
@@ -1958,6 +2302,19 @@ __global__ __launch_bounds__( kBlock ) void kLpsStateRows( const PDArgs* __restr
             }
             else
             {
+                if ( plain )
+                {
+                    const double sum0 = sum;
+                    uint64_t bad = 0;
+                    for ( int t = 0; t < R.y; t++ )
+                    {
+                        const bool live = __builtin_amdgcn_inverse_ballot_w64( scalarLoad( mwords + R.x + t ) );
+                        bad |= __ballot( fast( live, wb + lane + t ) );
+                    }
+                    if ( __builtin_expect( bad == 0, 1 ) )
+                        continue;
+                    sum = sum0;
+                }
                 for ( int t = 0; t < R.y; t++ )
                 {
                     const int32_t q = R.x + t;
@@ -1983,13 +2340,28 @@ __global__ __launch_bounds__( kBlock ) void kLpsStateRows( const PDArgs* __restr
                     const double infl = infl1 ? 1.0 / b.xi : 1.0;
                     m_i += infl * b.xi * b.xi * ( GEN ? wr[KV * kW] : volu );
                 }
-            } );
+            },
+            [&]( bool live, const double* wr ) {
+                // |xi| alone: its range is the lattice's
+                if ( live )
+                {
+                    const double xi_x = wr[3 * kW] - xi0, xi_y = wr[4 * kW] - xi1, xi_z = wr[5 * kW] - xi2;
+                    const double xi = rootRecip( xi_x * xi_x + xi_y * xi_y + xi_z * xi_z ).r;
+                    const double infl = infl1 ? 1.0 / xi : 1.0;
+                    m_i += infl * xi * xi * ( GEN ? wr[KV * kW] : volu );
+                }
+                return false;
+            },
+            m_i );
         }
         else if ( valid )
             m_i = A.m[p];
         const bool mpos = FRAC ? ( m_i > 0 ) : true;
         if ( do_theta )
         {
+            // one reciprocal of m_i for all its bonds
+            const double ym = recip64( m_i );
+            const bool gen_m = !( m_i >= 0x1p-300 && m_i <= 0x1p300 ) || lowWord( m_i ) == 0xffffffffu;
             walk( [&]( bool live, const double* wr, int32_t, double, double ) {
                 if ( live && mpos )
                 {
@@ -2000,7 +2372,22 @@ __global__ __launch_bounds__( kBlock ) void kLpsStateRows( const PDArgs* __restr
                     const double theta_b = infl * b.s * b.xi * b.xi * ( GEN ? wr[KV * kW] : volu );
                     th += 3.0 * theta_b / m_i;
                 }
-            } );
+            },
+            [&]( bool live, const double* wr ) {
+                bool gen = false;
+                if ( live && mpos )
+                {
+                    Fast64 b;
+                    getDistanceFast( xi0, xi1, xi2, ui0, ui1, ui2, wr[3 * kW], wr[4 * kW], wr[5 * kW], wr[0], wr[kW],
+                                     wr[2 * kW], b );
+                    const double infl = infl1 ? 1.0 / b.xi : 1.0;
+                    const double theta_b = infl * b.s * b.xi * b.xi * ( GEN ? wr[KV * kW] : volu );
+                    th += divBy( 3.0 * theta_b, m_i, ym );
+                    gen = gen_m || !( fabs( theta_b ) <= 0x1p300 ) || lowWord( b.xi ) == 0xffffffffu;
+                }
+                return gen;
+            },
+            th );
         }
     }
     else
@@ -2027,7 +2414,8 @@ __global__ __launch_bounds__( kBlock ) void kLpsStateRows( const PDArgs* __restr
                     th += static_cast<double>( w2 * b.s * vj32 );
                 }
             }
-        } );
+        },
+        []( bool, const double* ) { return false; }, th );
         if ( do_theta )
         {
             const bool mpos = FRAC ? ( m_i > 0 ) : true;
@@ -2316,8 +2704,14 @@ struct RowWalk64
     // bond(q, wr, g) for every slot q of the slice in slot order; wr is the
     // lane's window position (channel k at wr[k * kW]) and g + lane its
     // neighbour's id.  win: this wave's [2][NC][kW] LDS buffers.
-    template <class Bond>
-    __device__ __forceinline__ void walk( double* __restrict__ win, Bond&& bond ) const
+    // With plain, a row goes through fast( q, wr, g, limit ) first (the
+    // shared-reciprocal arithmetic; limit is 2^600, or 0 when out( v0, v1 )
+    // says that a lane's staged values are outside its range).  If it returns
+    // true for a lane, the row is evaluated again by bond, from the sums as
+    // they were before the row.
+    template <class Out, class Sums, class Bond, class Fast>
+    __device__ __forceinline__ void walk( double* __restrict__ win, bool plain, Out&& out, Sums& sums, Bond&& bond,
+                                          Fast&& fast ) const
     {
         double v0[NC], v1[NC];
 #pragma unroll
@@ -2351,6 +2745,7 @@ struct RowWalk64
                 if ( lane < R.y - 1 )
                     wb[k * kW + kSlice + lane] = v1[k];
             }
+            const double limit = plain && __ballot( out( v0, v1 ) ) == 0 ? 0x1p600 : 0.0;
             // LDS operations of one wavefront complete in order; the fences
             // keep the compiler from moving the window reads above the stores
             __builtin_amdgcn_fence( __ATOMIC_RELEASE, "wavefront" );
@@ -2358,6 +2753,16 @@ struct RowWalk64
             __builtin_amdgcn_fence( __ATOMIC_ACQUIRE, "wavefront" );
             if ( r + 1 < nrows )
                 loadRow( r + 1 );
+            if ( plain )
+            {
+                const Sums before = sums;
+                uint64_t bad = 0;
+                for ( int t = 0; t < R.y; t++ )
+                    bad |= __ballot( fast( R.x + t, wb + lane + t, p032 + R.z + t, limit ) );
+                if ( __builtin_expect( bad == 0, 1 ) )
+                    continue;
+                sums = before;
+            }
             for ( int t = 0; t < R.y; t++ )
                 bond( R.x + t, wb + lane + t, p032 + R.z + t );
         }
@@ -2459,13 +2864,12 @@ __global__ __launch_bounds__( kBlock ) void kEnergyRows( const PDArgs* __restric
                 num_bonds = static_cast<double>( A.cnt[pc] );
         }
         const double vol_i = volp[pc];
-        double W = 0.0, phi_i = 0.0, vol_H_i = 0.0;
-        rw.walk( &win[wv][0][0][0], [&]( int32_t q, const double* __restrict__ wr, int32_t g ) {
-            if ( !__builtin_amdgcn_inverse_ballot_w64( scalarLoad( ew + q ) ) )
-                return;
-            Bond64 b;
-            bond64<MODEL>( xi0, xi1, xi2, ui0, ui1, ui2, wr[3 * kW], wr[4 * kW], wr[5 * kW], wr[0], wr[kW],
-                           wr[2 * kW], b );
+        struct Sums
+        {
+            double W, phi_i, vol_H_i, Phi;
+        } S{ 0.0, 0.0, 0.0, 0.0 };
+        // one bond of stretch b.s and length b.xi
+        auto bondSum = [&]( auto& b, int32_t q, const double* __restrict__ wr, int32_t g ) {
             const double vj = GEN ? wr[6 * kW] : volu;
             double wb;
             if constexpr ( kIsLps<MODEL> )
@@ -2488,23 +2892,47 @@ __global__ __launch_bounds__( kBlock ) void kEnergyRows( const PDArgs* __restric
             {
                 const double mu = static_cast<double>( ( scalarLoad( iw + q ) >> lane ) & 1ull );
                 wb = mu * wb;
-                W += wb;
-                phi_i += mu * vj;
-                vol_H_i += vj;
+                S.W += wb;
+                S.phi_i += mu * vj;
+                S.vol_H_i += vj;
             }
             else
             {
-                W += wb;
-                Phi += wb * vol_i;
+                S.W += wb;
+                S.Phi += wb * vol_i;
             }
-        } );
+        };
+        // (no division by |r|: any displacement goes through the shared
+        // reciprocal of |xi|, except where the stretch is not a number)
+        const bool plain = !kIsLin<MODEL> && scalarLoad( &A.plain_range ) != 0;
+        rw.walk(
+            &win[wv][0][0][0], plain, []( const double*, const double* ) { return false; }, S,
+            [&]( int32_t q, const double* __restrict__ wr, int32_t g ) {
+                if ( !__builtin_amdgcn_inverse_ballot_w64( scalarLoad( ew + q ) ) )
+                    return;
+                Bond64 b;
+                bond64<MODEL>( xi0, xi1, xi2, ui0, ui1, ui2, wr[3 * kW], wr[4 * kW], wr[5 * kW], wr[0], wr[kW],
+                               wr[2 * kW], b );
+                bondSum( b, q, wr, g );
+            },
+            [&]( int32_t q, const double* __restrict__ wr, int32_t g, double lim ) {
+                if ( !__builtin_amdgcn_inverse_ballot_w64( scalarLoad( ew + q ) ) )
+                    return false;
+                Fast64 b;
+                getDistanceFast( xi0, xi1, xi2, ui0, ui1, ui2, wr[3 * kW], wr[4 * kW], wr[5 * kW], wr[0], wr[kW],
+                                 wr[2 * kW], b );
+                const bool gen = !( fabs( b.s ) <= lim ) || lowWord( b.xi ) == 0xffffffffu;
+                bondSum( b, q, wr, g );
+                return gen;
+            } );
+        Phi = S.Phi;
         if ( valid )
         {
-            A.W[p] = W;
+            A.W[p] = S.W;
             if constexpr ( FRAC )
             {
-                Phi = W * vol_i;
-                const double ph = 1 - phi_i / vol_H_i;
+                Phi = S.W * vol_i;
+                const double ph = 1 - S.phi_i / S.vol_H_i;
                 A.phi[p] = ph;
                 D = ph;
             }
@@ -2599,24 +3027,23 @@ __global__ __launch_bounds__( kBlock ) void kStressRows( const PDArgs* __restric
         Ai = A.lpsA[pc];
         Bi = A.lpsB[pc];
     }
-    double s00 = 0.0, s01 = 0.0, s02 = 0.0, s10 = 0.0, s11 = 0.0, s12 = 0.0, s20 = 0.0, s21 = 0.0, s22 = 0.0;
-    rw.walk( &win[wv][0][0][0], [&]( int32_t q, const double* __restrict__ wr, int32_t g ) {
+    struct Sums
+    {
+        double s00, s01, s02, s10, s11, s12, s20, s21, s22;
+    } S{};
+    // what the general and the shared-reciprocal form have in common: the
+    // bonds visited, the force coefficient, the nine terms
+    auto visited = [&]( int32_t q, uint64_t& intact ) {
         uint64_t live = scalarLoad( ew + q );
-        uint64_t intact = ~0ull;
         if constexpr ( FRAC )
         {
             intact = scalarLoad( iw + q );
             if constexpr ( kIsLps<MODEL> )
                 live &= intact; // LPS fracture visits unbroken bonds only
         }
-        if ( !__builtin_amdgcn_inverse_ballot_w64( live ) )
-            return;
-        const double xj0 = wr[3 * kW], xj1 = wr[4 * kW], xj2 = wr[5 * kW];
-        Bond64 b;
-        bond64<MODEL>( xi0, xi1, xi2, ui0, ui1, ui2, xj0, xj1, xj2, wr[0], wr[kW], wr[2 * kW], b );
-        const double xi_x = xj0 - xi0;
-        const double xi_y = xj1 - xi1;
-        const double xi_z = xj2 - xi2;
+        return __builtin_amdgcn_inverse_ballot_w64( live );
+    };
+    auto coefficient = [&]( auto& b, int32_t q, const double* __restrict__ wr, int32_t g, bool final_s ) {
         const double vj = GEN ? wr[KV * kW] : volu;
         double coeff;
         if constexpr ( kIsLps<MODEL> )
@@ -2627,47 +3054,106 @@ __global__ __launch_bounds__( kBlock ) void kStressRows( const PDArgs* __restric
         }
         else
         {
-            if constexpr ( TH )
-                b.s = b.s - ( A.alpha * thermalAvg( A, Ti, wr[KT * kW] ) );
-            const double sd = EP ? plasticStretch( spl + q * kSlice, b.s, A.sY ) : b.s;
+            double sd = b.s;
+            if constexpr ( EP )
+            {
+                if ( final_s )
+                    sd = plasticStretch( spl + q * kSlice, b.s, A.sY );
+            }
             coeff = 0.5 * ( ( MT ? A.mat_c[ti4 + mtp[g + lane]] : c ) * sd * vj );
         }
-        double fx, fy, fz;
-        if constexpr ( FRAC )
-        {
-            const double mu = static_cast<double>( ( intact >> lane ) & 1ull );
-            fx = mu * coeff * b.rx / b.r;
-            fy = mu * coeff * b.ry / b.r;
-            fz = mu * coeff * b.rz / b.r;
-        }
-        else
-        {
-            fx = coeff * b.rx / b.r;
-            fy = coeff * b.ry / b.r;
-            fz = coeff * b.rz / b.r;
-        }
-        s00 += fx * xi_x;
-        s11 += fy * xi_y;
-        s22 += fz * xi_z;
-        s01 += fx * xi_y;
-        s10 += fy * xi_x;
-        s02 += fx * xi_z;
-        s20 += fz * xi_x;
-        s12 += fy * xi_z;
-        s21 += fz * xi_y;
-    } );
+        return coeff;
+    };
+    auto add = [&]( const double* __restrict__ wr, double fx, double fy, double fz ) {
+        const double xi_x = wr[3 * kW] - xi0;
+        const double xi_y = wr[4 * kW] - xi1;
+        const double xi_z = wr[5 * kW] - xi2;
+        S.s00 += fx * xi_x;
+        S.s11 += fy * xi_y;
+        S.s22 += fz * xi_z;
+        S.s01 += fx * xi_y;
+        S.s10 += fy * xi_x;
+        S.s02 += fx * xi_z;
+        S.s20 += fz * xi_x;
+        S.s12 += fy * xi_z;
+        S.s21 += fz * xi_y;
+    };
+    const bool plain = !kIsLin<MODEL> && scalarLoad( &A.plain_range ) != 0;
+    int own_lo = 0, own_hi = 0, own_la = 0, own_ha = 0;
+    expRange( ui0, own_lo, own_hi );
+    expRange( ui1, own_lo, own_hi );
+    expRange( ui2, own_lo, own_hi );
+    expRange( Ti, own_lo, own_hi );
+    expRange( Ai, own_la, own_ha );
+    expRange( Bi, own_la, own_ha );
+    rw.walk(
+        &win[wv][0][0][0], plain,
+        [&]( const double* v0, const double* v1 ) {
+            int lo = own_lo, hi = own_hi, la = own_la, ha = own_ha;
+#pragma unroll
+            for ( int q = 0; q < 3; q++ )
+            {
+                expRange( v0[q], lo, hi );
+                expRange( v1[q], lo, hi );
+            }
+            if constexpr ( TH )
+            {
+                expRange( v0[KT], lo, hi );
+                expRange( v1[KT], lo, hi );
+            }
+#pragma unroll
+            for ( int q = 6; q < 6 + NE; q++ )
+            {
+                expRange( v0[q], la, ha );
+                expRange( v1[q], la, ha );
+            }
+            return lo < -kPlainExp || hi > kPlainExp || la < -kPlainExpAB || ha > kPlainExpAB;
+        },
+        S,
+        [&]( int32_t q, const double* __restrict__ wr, int32_t g ) {
+            uint64_t intact = ~0ull;
+            if ( !visited( q, intact ) )
+                return;
+            Bond64 b;
+            bond64<MODEL>( xi0, xi1, xi2, ui0, ui1, ui2, wr[3 * kW], wr[4 * kW], wr[5 * kW], wr[0], wr[kW],
+                           wr[2 * kW], b );
+            if constexpr ( TH )
+                b.s = b.s - ( A.alpha * thermalAvg( A, Ti, wr[KT * kW] ) );
+            double coeff = coefficient( b, q, wr, g, true );
+            if constexpr ( FRAC )
+                coeff = static_cast<double>( ( intact >> lane ) & 1ull ) * coeff;
+            add( wr, coeff * b.rx / b.r, coeff * b.ry / b.r, coeff * b.rz / b.r );
+        },
+        [&]( int32_t q, const double* __restrict__ wr, int32_t g, double lim ) {
+            uint64_t intact = ~0ull;
+            if ( !visited( q, intact ) )
+                return false;
+            Fast64 b;
+            getDistanceFast( xi0, xi1, xi2, ui0, ui1, ui2, wr[3 * kW], wr[4 * kW], wr[5 * kW], wr[0], wr[kW],
+                             wr[2 * kW], b );
+            if constexpr ( TH )
+                b.s = b.s - ( A.alpha * thermalAvg( A, Ti, wr[KT * kW] ) );
+            bool gen = !( fabs( b.s ) <= 0x1p600 ) || max( lowWord( b.r ), lowWord( b.xi ) ) == 0xffffffffu;
+            double coeff = coefficient( b, q, wr, g, !gen );
+            gen = gen || !( fabs( coeff ) <= lim );
+            if constexpr ( FRAC )
+                coeff = static_cast<double>( ( intact >> lane ) & 1ull ) * coeff;
+            add( wr, divBy( coeff * b.rx, b.r, b.yr ), divBy( coeff * b.ry, b.r, b.yr ),
+                 divBy( coeff * b.rz, b.r, b.yr ) );
+            return gen;
+        } );
     if ( !valid )
         return;
     double* __restrict__ st = A.stress;
-    st[p] = s00;
-    st[n + p] = s01;
-    st[2 * n + p] = s02;
-    st[3 * n + p] = s10;
-    st[4 * n + p] = s11;
-    st[5 * n + p] = s12;
-    st[6 * n + p] = s20;
-    st[7 * n + p] = s21;
-    st[8 * n + p] = s22;
+    st[p] = S.s00;
+    st[n + p] = S.s01;
+    st[2 * n + p] = S.s02;
+    st[3 * n + p] = S.s10;
+    st[4 * n + p] = S.s11;
+    st[5 * n + p] = S.s12;
+    st[6 * n + p] = S.s20;
+    st[7 * n + p] = S.s21;
+    st[8 * n + p] = S.s22;
 }
 
 // ---------------------------------------------------------------------------
@@ -2763,18 +3249,41 @@ __global__ __launch_bounds__( kBlock ) void kHeatConductionRows( const PDArgs* _
     const int lin = A.lin_micro;
     const double volu = A.vol_value;
     double conduction = 0.0;
-    rw.walk( &win[wv][0][0][0], [&]( int32_t q, const double* __restrict__ wr, int32_t g ) {
-        // intact bonds under fracture (a subset of the existing ones)
-        if ( !__builtin_amdgcn_inverse_ballot_w64( scalarLoad( mw + q ) ) )
-            return;
-        const double xi_x = wr[0] - xi0;
-        const double xi_y = wr[kW] - xi1;
-        const double xi_z = wr[2 * kW] - xi2;
-        const double xi = sqrt( xi_x * xi_x + xi_y * xi_y + xi_z * xi_z );
-        // microconductivity_function (CabanaPD_ForceModels.hpp:302-308)
-        const double coeff = lin ? 4.0 * tc * ( 1.0 - xi / th ) : tc;
-        conduction += coeff * ( wr[3 * kW] - Ti ) / xi / xi * ( GEN ? wr[4 * kW] : volu );
-    } );
+    int own_lo = 0, own_hi = 0;
+    expRange( Ti, own_lo, own_hi );
+    // (intact bonds under fracture, a subset of the existing ones; the linear
+    // microconductivity keeps the general code)
+    rw.walk(
+        &win[wv][0][0][0], lin == 0 && scalarLoad( &A.plain_range ) != 0,
+        [&]( const double* v0, const double* v1 ) {
+            int lo = own_lo, hi = own_hi;
+            expRange( v0[3], lo, hi );
+            expRange( v1[3], lo, hi );
+            return lo < -kPlainExp || hi > kPlainExp;
+        },
+        conduction,
+        [&]( int32_t q, const double* __restrict__ wr, int32_t g ) {
+            if ( !__builtin_amdgcn_inverse_ballot_w64( scalarLoad( mw + q ) ) )
+                return;
+            const double xi_x = wr[0] - xi0;
+            const double xi_y = wr[kW] - xi1;
+            const double xi_z = wr[2 * kW] - xi2;
+            const double xi = sqrt( xi_x * xi_x + xi_y * xi_y + xi_z * xi_z );
+            // microconductivity_function (CabanaPD_ForceModels.hpp:302-308)
+            const double coeff = lin ? 4.0 * tc * ( 1.0 - xi / th ) : tc;
+            conduction += coeff * ( wr[3 * kW] - Ti ) / xi / xi * ( GEN ? wr[4 * kW] : volu );
+        },
+        [&]( int32_t q, const double* __restrict__ wr, int32_t g, double lim ) {
+            if ( !__builtin_amdgcn_inverse_ballot_w64( scalarLoad( mw + q ) ) )
+                return false;
+            const double xi_x = wr[0] - xi0;
+            const double xi_y = wr[kW] - xi1;
+            const double xi_z = wr[2 * kW] - xi2;
+            const Root64 xi = rootRecip( xi_x * xi_x + xi_y * xi_y + xi_z * xi_z );
+            const double flow = tc * ( wr[3 * kW] - Ti );
+            conduction += divBy( divBy( flow, xi.r, xi.y ), xi.r, xi.y ) * ( GEN ? wr[4 * kW] : volu );
+            return !( fabs( flow ) <= lim ) || lowWord( xi.r ) == 0xffffffffu;
+        } );
     if ( valid )
         A.cond[p] = conduction;
 }

@@ -1,0 +1,80 @@
+"""FP64 row passes at values where their shared-reciprocal arithmetic must
+hand over to the general code: displacements far below the spacing (down to
+subnormal), bonds whose length is the double just below a power of two times
+the spacing (the one mantissa whose reciprocal the fast form does not round
+correctly), particles on top of each other (|r| = 0), and huge or non-finite
+displacements.  Every result equals the oracle's bit for bit (NaN where it
+has NaN)."""
+import numpy as np
+import pytest
+
+from cabanapd_amd import configs
+from cabanapd_amd._abi import make_desc
+from tests.parity import pair, say
+
+pytestmark = pytest.mark.gpu
+
+N = 9
+H = 1.0 / 64.0  # a power of two: bond vectors along the axes are exact
+
+
+def workload(kind, seed, wild):
+    x, vol, _ = configs.grid_node_centred(N, H)
+    rng = np.random.default_rng(seed)
+    n = x.shape[0]
+    sizes = np.array([0.0, 5e-324, 1e-310, 1e-200, 1e-40, 2.0 ** -59, 2.0 ** -58, 1e-9, 1e-5])
+    u = rng.choice(sizes, size=(n, 3)) * rng.choice([-1.0, 1.0], size=(n, 3))
+    u[rng.random(n) < 0.4] = 0.0
+    if wild:
+        c = (N // 2) * (1 + N + N * N)
+        u[c] = [-H, 0.0, 0.0]              # onto its neighbour
+        u[c + 1 + N] = [H, 0.0, 1e-200]    # onto the next one but for a tiny offset
+        u[3] = [1e180, 0.0, 0.0]
+        u[N * N * N - 4] = [np.inf, 1.0, 0.0]
+    kw = dict(horizon=3.01 * H, K=2e9, dt=1e-9)
+    model = "PMB"
+    frac = kind in ("pmb_fracture", "lps_fracture", "epp", "materials")
+    if frac:
+        kw.update(fracture=True, G0=0.5)
+    if kind.startswith("lps"):
+        model = "LPS"
+        kw.update(G=1.1e9, influence=1 if kind == "lps_influence1" else 0)
+    if kind == "epp":
+        kw.update(mechanics="epp", sigma_y=1e5)
+    if kind == "heat":
+        kw.update(thermal="dynamic", alpha=1e-5, temp0=0.0, kappa=1.0, cp=1.0, thermal_subcycle=1)
+    w = configs._base(make_desc(model, **kw), x, vol, 1000.0, "extreme_" + kind, H, 2)
+    w["u"] = u
+    if kind == "heat":
+        w["temperature"] = rng.choice([0.0, 1e-320, 1e-200, 1e-20, 1.0, 30.0], size=n)
+    if kind == "materials":
+        w["materials"] = ([(2e9, 1.1e9, 0.5), (5e9, 2e9, 2.0)], (rng.random(n) < 0.5).astype(np.int32))
+    return w
+
+
+def same(a, b, what):
+    a, b = np.asarray(a), np.asarray(b)
+    bad = (a != b) & ~(np.isnan(a) & np.isnan(b))
+    assert not bad.any(), f"{what}: {int(bad.sum())} values differ"
+
+
+@pytest.mark.parametrize("wild", [False, True])
+@pytest.mark.parametrize("kind", ["pmb", "pmb_fracture", "lps", "lps_influence1", "lps_fracture", "epp", "materials",
+                                  "heat"])
+def test_extreme_displacements_match_oracle(kind, wild):
+    say(f"case: {kind}, {N}^3 FP64, tiny to subnormal displacements, wild={wild}")
+    w = workload(kind, 17, wild)
+    g, o = pair(w)
+    assert "Rows" in g.kernel_name(0)
+    for fld in ("f", "W"):
+        same(g.get(fld), o.get(fld), fld + " at init")
+    g.compute_stress()
+    o.compute_stress()
+    same(g.get("stress"), o.get("stress"), "stress")
+    g.step(2)
+    o.step(2)
+    for fld in ("u", "v", "f") + (("m", "theta") if kind.startswith("lps") else ()) + (
+            ("temperature",) if kind == "heat" else ()):
+        same(g.get(fld), o.get(fld), fld)
+    assert np.array_equal(g.bonds()[2], o.bonds()[2])
+    g.close()
