@@ -1037,9 +1037,12 @@ struct SlotEntry
     double r2;
 };
 
-// Stencil entries of a full lattice in slot order.  margin: relative band
+// Stencil entries of a full lattice in slot order.  margin > 0: relative band
 // around the cutoff (in squared distance) inside which no lattice vector may
-// lie, since there the rounding of the actual positions decides.
+// lie, since there the rounding of the actual positions decides.  0: the
+// caller checks the entries against every row of the cell search (horizons of
+// a whole number of spacings plus 1e-10, as most input decks set them, have
+// lattice vectors within 1e-7 of the cutoff).
 bool slotStencil( int64_t n, const int64_t dims[3], const double h[3], double rc,
                   const std::vector<int64_t>& perm_host, double margin, std::vector<SlotEntry>& es,
                   LatticeBox& L, bool& identity )
@@ -1058,7 +1061,7 @@ bool slotStencil( int64_t n, const int64_t dims[3], const double h[3], double rc
         if ( !( h[d] > 0 ) )
             return false;
         // largest integer offset along d that can be within the cutoff
-        K[d] = static_cast<int32_t>( std::floor( rc / h[d] * ( 1.0 + margin ) ) );
+        K[d] = static_cast<int32_t>( std::floor( rc / h[d] * ( 1.0 + std::max( margin, 1e-6 ) ) ) );
         if ( K[d] > 40 || ( !identity && dims[d] <= 2 * K[d] ) )
             return false;
     }
@@ -1073,7 +1076,7 @@ bool slotStencil( int64_t n, const int64_t dims[3], const double h[3], double rc
                 const double r2 = gx * gx + gy * gy + gz * gz;
                 if ( r2 == 0.0 )
                     continue;
-                if ( std::fabs( r2 - rc2 ) <= margin * rc2 )
+                if ( margin > 0.0 && std::fabs( r2 - rc2 ) <= margin * rc2 )
                     return false;
                 if ( r2 > rc2 )
                     continue;
@@ -1256,7 +1259,7 @@ bool buildStencilSlots( const PDArgs& a, const int64_t dims[3], const double h[3
     std::vector<SlotEntry> es;
     LatticeBox L{};
     bool identity = false;
-    if ( !slotStencil( n, dims, h, rc, perm_host, 1e-6, es, L, identity ) )
+    if ( !slotStencil( n, dims, h, rc, perm_host, 0.0, es, L, identity ) )
         return false;
     const int32_t S = static_cast<int32_t>( es.size() );
     const std::vector<int4> ent = slotEntries( es );
