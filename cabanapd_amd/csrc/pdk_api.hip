@@ -422,6 +422,9 @@ struct pdk_spec_s
             h.rows = slot.nrows > 0 ? slot.rows.as<int4>() : nullptr;
             h.rowstart = slot.nrows > 0 ? slot.rowstart.as<uint32_t>() : nullptr;
             h.nrows = slot.nrows;
+            h.row_max = slot.row_max;
+            h.hole_win = slot.hole ? slot.hole_win.as<int2>() : nullptr;
+            h.hole_pos = slot.hole ? slot.hole_pos.as<uint8_t>() : nullptr;
             for ( int dd = 0; dd < 3; dd++ )
                 h.lat_n[dd] = static_cast<int32_t>( lat_dims[dd] );
         }
@@ -430,6 +433,9 @@ struct pdk_spec_s
             h.rows = nullptr;
             h.rowstart = nullptr;
             h.nrows = 0;
+            h.row_max = 0;
+            h.hole_win = nullptr;
+            h.hole_pos = nullptr;
         }
         // tuning knob: -1 = default (row windows where available, else groups
         // of 4, or of 2 for the mixed form in the compact layout, measured

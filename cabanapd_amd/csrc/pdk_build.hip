@@ -1200,6 +1200,9 @@ void finishSlots( int64_t n, int64_t nslices, const LatticeBox& L, const std::ve
     out.rows = std::move( drows );
     out.rowstart = std::move( drstart );
     out.nrows = nrows;
+    out.row_max = 0;
+    for ( const int4& r : rtab )
+        out.row_max = std::max( out.row_max, r.y );
     out.slots = S;
     total_rows = rows;
     col_capacity_rows = rows;

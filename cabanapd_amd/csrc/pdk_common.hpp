@@ -137,6 +137,12 @@ struct PDArgs
     const uint32_t* rowstart; // bit q set: slot q starts a row (9 words), or null
     int32_t nrows;          // 0: no row table
     int32_t lat_n[3];       // lattice extent (stencil-slot form)
+    // Lattices with missing sites in the stencil-slot form: per slice and row
+    // of the row table the neighbour window (first id, length <= 127) and each
+    // lane's place in it ([slice][row][lane]); null on full lattices.
+    const int2* hole_win;
+    const uint8_t* hole_pos;
+    int32_t row_max;        // longest row of the row table, in slots
     // FP64 row passes: positions, volumes and constants are within the ranges
     // for which the shared-reciprocal bond arithmetic gives the general
     // code's bits (the rows test displacements themselves)

@@ -1,484 +1,16 @@
 // pdk_force.hip -- PD bond passes with the velocity-Verlet update fused into
 // the force epilogue.
-//
-// Mapping: one wavefront per 64-row slice of the sliced CSR, one lane per
-// particle, a serial loop over the lane's bonds, no atomics -- the reference's
-// SerialOpTag traversal (CabanaPD_Neighbor.hpp:31,134-151) laid out for
-// 64-wide wavefronts: each slot row of 64 neighbor ids is one coalesced 256 B
-// load and the broken-bond word of a slot row is one uniform 8 B load.
-//
-// Precision forms:
-//   FP64  : the reference's expressions, operand order and rounding
-//           (contraction off, correctly rounded sqrt/div).  Rows are summed
-//           in the oracle's order, so f/u/v match the oracle bit for bit.
-//   MIXED : bond geometry in FP32 from FP64 differences (no large-coordinate
-//           cancellation: xi = x_j - x_i and eta = u_j - u_i are formed in
-//           FP64 and rounded once), stretch s = (2 xi.eta + eta.eta) /
-//           (|xi| (|xi+eta| + |xi|)), bond forces accumulated in FP64.  A
-//           bond whose FP32 stretch lies inside a guard band around s0 is
-//           re-tested with the FP64 expression, so break decisions equal the
-//           FP64 decisions for the same state.
+// (the arithmetic and the row-window passes are in pdk_rows.hpp; here the
+// passes that gather, the output passes and the launches).
 #include <cmath>
 #include <cstdio>
 
-#include "pdk_internal.hpp"
+#include "pdk_rows.hpp"
 
 namespace pdk
 {
 namespace
 {
-// Values equal the ABI's model kinds.  The linearized models take the force
-// model of their parent (LinearPMB: PMB, LinearLPS: LPS) and change only the
-// bond geometry of the force and energy passes.
-enum ModelT : int
-{
-    kPMB = 0,
-    kLPS = 1,
-    kLinPMB = 4,
-    kLinLPS = 5
-};
-template <int M>
-constexpr bool kIsLps = ( M == kLPS || M == kLinLPS );
-template <int M>
-constexpr bool kIsLin = ( M == kLinPMB || M == kLinLPS );
-enum PrecT : int
-{
-    kF64 = 0,
-    kMixed = 1
-};
-
-struct Bond64
-{
-    double xi, r, s, rx, ry, rz;
-};
-
-// getDistance (CabanaPD_Force.hpp:74-93), operation for operation.
-__device__ __forceinline__ void getDistance64( double xi0, double xi1, double xi2, double ui0,
-                                               double ui1, double ui2, double xj0, double xj1,
-                                               double xj2, double uj0, double uj1, double uj2,
-                                               Bond64& b )
-{
-#pragma clang fp contract( off )
-    const double xi_x = xj0 - xi0;
-    const double eta_u = uj0 - ui0;
-    const double xi_y = xj1 - xi1;
-    const double eta_v = uj1 - ui1;
-    const double xi_z = xj2 - xi2;
-    const double eta_w = uj2 - ui2;
-    b.rx = xi_x + eta_u;
-    b.ry = xi_y + eta_v;
-    b.rz = xi_z + eta_w;
-    b.r = sqrt( b.rx * b.rx + b.ry * b.ry + b.rz * b.rz );
-    b.xi = sqrt( xi_x * xi_x + xi_y * xi_y + xi_z * xi_z );
-    b.s = ( b.r - b.xi ) / b.xi;
-}
-
-// BaseFractureModel CriticalStretchTag (CabanaPD_ForceModels.hpp:123-128).
-__device__ __forceinline__ bool criticalStretch64( double r, double xi, double bcc )
-{
-#pragma clang fp contract( off )
-    return r * r >= bcc * xi * xi;
-}
-
-// TemperatureDependent (CabanaPD_ForceModels.hpp:203-211): the bond's
-// temp_avg; the stretch becomes s - alpha * temp_avg.
-__device__ __forceinline__ double thermalAvg( const PDArgs& A, double Ti, double Tj )
-{
-#pragma clang fp contract( off )
-    return 0.5 * ( Ti + Tj ) - A.temp0;
-}
-// ThermalFractureModel CriticalStretchTag coefficient (CabanaPD_ForceModels.hpp:246-255).
-__device__ __forceinline__ double thermalBcc( const PDArgs& A, double temp_avg )
-{
-#pragma clang fp contract( off )
-    return ( 1.0 + A.s0 + A.alpha * temp_avg ) * ( 1.0 + A.s0 + A.alpha * temp_avg );
-}
-// EPP ForceCoeffTag (force_models/CabanaPD_PMB.hpp:104-121): update the bond's
-// plastic stretch (written only when it changes) and return s - s_p.
-__device__ __forceinline__ double plasticStretch( double* slot, double s, double sY )
-{
-#pragma clang fp contract( off )
-    double sp = *slot;
-    if ( s >= sp + sY )
-    {
-        sp = s - sY;
-        *slot = sp;
-    }
-    else if ( s <= sp - sY )
-    {
-        sp = s + sY;
-        *slot = sp;
-    }
-    return s - sp;
-}
-// The same with the slot's stored plastic stretch already loaded (sp).
-__device__ __forceinline__ double plasticStretchAt( double* slot, double sp, double s, double sY )
-{
-#pragma clang fp contract( off )
-    if ( s >= sp + sY )
-    {
-        sp = s - sY;
-        *slot = sp;
-    }
-    else if ( s <= sp - sY )
-    {
-        sp = s + sY;
-        *slot = sp;
-    }
-    return s - sp;
-}
-// EPP EnergyTag stretch term (force_models/CabanaPD_PMB.hpp:123-146).
-__device__ __forceinline__ double plasticEnergyTerm( double s, double sp, double sY )
-{
-#pragma clang fp contract( off )
-    if ( s >= sp + sY )
-        return sY * ( 2.0 * s - sY );
-    if ( s <= sp - sY )
-        return sY * ( -2.0 * s - sY );
-    return s * s;
-}
-
-struct Bond32
-{
-    float s, rinv, rx, ry, rz, xi;
-};
-
-// Mixed-form bond geometry from the FP64 bond vector r = xi + (u_j - u_i)
-// (the reference bond xi of the stencil entry, or x_j - x_i, plus the
-// displacement difference, so no large coordinate cancels): the stretch
-// numerator |r|^2 - |xi|^2 in FP64 as one FMA chain seeded with -|xi|^2 (the
-// FP64 square of the reference bond), then 1/|r| and
-//   s = (|r|^2 - |xi|^2) / (|xi| (|r| + |xi|))
-// in FP32, with |r|^2 = |xi|^2 + numerator.  The numerator is exact to FP64
-// rounding for any rotation of the bond (no xi.eta against eta.eta
-// cancellation in FP32), so the FP32 stretch is within a few ulp of s.  The
-// force passes accumulate the bond force along the FP64 r.
-__device__ __forceinline__ void mixedBond( double r0, double r1, double r2, double xi2d, float xi, Bond32& b )
-{
-    const float num = static_cast<float>( fma( r0, r0, fma( r1, r1, fma( r2, r2, -xi2d ) ) ) );
-    const float r2f = fmaf( xi, xi, num );
-    b.rinv = __builtin_amdgcn_rsqf( r2f );
-    b.s = num * __builtin_amdgcn_rcpf( fmaf( r2f, b.rinv, xi ) * xi );
-    b.rx = static_cast<float>( r0 );
-    b.ry = static_cast<float>( r1 );
-    b.rz = static_cast<float>( r2 );
-    b.xi = xi;
-}
-
-// Wave-uniform read through the scalar data cache (p must be the same in
-// every lane).  Used for the stencil tables, which no kernel writes, and for
-// the per-slot bond-mask words, which a wave reads before it writes them (a
-// vector store) and which no other wave of the launch touches; the scalar
-// cache starts every kernel dispatch invalidated.
-template <class T>
-__device__ __forceinline__ T scalarLoad( const T* p )
-{
-    return *( const __attribute__( ( address_space( 4 ) ) ) T* )( p );
-}
-__device__ __forceinline__ float4 scalarLoad4( const float4* p )
-{
-    const auto* f = ( const __attribute__( ( address_space( 4 ) ) ) float* )( p );
-    return make_float4( f[0], f[1], f[2], f[3] );
-}
-// Raw buffer access for the row windows: an SGPR resource (uniform base and
-// byte size), a VGPR byte offset (the lane) and an SGPR byte offset (the
-// window start), so no address arithmetic runs on the vector ALUs.  Offsets
-// at or past the size read 0 (hardware range check), which also covers
-// windows that start before id 0 (their negative offsets wrap to values
-// above the size for any specimen of fewer than 2^28 particles).
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t bufferOf( const void* base, uint32_t bytes )
-{
-    // base is wave-uniform; readfirstlane keeps the resource in SGPRs
-    const uint64_t b = reinterpret_cast<uint64_t>( base );
-    const uint32_t lo = __builtin_amdgcn_readfirstlane( static_cast<uint32_t>( b ) );
-    const uint32_t hi = __builtin_amdgcn_readfirstlane( static_cast<uint32_t>( b >> 32 ) );
-    void* ub = reinterpret_cast<void*>( ( static_cast<uint64_t>( hi ) << 32 ) | lo );
-    // dword 3 of a raw (untyped) buffer resource on gfx9-family GPUs
-    return __builtin_amdgcn_make_buffer_rsrc( ub, 0, static_cast<int>( __builtin_amdgcn_readfirstlane( bytes ) ),
-                                              0x00020000 );
-}
-__device__ __forceinline__ double bufferLoad64( __amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff )
-{
-    return __builtin_bit_cast( double, __builtin_amdgcn_raw_buffer_load_b64( r, voff, soff, 0 ) );
-}
-__device__ __forceinline__ uint8_t bufferLoad8( __amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff )
-{
-    return __builtin_amdgcn_raw_buffer_load_b8( r, voff, soff, 0 );
-}
-
-__device__ __forceinline__ int4 scalarLoad4( const int4* p )
-{
-    const auto* f = ( const __attribute__( ( address_space( 4 ) ) ) int* )( p );
-    return make_int4( f[0], f[1], f[2], f[3] );
-}
-
-// getLinearizedDistance (CabanaPD_Force.hpp:114-138), operation for
-// operation: stretch linearized in eta, force along the reference bond.
-// Stored so that the force passes' coeff * rx / r is coeff * xi_x / xi.
-__device__ __forceinline__ void getLinearizedDistance64( double xi0, double xi1, double xi2, double ui0,
-                                                         double ui1, double ui2, double xj0, double xj1,
-                                                         double xj2, double uj0, double uj1, double uj2,
-                                                         Bond64& b )
-{
-#pragma clang fp contract( off )
-    const double xi_x = xj0 - xi0;
-    const double eta_u = uj0 - ui0;
-    const double xi_y = xj1 - xi1;
-    const double eta_v = uj1 - ui1;
-    const double xi_z = xj2 - xi2;
-    const double eta_w = uj2 - ui2;
-    b.xi = sqrt( xi_x * xi_x + xi_y * xi_y + xi_z * xi_z );
-    b.s = ( xi_x * eta_u + xi_y * eta_v + xi_z * eta_w ) / ( b.xi * b.xi );
-    b.rx = xi_x;
-    b.ry = xi_y;
-    b.rz = xi_z;
-    b.r = b.xi;
-}
-
-// Mixed form of the linearized stretch: s = xi.eta / |xi|^2 in FP32 from the
-// FP64 differences; direction and 1/r are those of the reference bond.
-__device__ __forceinline__ void linearized32( float gx, float gy, float gz, float xi, float xinv, double ui0,
-                                              double ui1, double ui2, double uj0, double uj1, double uj2, Bond32& b )
-{
-    const float ex = static_cast<float>( uj0 - ui0 );
-    const float ey = static_cast<float>( uj1 - ui1 );
-    const float ez = static_cast<float>( uj2 - ui2 );
-    b.rx = gx;
-    b.ry = gy;
-    b.rz = gz;
-    b.xi = xi;
-    b.rinv = xinv;
-    b.s = ( gx * ex + gy * ey + gz * ez ) * ( xinv * xinv );
-}
-
-// Bond geometry of the force and energy passes for the model.
-template <int MODEL>
-__device__ __forceinline__ void bond64( double xi0, double xi1, double xi2, double ui0, double ui1, double ui2,
-                                        double xj0, double xj1, double xj2, double uj0, double uj1, double uj2,
-                                        Bond64& b )
-{
-    if constexpr ( kIsLin<MODEL> )
-        getLinearizedDistance64( xi0, xi1, xi2, ui0, ui1, ui2, xj0, xj1, xj2, uj0, uj1, uj2, b );
-    else
-        getDistance64( xi0, xi1, xi2, ui0, ui1, ui2, xj0, xj1, xj2, uj0, uj1, uj2, b );
-}
-// Linearized stretch of the mixed form, bond vector gathered (x_j - x_i)
-// or from the stencil table (g = (xi_x, xi_y, xi_z, |xi|), xinv = 1/|xi|).
-__device__ __forceinline__ void linearized32g( double xi0, double xi1, double xi2, double ui0, double ui1,
-                                               double ui2, double xj0, double xj1, double xj2, double uj0,
-                                               double uj1, double uj2, Bond32& b )
-{
-    const float gx = static_cast<float>( xj0 - xi0 );
-    const float gy = static_cast<float>( xj1 - xi1 );
-    const float gz = static_cast<float>( xj2 - xi2 );
-    const float g2 = gx * gx + gy * gy + gz * gz;
-    const float xinv = __builtin_amdgcn_rsqf( g2 );
-    linearized32( gx, gy, gz, g2 * xinv, xinv, ui0, ui1, ui2, uj0, uj1, uj2, b );
-}
-
-// ---------------------------------------------------------------------------
-// The FP64 bond arithmetic without the range handling of the compiler's
-// square root and division (the row-window passes).  A bond takes two roots
-// and four divisions by them; the compiler's forms scale each operand into
-// range, iterate and fix up the special cases, every division from a
-// reciprocal of its own (117 VALU instructions per slot of the PMB pass).
-// Here one reciprocal square root starts both the root and the reciprocal of
-// the root (Goldschmidt's iteration, then Newton's), and the divisions by one
-// divisor share it, each corrected by its exact remainder (Markstein):
-// the same iterations, so the results are the correctly rounded ones, the
-// same bits.  That holds
-//   - for operands whose intermediate values neither overflow nor lose bits
-//     to underflow: PDArgs::plain_range (lattice, constants) and the rows'
-//     own test of the staged values (kPlainExp) see to that, together with
-//     the coefficient's bound plainLimit;
-//   - for roots that are neither zero, infinite nor NaN: those make the
-//     stretch NaN, and with it the coefficient;
-//   - for divisors other than 2^k (2 - 2^-52), the one mantissa whose
-//     reciprocal Newton's iteration misses by an ulp: lastBits finds every
-//     divisor whose low word is all ones.
-// A row in which a lane fails one of them is evaluated again by the general
-// code, from the sums as they were before the row.
-// (checked on the GPU against IEEE results: 1e8 roots and quotients, half of
-// them with mantissas within 16 ulp of a power of two, no difference but for
-// the excluded divisors.  The PMB fracture slot takes 75 VALU instructions;
-// 25 steps of the 1.44M-particle plate with their download 28.2 -> 23.6 ms,
-// 50 steps of a 41^3 cube 4.23 -> 3.52 ms, with the LPS model 8.50 -> 7.48.)
-// ---------------------------------------------------------------------------
-constexpr int kPlainExp = 100;   // staged u, x and T: zero or 2^-100 <= |.| < 2^100
-constexpr int kPlainExpAB = 200; // staged lpsA, lpsB: zero or 2^-200 <= |.| < 2^200
-
-struct Root64
-{
-    double r, y; // correctly rounded sqrt(a), and 1 / r to within an ulp
-};
-__device__ __forceinline__ Root64 rootRecip( double a )
-{
-#pragma clang fp contract( off )
-    const double y0 = __builtin_amdgcn_rsq( a );
-    const double g0 = a * y0;
-    const double h0 = 0.5 * y0;
-    const double e = fma( -h0, g0, 0.5 );
-    const double g1 = fma( g0, e, g0 );
-    const double h1 = fma( h0, e, h0 );
-    const double g2 = fma( fma( -g1, g1, a ), h1, g1 );
-    Root64 o;
-    o.r = fma( fma( -g2, g2, a ), h1, g2 );
-    const double y = h1 + h1;
-    o.y = fma( y, fma( -o.r, y, 1.0 ), y );
-    return o;
-}
-// The reciprocal of a divisor that is no root (a particle's m).
-__device__ __forceinline__ double recip64( double b )
-{
-    double y = __builtin_amdgcn_rcp( b );
-    y = fma( y, fma( -b, y, 1.0 ), y );
-    return fma( y, fma( -b, y, 1.0 ), y );
-}
-// a / b, y = 1 / b to within an ulp
-__device__ __forceinline__ double divBy( double a, double b, double y )
-{
-#pragma clang fp contract( off )
-    const double q = a * y;
-    return fma( fma( -b, q, a ), y, q );
-}
-__device__ __forceinline__ uint32_t lowWord( double a )
-{
-    return static_cast<uint32_t>( __builtin_bit_cast( uint64_t, a ) );
-}
-// Every finite nonzero argument has magnitude in [2^-(lim+1), 2^lim) (infinities and
-// NaN pass: they reach the coefficient as NaN).
-__device__ __forceinline__ void expRange( double a, int& lo, int& hi )
-{
-    const int e = __builtin_amdgcn_frexp_exp( a );
-    lo = min( lo, e );
-    hi = max( hi, e );
-}
-
-struct Fast64
-{
-    double xi, r, s, rx, ry, rz, yxi, yr;
-};
-// getDistance64 with shared reciprocals.
-__device__ __forceinline__ void getDistanceFast( double xi0, double xi1, double xi2, double ui0, double ui1,
-                                                 double ui2, double xj0, double xj1, double xj2, double uj0,
-                                                 double uj1, double uj2, Fast64& b )
-{
-#pragma clang fp contract( off )
-    const double xi_x = xj0 - xi0;
-    const double eta_u = uj0 - ui0;
-    const double xi_y = xj1 - xi1;
-    const double eta_v = uj1 - ui1;
-    const double xi_z = xj2 - xi2;
-    const double eta_w = uj2 - ui2;
-    b.rx = xi_x + eta_u;
-    b.ry = xi_y + eta_v;
-    b.rz = xi_z + eta_w;
-    const Root64 r = rootRecip( b.rx * b.rx + b.ry * b.ry + b.rz * b.rz );
-    const Root64 x = rootRecip( xi_x * xi_x + xi_y * xi_y + xi_z * xi_z );
-    b.r = r.r;
-    b.yr = r.y;
-    b.xi = x.r;
-    b.yxi = x.y;
-    b.s = divBy( b.r - b.xi, b.xi, b.yxi );
-}
-
-// Uniform per-wave access to the spec of this wave's slice.
-struct WaveCtx
-{
-    const PDArgs* A;
-    int64_t slice;
-    int32_t epi;
-    int32_t cur;
-};
-
-__device__ __forceinline__ bool waveSetup( const PDArgs* __restrict__ specs,
-                                           const int32_t* __restrict__ tile_spec,
-                                           const int64_t* __restrict__ tile_slice, int32_t epi,
-                                           int32_t parity, int64_t launch, WaveCtx& w )
-{
-    // uniform per wavefront; readfirstlane lets the compiler keep it (and the
-    // addresses derived from it) in scalar registers
-    const int wave = __builtin_amdgcn_readfirstlane( static_cast<int>( threadIdx.x / kSlice ) );
-    const int64_t t = xcdRemap( blockIdx.x, gridDim.x );
-    if ( tile_spec == nullptr )
-    {
-        w.A = specs;
-        w.slice = t * kSlicesPerBlock + wave;
-        w.epi = epi;
-        w.cur = parity;
-    }
-    else
-    {
-        // the tile tables are written by the host before the launch
-        w.A = specs + scalarLoad( tile_spec + t );
-        w.slice = scalarLoad( tile_slice + t ) + wave;
-        // launch < 0: step -1 - launch of a replayed graph, whose first step's
-        // index is the device counter (written by an earlier kernel of the
-        // stream; the scalar cache starts every dispatch invalidated)
-        const int64_t L = launch >= 0 ? launch : scalarLoad( scalarLoad( &w.A->launch_ctr ) ) + ( -1 - launch );
-        w.cur = static_cast<int32_t>( L & 1 ) ^ w.A->parity_offset;
-        w.epi = ( L + 1 < w.A->end_launch ) ? kEpiFinalInitial : kEpiFinal;
-    }
-    return w.slice < w.A->nslices;
-}
-
-// Force BC and body term (CabanaPD_Boundary.hpp:94-157, CabanaPD_BodyTerm.hpp:46-63),
-// then the velocity-Verlet halves (CabanaPD_Integrate.hpp:100-109, 128-134).
-__device__ __forceinline__ void epilogue( const PDArgs& A, int64_t p, int32_t epi, int32_t cur,
-                                          double fx, double fy, double fz )
-{
-#pragma clang fp contract( off )
-    const int64_t n = A.n;
-    if ( epi != kEpiStoreOnly )
-    {
-        if ( A.body )
-        {
-            fx = fx + A.body[p];
-            fy = fy + A.body[n + p];
-            fz = fz + A.body[2 * n + p];
-        }
-        if ( A.bc_kind >= 0 && A.bcflag[p] )
-        {
-            if ( A.bc_kind == PDK_BC_FORCE_VALUE )
-            {
-                fx = A.bc_value;
-                fy = A.bc_value;
-                fz = A.bc_value;
-            }
-            else
-            {
-                fx = fx + A.bc_value;
-                fy = fy + A.bc_value;
-                fz = fz + A.bc_value;
-            }
-        }
-    }
-    A.f[p] = fx;
-    A.f[n + p] = fy;
-    A.f[2 * n + p] = fz;
-    if ( epi == kEpiStoreOnly )
-        return;
-    const double half_dt_m = A.half_dt / A.rho[p];
-    double vx = A.v[p], vy = A.v[n + p], vz = A.v[2 * n + p];
-    vx = vx + half_dt_m * fx;
-    vy = vy + half_dt_m * fy;
-    vz = vz + half_dt_m * fz;
-    if ( epi == kEpiFinalInitial )
-    {
-        vx = vx + half_dt_m * fx;
-        vy = vy + half_dt_m * fy;
-        vz = vz + half_dt_m * fz;
-        const double* u = A.U[cur];
-        double* un = A.U[cur ^ 1];
-        un[p] = u[p] + A.dt * vx;
-        un[n + p] = u[n + p] + A.dt * vy;
-        un[2 * n + p] = u[2 * n + p] + A.dt * vz;
-    }
-    A.v[p] = vx;
-    A.v[n + p] = vy;
-    A.v[2 * n + p] = vz;
-}
-
 // ---------------------------------------------------------------------------
 // Force pass: Force<PMB|LPS, NoFracture|Fracture>::computeForceFull
 // (force/CabanaPD_PMB.hpp:89-125,222-287; force/CabanaPD_LPS.hpp:143-181,380-447)
@@ -984,1047 +516,6 @@ __global__ __launch_bounds__( kBlock ) __attribute__( ( amdgpu_waves_per_eu( ( P
 }
 
 // ---------------------------------------------------------------------------
-// The same force pass with the neighbor data staged in LDS (stencil-slot form
-// on lattice rows).  For a lattice row r = (dy, dz) of the stencil, slots
-// q0 .. q0+c-1 of the 64 lanes of a slice have their neighbors at the
-// contiguous ids g .. g+63+c-1 (g = first id of the slice + the row's offset):
-// the wave loads that window once with coalesced loads, stores it in its LDS
-// buffer, and slot q0+t of lane L reads window[L + t].  The window of the next
-// row is loaded while the current row is evaluated.  Per slot, one
-// wave-uniform 64-bit word (scalar load) gates the lanes: the intact word
-// under fracture (breaks and pre-notches only clear bits, so it is a subset
-// of the existence word) or the existence word.  Evaluation order and
-// arithmetic are kForce's, so results are identical.
-// ---------------------------------------------------------------------------
-// Waves per SIMD the register allocator must leave room for (the attribute
-// below): 6 for the PMB passes (80 VGPRs, one spill outside the loops;
-// measured 6 % faster on the fracture plate than the unconstrained
-// allocation at 5 waves); LPS (models 1 and 5) stays unconstrained, since
-// forcing it spills inside the slot loop (mixed LPS at 6 waves: 8 VGPRs
-// spilled, 0.349 -> 0.354 ms on a 128^3 cube).
-template <int MODEL, bool FRAC, int PREC, bool GEN>
-__global__ __launch_bounds__( kBlock ) __attribute__( ( amdgpu_waves_per_eu( ( MODEL == 1 || MODEL == 5 ) ? 1 : 6, 8 ) ) ) void
-kForceRows( const PDArgs* __restrict__ specs,
-                                                        const int32_t* __restrict__ tile_spec,
-                                                        const int64_t* __restrict__ tile_slice,
-                                                        int32_t epi, int32_t parity, int64_t launch,
-                                                        int32_t accumulate )
-{
-#pragma clang fp contract( off )
-    constexpr int kW = kSlice + kRowMaxSlots - 1;  // window width
-    constexpr int NX = ( PREC == kF64 ) ? 3 : 0;    // staged x components
-    // mixed form (non-linear stretch): the bond vector r = xi + (u_j - u_i)
-    // in FP64 from the slot's FP64 stencil offset xi; the windows hold u only
-    constexpr bool XV = ( PREC == kMixed ) && !kIsLin<MODEL>;
-    constexpr int NAB = kIsLps<MODEL> ? 2 : 0;  // staged lpsA, lpsB
-    constexpr bool FAST = ( PREC == kF64 ) && !kIsLin<MODEL>; // shared reciprocals where they give the same bits
-    constexpr int KV = 3 + NX + NAB;                // staged vol (GEN)
-    constexpr int KNF = KV + 1;                     // staged no-fail flag (GEN)
-    constexpr int NC = KV + ( GEN ? 2 : 0 );
-    // channel stride: PMB mixed rows pad each channel to 128 values, so the
-    // second window half is stored by every lane (no per-row store masks);
-    // values past the row's window are never read
-    constexpr bool PAD = ( PREC == kMixed ) && !kIsLps<MODEL> && !GEN;
-    constexpr int kWS = PAD ? 2 * kSlice : kW;
-    __shared__ double win[kSlicesPerBlock][2][NC][kWS];
-    WaveCtx w;
-    if ( !waveSetup( specs, tile_spec, tile_slice, epi, parity, launch, w ) )
-        return; // waves are independent: no block-level synchronisation
-    const PDArgs& A = *w.A;
-    const int wv = __builtin_amdgcn_readfirstlane( static_cast<int>( threadIdx.x / kSlice ) );
-    const int lane = threadIdx.x & ( kSlice - 1 );
-    const int64_t n = scalarLoad( &A.n );
-    const int64_t p0 = w.slice * kSlice;
-    const int64_t p = p0 + lane;
-    const bool valid = p < n;
-    const int64_t pc = valid ? p : p0;
-    // Base pointers, the row table and the slice table through scalar loads
-    // (the argument block and the tables are written by the host only), so
-    // window addresses are an SGPR base plus the lane offset.
-    const double* __restrict__ x = scalarLoad( &A.x );
-    const double* __restrict__ u = scalarLoad( &A.U[w.cur] );
-    const int4* __restrict__ rows = scalarLoad( &A.rows );
-    // particle i: reference position (FP64 form) and displacement
-    double xi0 = 0.0, xi1 = 0.0, xi2 = 0.0;
-    if constexpr ( PREC == kF64 )
-    {
-        xi0 = x[pc];
-        xi1 = x[n + pc];
-        xi2 = x[2 * n + pc];
-    }
-    const double ui0 = u[pc], ui1 = u[n + pc], ui2 = u[2 * n + pc];
-    // Per-slot lane masks of the slice: the intact words (a subset of the
-    // existence words, so they alone gate the fracture forms) or, without
-    // fracture, the existence words.  Lanes past n hold no bonds.
-    // (the argument block and the slice table are written by the host only)
-    const int64_t row0 = scalarLoad( scalarLoad( &A.slice_ptr ) + w.slice );
-    uint64_t* __restrict__ bits = scalarLoad( &A.intact ) + row0;
-    const uint64_t* __restrict__ mwords = FRAC ? bits : scalarLoad( &A.exist ) + row0;
-    const float4* __restrict__ sten = scalarLoad( &A.stencil );
-    const float4* __restrict__ saux = scalarLoad( &A.stencil_aux );
-    const double* __restrict__ sxiv = scalarLoad( &A.stencil_xiv );
-    const bool nf_i = FRAC ? ( A.nofail[pc] != 0 ) : false;
-    // Loop-invariant scalars held in registers (the args block lives in
-    // global memory, which the bit-word stores could alias).
-    const double c = A.c;
-    const double bcc = A.bcc;
-    const float c32 = static_cast<float>( A.c );
-    const double s0near = A.s0 - 0x1p-30 * ( 1.0 + A.s0 );
-    const double volu = A.vol_value;
-    const float s0f = A.s0f;
-    const float bandK = A.bandK;
-    // lower edge of the decision path: every stretch within bandK of s0 or
-    // above it lies at or above s0 - 2 bandK
-    const float s0lo = s0f - 2.0f * bandK;
-    // uniform volume: c vol (PMB) or vol (LPS) scales each FP32 row sum
-    const double rscale = GEN ? 1.0 : A.row_scale;
-    const int infl1 = A.influence;
-    // lanes whose particle may break bonds (every lane of the wave is active here)
-    const uint64_t nfi_ok = FRAC ? __ballot( !nf_i ) : 0ull;
-    double Ai = 0.0, Bi = 0.0;
-    if constexpr ( kIsLps<MODEL> )
-    {
-        Ai = A.lpsA[pc]; // theta_coeff * theta_i / m_i
-        Bi = A.lpsB[pc]; // s_coeff / m_i
-    }
-
-    double fx = 0.0, fy = 0.0, fz = 0.0;
-    if ( accumulate && valid )
-    {
-        fx = A.f[p];
-        fy = A.f[n + p];
-        fz = A.f[2 * n + p];
-    }
-    // XV: the bond forces fr r (FP32 fr, FP64 bond vector r) summed in FP64
-    double sx = 0.0, sy = 0.0, sz = 0.0;
-
-    const double* src[KV];
-    src[0] = u;
-    src[1] = u + n;
-    src[2] = u + 2 * n;
-    if constexpr ( NX )
-    {
-        src[3] = x;
-        src[4] = x + n;
-        src[5] = x + 2 * n;
-    }
-    if constexpr ( NAB )
-    {
-        src[3 + NX] = scalarLoad( &A.lpsA );
-        src[4 + NX] = scalarLoad( &A.lpsB );
-    }
-    const double* __restrict__ volp = scalarLoad( &A.vol );
-    const uint8_t* __restrict__ nfp = scalarLoad( &A.nofail );
-    double v0[NC], v1[NC];
-#pragma unroll
-    for ( int k = 0; k < NC; k++ )
-        v1[k] = 0.0;
-    // Row tables exist only for n < 2^28 (byte sizes and offsets fit 32 bits).
-    const int32_t p032 = static_cast<int32_t>( p0 );
-    const uint32_t nbytes = static_cast<uint32_t>( n ) * 8u;
-    __amdgpu_buffer_rsrc_t rs[KV + ( GEN ? 1 : 0 )];
-#pragma unroll
-    for ( int k = 0; k < KV; k++ )
-        rs[k] = bufferOf( src[k], nbytes );
-    const __amdgpu_buffer_rsrc_t rnf = bufferOf( nfp, GEN ? static_cast<uint32_t>( n ) : 0u );
-    if constexpr ( GEN )
-        rs[KV] = bufferOf( volp, nbytes );
-    const uint32_t lane8 = static_cast<uint32_t>( lane ) * 8u;
-    // 64 window values starting at id g (uniform) into dst.
-    auto loadHalf = [&]( double* dst, int32_t g ) {
-        // g >= 0: lane offset + uniform start; g < 0: per-lane offsets, the
-        // negative ones wrap out of range and read 0
-        const uint32_t vo = g >= 0 ? lane8 : static_cast<uint32_t>( g + lane ) * 8u;
-        const uint32_t so = g >= 0 ? static_cast<uint32_t>( g ) * 8u : 0u;
-#pragma unroll
-        for ( int k = 0; k < KV; k++ )
-            dst[k] = bufferLoad64( rs[k], vo, so );
-        if constexpr ( GEN )
-        {
-            dst[KV] = bufferLoad64( rs[KV], vo, so );
-            dst[KNF] = ( FRAC && bufferLoad8( rnf, vo >> 3, so >> 3 ) != 0 ) ? 1.0 : 0.0;
-        }
-    };
-    // Window of row r: ids g .. g + 63 (every lane) and g + 64 .. g + 64 + c - 2
-    // (lanes < c - 1).
-    auto loadRow = [&]( int r ) {
-        const int4 R = scalarLoad4( rows + r );
-        const int32_t g = p032 + R.z; // uniform
-        loadHalf( v0, g );
-        if ( lane < R.y - 1 )
-            loadHalf( v1, g + kSlice );
-    };
-
-    // FAST: the range test of a row's staged values and of particle i's own
-    const bool plain = FAST && scalarLoad( &A.plain_range ) != 0;
-    int own_lo = 0, own_hi = 0;
-    if constexpr ( FAST )
-    {
-        expRange( ui0, own_lo, own_hi );
-        expRange( ui1, own_lo, own_hi );
-        expRange( ui2, own_lo, own_hi );
-    }
-    auto rowPlain = [&]() {
-        int lo = own_lo, hi = own_hi;
-#pragma unroll
-        for ( int q = 0; q < 3; q++ )
-        {
-            expRange( v0[q], lo, hi );
-            expRange( v1[q], lo, hi );
-        }
-        bool out = lo < -kPlainExp || hi > kPlainExp;
-        if constexpr ( NAB )
-        {
-            int la = 0, ha = 0;
-#pragma unroll
-            for ( int q = 3 + NX; q < 5 + NX; q++ )
-            {
-                expRange( v0[q], la, ha );
-                expRange( v1[q], la, ha );
-            }
-            expRange( Ai, la, ha );
-            expRange( Bi, la, ha );
-            out = out || la < -kPlainExpAB || ha > kPlainExpAB;
-        }
-        return __ballot( out ) == 0;
-    };
-    const int nrows = scalarLoad( &A.nrows );
-    loadRow( 0 );
-    for ( int r = 0; r < nrows; r++ )
-    {
-        const int4 R = scalarLoad4( rows + r );
-        double* __restrict__ wb = &win[wv][r & 1][0][0];
-#pragma unroll
-        for ( int k = 0; k < NC; k++ )
-        {
-            wb[k * kWS + lane] = v0[k];
-            if ( PAD || lane < R.y - 1 )
-                wb[k * kWS + kSlice + lane] = v1[k];
-        }
-        // a tiny (or huge) displacement in the row: only bonds without force
-        // may take the shared reciprocals
-        const double limit = FAST && rowPlain() ? 0x1p600 : 0.0;
-        // LDS operations of one wavefront complete in order; the fences keep
-        // the compiler from moving the window reads above the stores.
-        __builtin_amdgcn_fence( __ATOMIC_RELEASE, "wavefront" );
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence( __ATOMIC_ACQUIRE, "wavefront" );
-        if ( r + 1 < nrows )
-            loadRow( r + 1 );
-        float px = 0.0f, py = 0.0f, pz = 0.0f; // FP32 sum of this row's bond forces (mixed form)
-        // the row's slots q = R.x + t through row base pointers, so the
-        // unrolled slots address their words and table entries with
-        // immediate offsets (no per-slot 64-bit address arithmetic)
-        const uint64_t* __restrict__ mw_r = mwords + R.x;
-        uint64_t* __restrict__ bits_r = bits + R.x;
-        const float4* __restrict__ st_r = sten + R.x;
-        const float4* __restrict__ sa_r = saux + R.x;
-        const double* __restrict__ xv_r = sxiv + 4 * R.x;
-        // XV: xi_y - u_i,y and xi_z - u_i,z, one value each for the row (the
-        // slots of a lattice row differ in xi_x only)
-        double ay = 0.0, az = 0.0;
-        if constexpr ( XV )
-        {
-            ay = scalarLoad( xv_r + kXiY ) - ui1;
-            az = scalarLoad( xv_r + kXiZ ) - ui2;
-        }
-        // The wave-uniform data of slot t: its intact word (fracture) or
-        // existence word, its FP32 stencil entries and (XV) its FP64 offset
-        // and |xi|^2 (one 32-byte record).  Loading slot t + 1's data while
-        // slot t computes measured slower on the fracture plate (0.209 vs
-        // 0.202 ms): the register copies between slots cost more scalar
-        // issue than the hidden load latency saved.
-        // (the 48-byte records of the other row passes, one scalar load for
-        // all of a slot's values, measured 2.8 % slower here: the 32-byte FP64
-        // record and the FP32 table entry are two loads but stay within one
-        // scalar-cache line each)
-        struct SlotK
-        {
-            uint64_t ww;
-            float4 g, ga;
-            double x0, x2d;
-        };
-        auto loadK = [&]( const int t ) __attribute__( ( always_inline ) ) {
-            SlotK K{};
-            K.ww = scalarLoad( mw_r + t );
-            if constexpr ( PREC == kMixed )
-            {
-                K.g = scalarLoad4( st_r + t );
-                K.ga = scalarLoad4( sa_r + t ); // (1/|xi|, |xi|^2, infl |xi|, infl |xi|^2)
-                if constexpr ( XV )
-                {
-                    const double* xv = xv_r + 4 * t;
-                    K.x0 = scalarLoad( xv + kXiX );
-                    K.x2d = scalarLoad( xv + kXi2 );
-                }
-            }
-            return K;
-        };
-        auto slot = [&]( const int t, const SlotK& K ) __attribute__( ( always_inline ) ) {
-            const uint64_t ww = K.ww;
-            // A slot with no live bond in the wave (the slots past a face of
-            // the specimen, fully broken slots) adds nothing: the LPS passes
-            // skip it (measured 8 % faster on the 128^3 LPS fracture cube; the
-            // branch made the PMB plate pass 3 % slower, so PMB evaluates
-            // and masks).  The FP64 form skips through its exec mask.
-            if constexpr ( PREC == kMixed && kIsLps<MODEL> )
-                if ( ww == 0 )
-                    return;
-            // The window always holds readable values; bonds that do not
-            // exist are masked out below.
-            const double* __restrict__ wr = wb + lane + t;
-            const double uj0 = wr[0], uj1 = wr[kWS], uj2 = wr[2 * kWS];
-            // candidates for the break test: intact, neither end no-fail
-            // (LPS tests nofail(i) twice, force/CabanaPD_LPS.hpp:417-418)
-            uint64_t cand = 0;
-            if constexpr ( FRAC )
-            {
-                cand = ww & nfi_ok;
-                if constexpr ( !kIsLps<MODEL> && GEN )
-                    cand &= __ballot( wr[KNF * kWS] == 0.0 );
-            }
-            // Masks below are wave-uniform (ballots in converged code).
-            uint64_t brkm = 0; // bonds that break in this pass
-            if constexpr ( PREC == kF64 )
-            {
-                bool brk = false;
-                if ( __builtin_amdgcn_inverse_ballot_w64( ww ) )
-                {
-                    const double vj = GEN ? wr[KV * kWS] : volu;
-                    Bond64 b;
-                    bond64<MODEL>( xi0, xi1, xi2, ui0, ui1, ui2, wr[3 * kWS], wr[4 * kWS], wr[5 * kWS], uj0, uj1,
-                                   uj2, b );
-                    if constexpr ( FRAC )
-                        brk = criticalStretch64( b.r, b.xi, bcc ) && __builtin_amdgcn_inverse_ballot_w64( cand );
-                    if ( !brk )
-                    {
-                        double coeff;
-                        if constexpr ( !kIsLps<MODEL> )
-                            coeff = c * b.s * vj;
-                        else
-                        {
-                            const double infl = infl1 ? 1.0 / b.xi : 1.0;
-                            coeff = ( Ai + wr[( 3 + NX ) * kWS] + b.s * ( Bi + wr[( 4 + NX ) * kWS] ) ) * infl * b.xi * vj;
-                        }
-                        fx += coeff * b.rx / b.r;
-                        fy += coeff * b.ry / b.r;
-                        fz += coeff * b.rz / b.r;
-                    }
-                }
-                if constexpr ( FRAC )
-                    brkm = __ballot( brk );
-            }
-            else
-            {
-                const float4 g = K.g;
-                const float4 ga = K.ga;
-                Bond32 b;
-                double r0 = 0.0, r1 = 0.0, r2 = 0.0; // XV: the FP64 bond vector
-                if constexpr ( XV )
-                {
-                    r0 = ( uj0 - ui0 ) + K.x0;
-                    r1 = uj1 + ay;
-                    r2 = uj2 + az;
-                    mixedBond( r0, r1, r2, K.x2d, g.w, b );
-                }
-                else
-                    linearized32( g.x, g.y, g.z, g.w, ga.x, ui0, ui1, ui2, uj0, uj1, uj2, b );
-                if constexpr ( FRAC )
-                {
-                    // FP32 decision, except within bandK of s0 where the
-                    // reference's FP64 test decides.  One compare first:
-                    // only a wave with a candidate at or above s0 - 2 bandK
-                    // (rare: bonds near breaking) takes the decision path.
-                    if ( __ballot( b.s >= s0lo ) & cand )
-                    {
-                    const uint64_t inb = __ballot( fabsf( b.s - s0f ) <= bandK ) & cand;
-                    brkm = __ballot( b.s > s0f ) & cand & ~inb;
-                    if ( inb )
-                    {
-                        bool crit = false;
-                        if ( __builtin_amdgcn_inverse_ballot_w64( inb ) )
-                        {
-                            // neighbor j = p + R.z + t: uniform base + lane; the
-                            // reference positions of i and j are loaded here
-                            // (rare path; the compiler barrier keeps the loads of
-                            // x_i from being hoisted into registers held for the
-                            // whole pass), the displacements are the registers
-                            // and the window
-                            __asm__ volatile( "" ::: "memory" );
-                            const int64_t jo = p0 + R.z + t;
-                            const double* __restrict__ xj = x + jo;
-                            const double* __restrict__ xp = x + p0;
-                            Bond64 e;
-                            getDistance64( xp[lane], ( xp + n )[lane], ( xp + 2 * n )[lane], ui0, ui1, ui2, xj[lane],
-                                           ( xj + n )[lane], ( xj + 2 * n )[lane], uj0, uj1, uj2, e );
-                            crit = criticalStretch64( e.r, e.xi, bcc );
-                        }
-                        brkm |= __ballot( crit ) & inb;
-                    }
-                    }
-                }
-                // dead lanes (absent, broken or breaking bonds) add exactly
-                // zero: their window values are finite, fr is selected to 0
-                const bool live = __builtin_amdgcn_inverse_ballot_w64( ww & ~brkm );
-                float fr;
-                if constexpr ( !kIsLps<MODEL> )
-                    fr = ( GEN ? ( c32 * static_cast<float>( wr[KV * kWS] ) ) * b.s : b.s ) * b.rinv;
-                else
-                {
-                    const float coeff = static_cast<float>( Ai + wr[( 3 + NX ) * kWS] ) +
-                                        b.s * static_cast<float>( Bi + wr[( 4 + NX ) * kWS] );
-                    fr = ( GEN ? ( coeff * ga.z ) * static_cast<float>( wr[KV * kWS] ) : coeff * ga.z ) * b.rinv;
-                }
-                fr = live ? fr : 0.0f;
-                if constexpr ( XV )
-                {
-                    const double frd = static_cast<double>( fr );
-                    sx = fma( frd, r0, sx );
-                    sy = fma( frd, r1, sy );
-                    sz = fma( frd, r2, sz );
-                }
-                else
-                {
-                    px = fmaf( fr, b.rx, px );
-                    py = fmaf( fr, b.ry, py );
-                    pz = fmaf( fr, b.rz, pz );
-                }
-            }
-            if constexpr ( FRAC )
-            {
-                // wave-uniform test first (rare: a bond of the wave breaks),
-                // then one lane writes the word
-                if ( __builtin_expect( brkm != 0, 0 ) )
-                {
-                    if ( lane == 0 )
-                        bits_r[t] = ww & ~brkm;
-                }
-            }
-        };
-        // FP64 with shared reciprocals: the lanes whose bond the general code
-        // has to evaluate (nothing of such a lane is kept; a bond that breaks
-        // in another lane is recorded, and breaks again if the row is
-        // evaluated again).
-        auto slotFast = [&]( const int t, const double lim ) __attribute__( ( always_inline ) ) {
-            const uint64_t ww = scalarLoad( mw_r + t );
-            const double* __restrict__ wr = wb + lane + t;
-            bool brk = false, gen = false;
-            if ( __builtin_amdgcn_inverse_ballot_w64( ww ) )
-            {
-                const double vj = GEN ? wr[KV * kWS] : volu;
-                Fast64 b;
-                getDistanceFast( xi0, xi1, xi2, ui0, ui1, ui2, wr[3 * kWS], wr[4 * kWS], wr[5 * kWS], wr[0], wr[kWS],
-                                 wr[2 * kWS], b );
-                if constexpr ( FRAC )
-                {
-                    // a bond below s0 by more than rounding cannot break: the
-                    // reference's test runs only in a wave with a stretch near
-                    // s0 or above it
-                    if ( __ballot( b.s >= s0near ) )
-                    {
-                        bool ok = !nf_i;
-                        if constexpr ( !kIsLps<MODEL> && GEN )
-                            ok = ok && wr[KNF * kWS] == 0.0;
-                        brk = criticalStretch64( b.r, b.xi, bcc ) && ok;
-                    }
-                }
-                double coeff;
-                if constexpr ( !kIsLps<MODEL> )
-                    coeff = c * b.s * vj;
-                else
-                {
-                    const double infl = infl1 ? 1.0 / b.xi : 1.0;
-                    coeff = ( Ai + wr[( 3 + NX ) * kWS] + b.s * ( Bi + wr[( 4 + NX ) * kWS] ) ) * infl * b.xi * vj;
-                }
-                gen = !( fabs( coeff ) <= lim ) || max( lowWord( b.r ), lowWord( b.xi ) ) == 0xffffffffu;
-                brk = brk && !gen;
-                if ( !brk )
-                {
-                    fx += divBy( coeff * b.rx, b.r, b.yr );
-                    fy += divBy( coeff * b.ry, b.r, b.yr );
-                    fz += divBy( coeff * b.rz, b.r, b.yr );
-                }
-            }
-            if constexpr ( FRAC )
-            {
-                const uint64_t brkm = __ballot( brk );
-                if ( __builtin_expect( brkm != 0, 0 ) )
-                {
-                    if ( lane == 0 )
-                        bits_r[t] = ww & ~brkm;
-                }
-            }
-            return __ballot( gen );
-        };
-        // Mixed forms: the slots of a row (at most kRowMaxSlots) unrolled, so
-        // the window reads take immediate offsets and the PMB pass fits 70
-        // VGPRs without spills (7 % faster on the fracture plate, 2 % on the
-        // LPS cube; unrolling the FP64 form measured slower)
-        if constexpr ( PREC == kMixed )
-        {
-#pragma unroll
-            for ( int t = 0; t < kRowMaxSlots; t++ )
-                if ( t < R.y )
-                    slot( t, loadK( t ) );
-        }
-        else
-        {
-            if constexpr ( FAST )
-            {
-                if ( plain )
-                {
-                    const double fx0 = fx, fy0 = fy, fz0 = fz;
-                    uint64_t bad = 0;
-                    for ( int t = 0; t < R.y; t++ )
-                        bad |= slotFast( t, limit );
-                    if ( __builtin_expect( bad == 0, 1 ) )
-                        continue;
-                    fx = fx0;
-                    fy = fy0;
-                    fz = fz0;
-                }
-            }
-            for ( int t = 0; t < R.y; t++ )
-                slot( t, loadK( t ) );
-        }
-        if constexpr ( PREC == kMixed && !XV )
-        {
-            fx = fma( rscale, static_cast<double>( px ), fx );
-            fy = fma( rscale, static_cast<double>( py ), fy );
-            fz = fma( rscale, static_cast<double>( pz ), fz );
-        }
-    }
-    if constexpr ( XV )
-    {
-        fx = fma( rscale, sx, fx );
-        fy = fma( rscale, sy, fy );
-        fz = fma( rscale, sz, fz );
-    }
-    if ( !valid )
-        return;
-    epilogue( A, p, w.epi, w.cur, fx, fy, fz );
-}
-
-// ---------------------------------------------------------------------------
-// The row-window force pass for specimens with per-particle features: several
-// materials (pair tables), TemperatureDependent (per-particle temperature) and
-// ElasticPerfectlyPlastic (per-bond plastic stretch).  FEAT is a set of
-// kFeat* bits.  The window channels are u, x (FP64 form), lpsA/lpsB (LPS),
-// the volume, a tag (2 x material + no-fail flag) and the temperature; the
-// plastic stretch of slot q sits at splas[(row0 + q) * 64 + lane].  Per bond
-// the arithmetic and the order of the sums are those of the gather pass
-// (kForce with the slot layout), so both forms give identical results.
-// ---------------------------------------------------------------------------
-enum : int
-{
-    kFeatMT = 1, // pair tables (multi-material)
-    kFeatTH = 2, // temperature-dependent stretch
-    kFeatEP = 4  // elastic-perfectly-plastic bonds
-};
-
-// Waves per SIMD the register allocator must leave room for: 6 for the mixed
-// PMB instances with several materials or a plastic stretch (measured 8 % and
-// 10 % faster on the fracture plate than at 4-5 waves); the temperature
-// instances spill at 6 and stay unconstrained.
-template <int MODEL, bool FRAC, int PREC, int FEAT>
-__global__ __launch_bounds__( kBlock ) __attribute__( ( amdgpu_waves_per_eu( ( PREC == kMixed && !kIsLps<MODEL> && ( FEAT == kFeatMT || FEAT == kFeatEP ) ) ? 6 : 1, 8 ) ) ) void kForceRowsF( const PDArgs* __restrict__ specs,
-                                                         const int32_t* __restrict__ tile_spec,
-                                                         const int64_t* __restrict__ tile_slice,
-                                                         int32_t epi, int32_t parity, int64_t launch,
-                                                         int32_t accumulate )
-{
-#pragma clang fp contract( off )
-    constexpr bool MT = ( FEAT & kFeatMT ) != 0;
-    constexpr bool TH = ( FEAT & kFeatTH ) != 0 && !kIsLps<MODEL>;
-    constexpr bool EP = ( FEAT & kFeatEP ) != 0 && !kIsLps<MODEL>;
-    constexpr int kW = kSlice + kRowMaxSlots - 1; // window width
-    constexpr int NX = ( PREC == kF64 ) ? 3 : 0;  // staged x components
-    constexpr int NAB = kIsLps<MODEL> ? 2 : 0;    // staged lpsA, lpsB
-    constexpr int KV = 3 + NX + NAB;              // volume
-    constexpr int KT = KV + 1;                    // tag: 2 x material + no-fail flag
-    constexpr bool TAG = MT || ( FRAC && !kIsLps<MODEL> );
-    constexpr int KH = KT + ( TAG ? 1 : 0 );      // temperature
-    constexpr int NC = KH + ( TH ? 1 : 0 );
-    // one buffer per wave: the next row's window waits in registers until
-    // the current row's reads are done
-    __shared__ double win[kSlicesPerBlock][NC][kW];
-    // several materials: the pair tables (c, bond_break_coeff, FP32 s0 and
-    // band) of the block's spec, indexed 4 a + b
-    __shared__ double tab_c[MT ? 16 : 1], tab_bcc[MT ? 16 : 1];
-    __shared__ float tab_s0[MT ? 16 : 1], tab_band[MT ? 16 : 1];
-    WaveCtx w;
-    const bool active = waveSetup( specs, tile_spec, tile_slice, epi, parity, launch, w );
-    if constexpr ( MT )
-    {
-        // every wave of a block belongs to one spec
-        if ( threadIdx.x < 16 )
-        {
-            tab_c[threadIdx.x] = w.A->mat_c[threadIdx.x];
-            tab_bcc[threadIdx.x] = w.A->mat_bcc[threadIdx.x];
-            tab_s0[threadIdx.x] = w.A->mat_s0f[threadIdx.x];
-            tab_band[threadIdx.x] = w.A->mat_bandK[threadIdx.x];
-        }
-        __syncthreads();
-    }
-    if ( !active )
-        return; // waves are otherwise independent: no further block-level synchronisation
-    const PDArgs& A = *w.A;
-    const int wv = __builtin_amdgcn_readfirstlane( static_cast<int>( threadIdx.x / kSlice ) );
-    const int lane = threadIdx.x & ( kSlice - 1 );
-    const int64_t n = scalarLoad( &A.n );
-    const int64_t p0 = w.slice * kSlice;
-    const int64_t p = p0 + lane;
-    const bool valid = p < n;
-    const int64_t pc = valid ? p : p0;
-    const double* __restrict__ x = scalarLoad( &A.x );
-    const double* __restrict__ u = scalarLoad( &A.U[w.cur] );
-    const int4* __restrict__ rows = scalarLoad( &A.rows );
-    double xi0 = 0.0, xi1 = 0.0, xi2 = 0.0;
-    if constexpr ( PREC == kF64 )
-    {
-        xi0 = x[pc];
-        xi1 = x[n + pc];
-        xi2 = x[2 * n + pc];
-    }
-    const double ui0 = u[pc], ui1 = u[n + pc], ui2 = u[2 * n + pc];
-    const int64_t row0 = scalarLoad( scalarLoad( &A.slice_ptr ) + w.slice );
-    uint64_t* __restrict__ bits = scalarLoad( &A.intact ) + row0;
-    const uint64_t* __restrict__ mwords = FRAC ? bits : scalarLoad( &A.exist ) + row0;
-    const double* __restrict__ srec = scalarLoad( &A.stencil_rec );
-    const uint8_t* __restrict__ nfp = scalarLoad( &A.nofail );
-    const uint8_t* __restrict__ mtp = MT ? scalarLoad( &A.mtype ) : nullptr;
-    const double* __restrict__ tmpp = TH ? scalarLoad( &A.temp ) : nullptr;
-    double* __restrict__ spl = EP ? scalarLoad( &A.splas ) + row0 * kSlice + lane : nullptr;
-    const bool nf_i = FRAC ? ( nfp[pc] != 0 ) : false;
-    const int ti4 = MT ? 4 * static_cast<int>( mtp[pc] ) : 0;
-    const double Ti = TH ? tmpp[pc] : 0.0;
-    const double c = A.c;
-    const double bcc = A.bcc;
-    const float c32 = static_cast<float>( A.c );
-    const float s0f = A.s0f;
-    const float bandK = A.bandK;
-    const int infl1 = A.influence;
-    // uniform volume: c vol (PMB, one material) or vol (LPS) scales the sum
-    // (as in the gather pass)
-    const bool fold = A.vol_uniform != 0 && !( FRAC && A.any_nofail != 0 ) && !( MT && !kIsLps<MODEL> );
-    const double rscale = ( PREC == kMixed && fold ) ? A.row_scale : 1.0;
-    double Ai = 0.0, Bi = 0.0;
-    if constexpr ( kIsLps<MODEL> )
-    {
-        Ai = A.lpsA[pc]; // theta_coeff * theta_i / m_i
-        Bi = A.lpsB[pc]; // s_coeff / m_i
-    }
-    double fx = 0.0, fy = 0.0, fz = 0.0;
-    if ( accumulate && valid )
-    {
-        fx = A.f[p];
-        fy = A.f[n + p];
-        fz = A.f[2 * n + p];
-    }
-    double sx = 0.0, sy = 0.0, sz = 0.0; // mixed form: the bond forces fr r summed in FP64
-
-    const double* src[KV + 1];
-    src[0] = u;
-    src[1] = u + n;
-    src[2] = u + 2 * n;
-    if constexpr ( NX )
-    {
-        src[3] = x;
-        src[4] = x + n;
-        src[5] = x + 2 * n;
-    }
-    if constexpr ( NAB )
-    {
-        src[3 + NX] = scalarLoad( &A.lpsA );
-        src[4 + NX] = scalarLoad( &A.lpsB );
-    }
-    src[KV] = scalarLoad( &A.vol );
-    // row tables exist only for n < 2^28 (byte sizes and offsets fit 32 bits)
-    const int32_t p032 = static_cast<int32_t>( p0 );
-    const uint32_t nbytes = static_cast<uint32_t>( n ) * 8u;
-    __amdgpu_buffer_rsrc_t rs[KV + 1];
-#pragma unroll
-    for ( int k = 0; k <= KV; k++ )
-        rs[k] = bufferOf( src[k], nbytes );
-    const __amdgpu_buffer_rsrc_t rnf = bufferOf( nfp, static_cast<uint32_t>( n ) );
-    const __amdgpu_buffer_rsrc_t rmt = bufferOf( MT ? mtp : nfp, static_cast<uint32_t>( n ) );
-    const __amdgpu_buffer_rsrc_t rth = bufferOf( TH ? tmpp : src[0], nbytes );
-    const uint32_t lane8 = static_cast<uint32_t>( lane ) * 8u;
-    double v0[NC], v1[NC];
-#pragma unroll
-    for ( int k = 0; k < NC; k++ )
-        v1[k] = 0.0;
-    auto loadHalf = [&]( double* dst, int32_t g ) {
-        // g >= 0: lane offset + uniform start; g < 0: per-lane offsets, the
-        // negative ones wrap out of range and read 0
-        const uint32_t vo = g >= 0 ? lane8 : static_cast<uint32_t>( g + lane ) * 8u;
-        const uint32_t so = g >= 0 ? static_cast<uint32_t>( g ) * 8u : 0u;
-#pragma unroll
-        for ( int k = 0; k <= KV; k++ )
-            dst[k] = bufferLoad64( rs[k], vo, so );
-        if constexpr ( TAG )
-        {
-            int tag = 0;
-            if constexpr ( FRAC && !kIsLps<MODEL> )
-                tag = bufferLoad8( rnf, vo >> 3, so >> 3 ) != 0 ? 1 : 0;
-            if constexpr ( MT )
-                tag += 2 * static_cast<int>( bufferLoad8( rmt, vo >> 3, so >> 3 ) );
-            dst[KT] = static_cast<double>( tag );
-        }
-        if constexpr ( TH )
-            dst[KH] = bufferLoad64( rth, vo, so );
-    };
-    auto loadRow = [&]( int r ) {
-        const int4 R = scalarLoad4( rows + r );
-        const int32_t g = p032 + R.z; // uniform
-        loadHalf( v0, g );
-        if ( lane < R.y - 1 )
-            loadHalf( v1, g + kSlice );
-    };
-
-    // FP64: rows of ordinary values take the shared reciprocals (see kForceRows)
-    constexpr bool FAST = ( PREC == kF64 );
-    const bool plain = FAST && scalarLoad( &A.plain_range ) != 0;
-    int own_lo = 0, own_hi = 0;
-    if constexpr ( FAST )
-    {
-        expRange( ui0, own_lo, own_hi );
-        expRange( ui1, own_lo, own_hi );
-        expRange( ui2, own_lo, own_hi );
-        expRange( Ti, own_lo, own_hi );
-    }
-    auto rowPlain = [&]() {
-        int lo = own_lo, hi = own_hi;
-#pragma unroll
-        for ( int q = 0; q < 3; q++ )
-        {
-            expRange( v0[q], lo, hi );
-            expRange( v1[q], lo, hi );
-        }
-        if constexpr ( TH )
-        {
-            expRange( v0[KH], lo, hi );
-            expRange( v1[KH], lo, hi );
-        }
-        bool out = lo < -kPlainExp || hi > kPlainExp;
-        if constexpr ( NAB )
-        {
-            int la = 0, ha = 0;
-#pragma unroll
-            for ( int q = 3 + NX; q < 5 + NX; q++ )
-            {
-                expRange( v0[q], la, ha );
-                expRange( v1[q], la, ha );
-            }
-            expRange( Ai, la, ha );
-            expRange( Bi, la, ha );
-            out = out || la < -kPlainExpAB || ha > kPlainExpAB;
-        }
-        return __ballot( out ) == 0;
-    };
-    double* __restrict__ wb = &win[wv][0][0];
-    const int nrows = scalarLoad( &A.nrows );
-    loadRow( 0 );
-    for ( int r = 0; r < nrows; r++ )
-    {
-        const int4 R = scalarLoad4( rows + r );
-        // the previous row's window reads stay above this row's stores (a
-        // lane's read of a position another lane overwrites)
-        __builtin_amdgcn_fence( __ATOMIC_RELEASE, "wavefront" );
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence( __ATOMIC_ACQUIRE, "wavefront" );
-#pragma unroll
-        for ( int k = 0; k < NC; k++ )
-        {
-            wb[k * kW + lane] = v0[k];
-            if ( lane < R.y - 1 )
-                wb[k * kW + kSlice + lane] = v1[k];
-        }
-        const double limit = FAST && rowPlain() ? 0x1p600 : 0.0;
-        __builtin_amdgcn_fence( __ATOMIC_RELEASE, "wavefront" );
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence( __ATOMIC_ACQUIRE, "wavefront" );
-        if ( r + 1 < nrows )
-            loadRow( r + 1 );
-        auto slot = [&]( const int t ) __attribute__( ( always_inline ) ) {
-            const int32_t q = R.x + t;
-            const uint64_t ww = scalarLoad( mwords + q );
-            const double* __restrict__ wr = wb + lane + t;
-            const bool live = __builtin_amdgcn_inverse_ballot_w64( ww );
-            int mj = 0;
-            bool nf_j = false;
-            if constexpr ( TAG )
-            {
-                const int tag = static_cast<int>( wr[KT * kW] );
-                mj = tag >> 1;
-                nf_j = ( tag & 1 ) != 0;
-            }
-            if constexpr ( kIsLps<MODEL> )
-                nf_j = nf_i; // LPS tests nofail(i) twice (force/CabanaPD_LPS.hpp:417-418)
-            // ElasticPerfectlyPlastic: the slot's plastic stretch is loaded
-            // up front (every lane has an entry), so its latency overlaps the
-            // bond arithmetic; it is written back only where it changes
-            double spv = 0.0;
-            if constexpr ( EP )
-                spv = spl[q * kSlice];
-            if constexpr ( PREC == kF64 )
-            {
-                bool brk = false;
-                if ( live )
-                {
-                    const double uj0 = wr[0], uj1 = wr[kW], uj2 = wr[2 * kW];
-                    const double vj = wr[KV * kW];
-                    const double tj = TH ? wr[KH * kW] : 0.0;
-                    Bond64 b;
-                    bond64<MODEL>( xi0, xi1, xi2, ui0, ui1, ui2, wr[3 * kW], wr[4 * kW], wr[5 * kW], uj0, uj1, uj2,
-                                   b );
-                    double temp_avg = 0.0;
-                    if constexpr ( TH )
-                    {
-                        temp_avg = thermalAvg( A, Ti, tj );
-                        b.s = b.s - ( A.alpha * temp_avg );
-                    }
-                    if constexpr ( FRAC )
-                    {
-                        const double bcc_ij = TH ? thermalBcc( A, temp_avg ) : ( MT ? tab_bcc[ti4 + mj] : bcc );
-                        if ( criticalStretch64( b.r, b.xi, bcc_ij ) && !nf_i && !nf_j )
-                            brk = true;
-                    }
-                    if ( !brk )
-                    {
-                        double coeff;
-                        if constexpr ( !kIsLps<MODEL> )
-                        {
-                            const double sd = EP ? plasticStretchAt( spl + q * kSlice, spv, b.s, A.sY ) : b.s;
-                            coeff = ( MT ? tab_c[ti4 + mj] : c ) * sd * vj;
-                        }
-                        else
-                        {
-                            const double infl = infl1 ? 1.0 / b.xi : 1.0;
-                            coeff = ( Ai + wr[( 3 + NX ) * kW] + b.s * ( Bi + wr[( 4 + NX ) * kW] ) ) * infl * b.xi *
-                                    vj;
-                        }
-                        fx += coeff * b.rx / b.r;
-                        fy += coeff * b.ry / b.r;
-                        fz += coeff * b.rz / b.r;
-                    }
-                }
-                if constexpr ( FRAC )
-                {
-                    // wave-uniform test first (rare: a bond of the wave
-                    // breaks), then one lane writes the word
-                    const uint64_t m = __ballot( brk ) & ww;
-                    if ( __builtin_expect( m != 0, 0 ) )
-                    {
-                        if ( lane == 0 )
-                            bits[q] = ww & ~m;
-                    }
-                }
-            }
-            else
-            {
-                // every lane evaluates (window values are finite for every
-                // lane); bonds that do not exist, are broken or break add
-                // exactly zero.  r = xi + (u_j - u_i) from the slot's FP64
-                // stencil record.
-                const double* rr = srec + kRecStride * q;
-                const double uj0 = wr[0], uj1 = wr[kW], uj2 = wr[2 * kW];
-                const double r0 = ( uj0 - ui0 ) + scalarLoad( rr + kRecXiX );
-                const double r1 = uj1 + ( scalarLoad( rr + kRecXiY ) - ui1 );
-                const double r2 = uj2 + ( scalarLoad( rr + kRecXiZ ) - ui2 );
-                const float xil = scalarLoad( reinterpret_cast<const float*>( rr + kRecF ) ); // |xi|
-                Bond32 b;
-                mixedBond( r0, r1, r2, scalarLoad( rr + kRecXi2 ), xil, b );
-                double temp_avg = 0.0;
-                float ath = 0.0f;
-                const float s_mech = b.s;
-                if constexpr ( TH )
-                {
-                    temp_avg = thermalAvg( A, Ti, wr[KH * kW] );
-                    ath = static_cast<float>( A.alpha * temp_avg );
-                    b.s = b.s - ath;
-                }
-                uint64_t brkm = 0; // bonds that break in this pass
-                if constexpr ( FRAC )
-                {
-                    // candidates: intact, neither end no-fail; FP32 decision
-                    // except within the pair's band of s0, where the
-                    // reference's FP64 test decides
-                    const uint64_t cand = ww & __ballot( !nf_i && !nf_j );
-                    const float s0p = MT ? tab_s0[ti4 + mj] : s0f;
-                    const float bandp = MT ? tab_band[ti4 + mj] : bandK;
-                    const float band = TH ? fmaf( A.bandf, fabsf( s_mech ) + s0p + fabsf( ath ), bandp ) : bandp;
-                    const uint64_t inb = __ballot( fabsf( b.s - s0p ) <= band ) & cand;
-                    brkm = __ballot( b.s > s0p ) & cand & ~inb;
-                    if ( inb )
-                    {
-                        bool crit = false;
-                        if ( __builtin_amdgcn_inverse_ballot_w64( inb ) )
-                        {
-                            // rare path: the reference positions are loaded
-                            // here (the compiler barrier keeps the loads of
-                            // x_i from being hoisted into registers held for
-                            // the whole pass)
-                            __asm__ volatile( "" ::: "memory" );
-                            const int64_t j = p + R.z + t;
-                            Bond64 e;
-                            getDistance64( x[p], x[n + p], x[2 * n + p], ui0, ui1, ui2, x[j], x[n + j], x[2 * n + j],
-                                           uj0, uj1, uj2, e );
-                            crit = criticalStretch64( e.r, e.xi,
-                                                      TH ? thermalBcc( A, temp_avg ) : ( MT ? tab_bcc[ti4 + mj] : bcc ) );
-                        }
-                        brkm |= __ballot( crit ) & inb;
-                    }
-                }
-                const bool ok = __builtin_amdgcn_inverse_ballot_w64( ww & ~brkm );
-                float fr;
-                if constexpr ( !kIsLps<MODEL> )
-                {
-                    // ElasticPerfectlyPlastic: the plastic stretch stays FP64
-                    // and is updated on the bonds that carry force
-                    float sd = b.s;
-                    if constexpr ( EP )
-                    {
-                        if ( ok )
-                            sd = static_cast<float>(
-                                plasticStretchAt( spl + q * kSlice, spv, static_cast<double>( b.s ), A.sY ) );
-                    }
-                    const float cp = MT ? static_cast<float>( tab_c[ti4 + mj] ) : c32;
-                    fr = ( fold ? sd : ( cp * static_cast<float>( wr[KV * kW] ) ) * sd ) * b.rinv;
-                }
-                else
-                {
-                    const float wl = infl1 ? 1.0f : xil; // infl |xi|
-                    const float coeff = static_cast<float>( Ai + wr[( 3 + NX ) * kW] ) +
-                                        b.s * static_cast<float>( Bi + wr[( 4 + NX ) * kW] );
-                    fr = ( fold ? coeff * wl : ( coeff * wl ) * static_cast<float>( wr[KV * kW] ) ) * b.rinv;
-                }
-                fr = ok ? fr : 0.0f;
-                const double frd = static_cast<double>( fr );
-                sx = fma( frd, r0, sx );
-                sy = fma( frd, r1, sy );
-                sz = fma( frd, r2, sz );
-                if constexpr ( FRAC )
-                {
-                    if ( __builtin_expect( brkm != 0, 0 ) )
-                    {
-                        if ( lane == 0 )
-                            bits[q] = ww & ~brkm;
-                    }
-                }
-            }
-        };
-        // FP64 with shared reciprocals: the lanes the general code has to
-        // evaluate (a plastic stretch is updated only where s is final, and
-        // updating it again with the same s changes nothing)
-        auto slotFast = [&]( const int t, const double lim ) __attribute__( ( always_inline ) ) {
-            const int32_t q = R.x + t;
-            const uint64_t ww = scalarLoad( mwords + q );
-            const double* __restrict__ wr = wb + lane + t;
-            double spv = 0.0;
-            if constexpr ( EP )
-                spv = spl[q * kSlice];
-            bool brk = false, gen = false;
-            if ( __builtin_amdgcn_inverse_ballot_w64( ww ) )
-            {
-                int mj = 0;
-                bool nf_j = false;
-                if constexpr ( TAG )
-                {
-                    const int tag = static_cast<int>( wr[KT * kW] );
-                    mj = tag >> 1;
-                    nf_j = ( tag & 1 ) != 0;
-                }
-                if constexpr ( kIsLps<MODEL> )
-                    nf_j = nf_i;
-                const double vj = wr[KV * kW];
-                Fast64 b;
-                getDistanceFast( xi0, xi1, xi2, ui0, ui1, ui2, wr[3 * kW], wr[4 * kW], wr[5 * kW], wr[0], wr[kW],
-                                 wr[2 * kW], b );
-                double temp_avg = 0.0;
-                if constexpr ( TH )
-                {
-                    temp_avg = thermalAvg( A, Ti, wr[KH * kW] );
-                    b.s = b.s - ( A.alpha * temp_avg );
-                }
-                gen = !( fabs( b.s ) <= 0x1p600 ) || max( lowWord( b.r ), lowWord( b.xi ) ) == 0xffffffffu;
-                if constexpr ( FRAC )
-                {
-                    const double bcc_ij = TH ? thermalBcc( A, temp_avg ) : ( MT ? tab_bcc[ti4 + mj] : bcc );
-                    brk = !gen && criticalStretch64( b.r, b.xi, bcc_ij ) && !nf_i && !nf_j;
-                }
-                if ( !brk )
-                {
-                    double coeff;
-                    if constexpr ( !kIsLps<MODEL> )
-                    {
-                        double sd = b.s;
-                        if constexpr ( EP )
-                        {
-                            if ( !gen )
-                                sd = plasticStretchAt( spl + q * kSlice, spv, b.s, A.sY );
-                        }
-                        coeff = ( MT ? tab_c[ti4 + mj] : c ) * sd * vj;
-                    }
-                    else
-                    {
-                        const double infl = infl1 ? 1.0 / b.xi : 1.0;
-                        coeff = ( Ai + wr[( 3 + NX ) * kW] + b.s * ( Bi + wr[( 4 + NX ) * kW] ) ) * infl * b.xi * vj;
-                    }
-                    gen = gen || !( fabs( coeff ) <= lim );
-                    fx += divBy( coeff * b.rx, b.r, b.yr );
-                    fy += divBy( coeff * b.ry, b.r, b.yr );
-                    fz += divBy( coeff * b.rz, b.r, b.yr );
-                }
-            }
-            if constexpr ( FRAC )
-            {
-                const uint64_t brkm = __ballot( brk );
-                if ( __builtin_expect( brkm != 0, 0 ) )
-                {
-                    if ( lane == 0 )
-                        bits[q] = ww & ~brkm;
-                }
-            }
-            return __ballot( gen );
-        };
-        if constexpr ( PREC == kMixed )
-        {
-#pragma unroll
-            for ( int t = 0; t < kRowMaxSlots; t++ )
-                if ( t < R.y )
-                    slot( t );
-        }
-        else
-        {
-            if ( plain )
-            {
-                const double fx0 = fx, fy0 = fy, fz0 = fz;
-                uint64_t bad = 0;
-                for ( int t = 0; t < R.y; t++ )
-                    bad |= slotFast( t, limit );
-                if ( __builtin_expect( bad == 0, 1 ) )
-                    continue;
-                fx = fx0;
-                fy = fy0;
-                fz = fz0;
-            }
-            for ( int t = 0; t < R.y; t++ )
-                slot( t );
-        }
-    }
-    if constexpr ( PREC == kMixed )
-    {
-        fx = fma( rscale, sx, fx );
-        fy = fma( rscale, sy, fy );
-        fz = fma( rscale, sz, fz );
-    }
-    if ( !valid )
-        return;
-    epilogue( A, p, w.epi, w.cur, fx, fy, fz );
-}
-
-// ---------------------------------------------------------------------------
 // LPS state pass: Force<LPS,*>::computeWeightedVolume + computeDilatation
 // (force/CabanaPD_LPS.hpp:89-141, 287-378), fused: m_i and theta_i need only
 // particle i's own bonds.  Also stores the per-particle force-coefficient
@@ -2163,274 +654,6 @@ __global__ __launch_bounds__( kBlock ) void kLpsState( const PDArgs* __restrict_
             if ( mycnt > 0 )
                 th = 3.0 * th / m_i;
     }
-    A.theta[p] = th;
-    // ForceCoeffTag per-particle subexpressions (force_models/CabanaPD_LPS.hpp:131-132),
-    // with the particle's own material coefficients in a multi-material specimen
-    const double tc = A.mtype ? A.mat_tc[A.mtype[p]] : A.theta_coeff;
-    const double sc = A.mtype ? A.mat_sc[A.mtype[p]] : A.s_coeff;
-    A.lpsA[p] = tc * th / m_i;
-    A.lpsB[p] = sc / m_i;
-}
-
-// ---------------------------------------------------------------------------
-// The LPS state pass with neighbor data staged in LDS row windows (stencil-slot
-// form on lattice rows), as kForceRows does for the force pass.  Same bonds,
-// order and expressions as kLpsState, so the results are identical; the FP64
-// form walks the rows twice (m_i must be complete before each bond's share of
-// theta_i is divided by it), the mixed form once.
-// ---------------------------------------------------------------------------
-template <bool FRAC, int PREC, bool GEN>
-__global__ __launch_bounds__( kBlock ) void kLpsStateRows( const PDArgs* __restrict__ specs,
-                                                           const int32_t* __restrict__ tile_spec,
-                                                           const int64_t* __restrict__ tile_slice,
-                                                           int32_t parity, int64_t launch,
-                                                           int32_t do_m, int32_t do_theta )
-{
-#pragma clang fp contract( off )
-    constexpr int kW = kSlice + kRowMaxSlots - 1;
-    constexpr int NX = ( PREC == kF64 ) ? 3 : 0; // staged x components
-    constexpr int KV = 3 + NX;                   // staged vol (GEN)
-    // mixed form: the bond vector r = xi + (u_j - u_i) in FP64 from the slot's
-    // FP64 stencil offset xi; the windows hold u only
-    constexpr int NC = KV + ( GEN ? 1 : 0 );
-    __shared__ double win[kSlicesPerBlock][2][NC][kW];
-    WaveCtx w;
-    if ( !waveSetup( specs, tile_spec, tile_slice, 0, parity, launch, w ) )
-        return; // waves are independent: no block-level synchronisation
-    const PDArgs& A = *w.A;
-    const int wv = __builtin_amdgcn_readfirstlane( static_cast<int>( threadIdx.x / kSlice ) );
-    const int lane = threadIdx.x & ( kSlice - 1 );
-    const int64_t n = scalarLoad( &A.n );
-    const int64_t p0 = w.slice * kSlice;
-    const int64_t p = p0 + lane;
-    const bool valid = p < n;
-    const int64_t pc = valid ? p : p0;
-    const double* __restrict__ x = scalarLoad( &A.x );
-    const double* __restrict__ u = scalarLoad( &A.U[w.cur] );
-    const int4* __restrict__ rows = scalarLoad( &A.rows );
-    const double xi0 = x[pc], xi1 = x[n + pc], xi2 = x[2 * n + pc];
-    const double ui0 = u[pc], ui1 = u[n + pc], ui2 = u[2 * n + pc];
-    // per-slot lane masks (intact words, a subset of the existence words,
-    // or the existence words without fracture) and the stencil tables, all
-    // wave-uniform: scalar loads
-    const int64_t row0 = scalarLoad( scalarLoad( &A.slice_ptr ) + w.slice );
-    const uint64_t* __restrict__ mwords = scalarLoad( FRAC ? &A.intact : &A.exist ) + row0;
-    const double* __restrict__ srec = scalarLoad( &A.stencil_rec );
-    const int infl1 = A.influence;
-    const double volu = A.vol_value;
-    const float vol32 = static_cast<float>( A.vol_value );
-
-    const double* src[KV];
-    src[0] = u;
-    src[1] = u + n;
-    src[2] = u + 2 * n;
-    if constexpr ( NX )
-    {
-        src[3] = x;
-        src[4] = x + n;
-        src[5] = x + 2 * n;
-    }
-    const double* __restrict__ volp = scalarLoad( &A.vol );
-    const int32_t p032 = static_cast<int32_t>( p0 );
-    double v0[NC], v1[NC];
-#pragma unroll
-    for ( int k = 0; k < NC; k++ )
-        v1[k] = 0.0;
-    // Row windows through raw buffer loads, as in kForceRows (n < 2^28).
-    const uint32_t nbytes = static_cast<uint32_t>( n ) * 8u;
-    __amdgpu_buffer_rsrc_t rs[NC];
-#pragma unroll
-    for ( int k = 0; k < KV; k++ )
-        rs[k] = bufferOf( src[k], nbytes );
-    if constexpr ( GEN )
-        rs[KV] = bufferOf( volp, nbytes );
-    const uint32_t lane8 = static_cast<uint32_t>( lane ) * 8u;
-    auto loadHalf = [&]( double* dst, int32_t g ) {
-        const uint32_t vo = g >= 0 ? lane8 : static_cast<uint32_t>( g + lane ) * 8u;
-        const uint32_t so = g >= 0 ? static_cast<uint32_t>( g ) * 8u : 0u;
-#pragma unroll
-        for ( int k = 0; k < NC; k++ )
-            dst[k] = bufferLoad64( rs[k], vo, so );
-    };
-    auto loadRow = [&]( int r ) {
-        const int4 R = scalarLoad4( rows + r );
-        const int32_t g = p032 + R.z; // uniform
-        loadHalf( v0, g );
-        if ( lane < R.y - 1 )
-            loadHalf( v1, g + kSlice );
-    };
-    // Walk every bond slot in slot order; bond(live, wr, q) gets the window
-    // position of the neighbor's staged values.  FP64: a row goes through
-    // fast first where plain; rows with a lane for which it returns true are
-    // evaluated again by bond, from the sums as save left them.
-    const bool plain = PREC == kF64 && scalarLoad( &A.plain_range ) != 0;
-    auto walk = [&]( auto&& bond, auto&& fast, double& sum ) {
-        const int nrows = scalarLoad( &A.nrows );
-        loadRow( 0 );
-        for ( int r = 0; r < nrows; r++ )
-        {
-            const int4 R = scalarLoad4( rows + r );
-            double* __restrict__ wb = &win[wv][r & 1][0][0];
-#pragma unroll
-            for ( int k = 0; k < NC; k++ )
-            {
-                wb[k * kW + lane] = v0[k];
-                if ( lane < R.y - 1 )
-                    wb[k * kW + kSlice + lane] = v1[k];
-            }
-            __builtin_amdgcn_fence( __ATOMIC_RELEASE, "wavefront" );
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence( __ATOMIC_ACQUIRE, "wavefront" );
-            if ( r + 1 < nrows )
-                loadRow( r + 1 );
-            // mixed form: the row's slots unrolled (immediate window offsets);
-            // xi_y - u_i,y and xi_z - u_i,z once per row (the slots of a
-            // lattice row differ in xi_x only)
-            if constexpr ( PREC == kMixed )
-            {
-                const double* rec_r = srec + kRecStride * R.x;
-                const double ay = scalarLoad( rec_r + kRecXiY ) - ui1;
-                const double az = scalarLoad( rec_r + kRecXiZ ) - ui2;
-#pragma unroll
-                for ( int t = 0; t < kRowMaxSlots; t++ )
-                    if ( t < R.y )
-                    {
-                        const int32_t q = R.x + t;
-                        const bool live = __builtin_amdgcn_inverse_ballot_w64( scalarLoad( mwords + q ) );
-                        bond( live, wb + lane + t, q, ay, az );
-                    }
-            }
-            else
-            {
-                if ( plain )
-                {
-                    const double sum0 = sum;
-                    uint64_t bad = 0;
-                    for ( int t = 0; t < R.y; t++ )
-                    {
-                        const bool live = __builtin_amdgcn_inverse_ballot_w64( scalarLoad( mwords + R.x + t ) );
-                        bad |= __ballot( fast( live, wb + lane + t ) );
-                    }
-                    if ( __builtin_expect( bad == 0, 1 ) )
-                        continue;
-                    sum = sum0;
-                }
-                for ( int t = 0; t < R.y; t++ )
-                {
-                    const int32_t q = R.x + t;
-                    const bool live = __builtin_amdgcn_inverse_ballot_w64( scalarLoad( mwords + q ) );
-                    bond( live, wb + lane + t, q, 0.0, 0.0 );
-                }
-            }
-        }
-    };
-
-    double m_i = 0.0;
-    double th = 0.0;
-    if constexpr ( PREC == kF64 )
-    {
-        if ( do_m )
-        {
-            walk( [&]( bool live, const double* wr, int32_t, double, double ) {
-                if ( live )
-                {
-                    Bond64 b;
-                    getDistance64( xi0, xi1, xi2, ui0, ui1, ui2, wr[3 * kW], wr[4 * kW], wr[5 * kW], wr[0], wr[kW],
-                                   wr[2 * kW], b );
-                    const double infl = infl1 ? 1.0 / b.xi : 1.0;
-                    m_i += infl * b.xi * b.xi * ( GEN ? wr[KV * kW] : volu );
-                }
-            },
-            [&]( bool live, const double* wr ) {
-                // |xi| alone: its range is the lattice's
-                if ( live )
-                {
-                    const double xi_x = wr[3 * kW] - xi0, xi_y = wr[4 * kW] - xi1, xi_z = wr[5 * kW] - xi2;
-                    const double xi = rootRecip( xi_x * xi_x + xi_y * xi_y + xi_z * xi_z ).r;
-                    const double infl = infl1 ? 1.0 / xi : 1.0;
-                    m_i += infl * xi * xi * ( GEN ? wr[KV * kW] : volu );
-                }
-                return false;
-            },
-            m_i );
-        }
-        else if ( valid )
-            m_i = A.m[p];
-        const bool mpos = FRAC ? ( m_i > 0 ) : true;
-        if ( do_theta )
-        {
-            // one reciprocal of m_i for all its bonds
-            const double ym = recip64( m_i );
-            const bool gen_m = !( m_i >= 0x1p-300 && m_i <= 0x1p300 ) || lowWord( m_i ) == 0xffffffffu;
-            walk( [&]( bool live, const double* wr, int32_t, double, double ) {
-                if ( live && mpos )
-                {
-                    Bond64 b;
-                    getDistance64( xi0, xi1, xi2, ui0, ui1, ui2, wr[3 * kW], wr[4 * kW], wr[5 * kW], wr[0], wr[kW],
-                                   wr[2 * kW], b );
-                    const double infl = infl1 ? 1.0 / b.xi : 1.0;
-                    const double theta_b = infl * b.s * b.xi * b.xi * ( GEN ? wr[KV * kW] : volu );
-                    th += 3.0 * theta_b / m_i;
-                }
-            },
-            [&]( bool live, const double* wr ) {
-                bool gen = false;
-                if ( live && mpos )
-                {
-                    Fast64 b;
-                    getDistanceFast( xi0, xi1, xi2, ui0, ui1, ui2, wr[3 * kW], wr[4 * kW], wr[5 * kW], wr[0], wr[kW],
-                                     wr[2 * kW], b );
-                    const double infl = infl1 ? 1.0 / b.xi : 1.0;
-                    const double theta_b = infl * b.s * b.xi * b.xi * ( GEN ? wr[KV * kW] : volu );
-                    th += divBy( 3.0 * theta_b, m_i, ym );
-                    gen = gen_m || !( fabs( theta_b ) <= 0x1p300 ) || lowWord( b.xi ) == 0xffffffffu;
-                }
-                return gen;
-            },
-            th );
-        }
-    }
-    else
-    {
-        if ( !do_m && valid )
-            m_i = A.m[p];
-        // m_i for the theta condition is only known after the walk: sum both,
-        // apply the condition at the end (the sums are the same per-bond terms)
-        walk( [&]( bool live, const double* wr, int32_t q, double ay, double az ) {
-            if ( live )
-            {
-                // the slot's record: xi_x, |xi|^2, |xi|, infl |xi|^2
-                const double* rr = srec + kRecStride * q;
-                const float* rf = reinterpret_cast<const float*>( rr + kRecF );
-                const float w2 = scalarLoad( rf + 2 ); // infl |xi|^2
-                const float vj32 = GEN ? static_cast<float>( wr[KV * kW] ) : vol32;
-                if ( do_m )
-                    m_i += static_cast<double>( w2 * vj32 );
-                if ( do_theta )
-                {
-                    Bond32 b;
-                    mixedBond( ( wr[0] - ui0 ) + scalarLoad( rr + kRecXiX ), wr[kW] + ay, wr[2 * kW] + az,
-                               scalarLoad( rr + kRecXi2 ), scalarLoad( rf ), b );
-                    th += static_cast<double>( w2 * b.s * vj32 );
-                }
-            }
-        },
-        []( bool, const double* ) { return false; }, th );
-        if ( do_theta )
-        {
-            const bool mpos = FRAC ? ( m_i > 0 ) : true;
-            if ( !mpos )
-                th = 0.0;
-            else if ( valid && A.cnt[p] > 0 )
-                th = 3.0 * th / m_i;
-        }
-    }
-    if ( !valid )
-        return;
-    if ( do_m )
-        A.m[p] = m_i;
-    if ( !do_theta )
-        return;
     A.theta[p] = th;
     // ForceCoeffTag per-particle subexpressions (force_models/CabanaPD_LPS.hpp:131-132),
     // with the particle's own material coefficients in a multi-material specimen
@@ -3455,7 +1678,6 @@ __global__ __launch_bounds__( 256 ) void kPrescribe( const int64_t* __restrict__
     }
 }
 
-using ForceFn = void ( * )( const PDArgs*, const int32_t*, const int64_t*, int32_t, int32_t, int64_t, int32_t );
 
 template <int MODEL, bool FRAC, int PREC, bool SLOTS, bool MM = false>
 ForceFn pickUnroll( int unroll )
@@ -3499,6 +1721,13 @@ ForceFn pickForceForm( const PDArgs& a )
     }
 }
 
+// A force launch: the kernel and its waves per slice.
+struct ForcePick
+{
+    ForceFn fn = nullptr;
+    int waves = 1;
+};
+
 template <int MODEL, bool GEN>
 ForceFn pickRowsModel( const PDArgs& a )
 {
@@ -3536,14 +1765,6 @@ ForceFn pickForceRows( const PDArgs& a )
     return rowsGeneral( a ) ? pickForceRowsGen<true>( a ) : pickForceRowsGen<false>( a );
 }
 
-// Per-particle features of the force pass (kFeat* bits): several materials,
-// temperature, plastic stretch (the LPS model has the first only).
-int rowFeatures( const PDArgs& a )
-{
-    const bool lps = a.model == kLPS || a.model == kLinLPS;
-    return ( a.mtype ? kFeatMT : 0 ) | ( !lps && a.temp ? kFeatTH : 0 ) | ( !lps && a.splas ? kFeatEP : 0 );
-}
-
 template <int MODEL, int FEAT>
 ForceFn pickRowsFeat( const PDArgs& a )
 {
@@ -3570,11 +1791,56 @@ ForceFn pickForceRowsFeat( const PDArgs& a )
     }
 }
 
-ForceFn pickForce( const PDArgs& a )
+// Waves per slice of a launch over nslices slices.  With one wave per slice a
+// launch of fewer than about four waves per SIMD (1024 SIMDs) lasts as long
+// as one wave's chain of slots; the split form (pdk_rows.hpp) shortens that
+// chain but leaves waves waiting at its barriers, so it loses once the SIMDs
+// are full.  Measured, one step of a cube, 1 / 4 / 8 waves per slice, in us:
+//   slices                  200            512           1077          2197
+//   FP64 PMB fracture   55/ 20/ 15    56/ 25/ 28    71/ 48/ 66    91/ 80/118
+//   FP64 LPS fracture  148/ 54/ 39   150/ 68/ 75   189/128/181   242/210/328
+//   FP64 two materials 168/ 62/ 45   168/ 75/ 85   205/163/205   256/271/371
+//   mixed PMB fracture  32/ 16/ 12    32/ 18/ 21    33/ 33/ 47    37/ 54/ 82
+//   mixed LPS fracture  81/ 35/ 25    81/ 38/ 38    82/ 63/ 85    95/106/153
+//   mixed plastic       75/ 25/ 17    88/ 32/ 36   102/ 60/ 85   114/ 97/152
+// Eight waves (up to 89 KB of LDS) fit once on a CU, so they serve up to 256
+// slices.
+int splitWaves( const PDArgs& a, int64_t nslices )
 {
-    if ( useRowWindows( a ) )
-        return rowFeatures( a ) ? pickForceRowsFeat( a ) : pickForceRows( a );
-    return a.exist ? pickForceForm<true>( a ) : pickForceForm<false>( a );
+    if ( a.row_max > kSplitSlots )
+        return 1;
+    if ( nslices <= 256 )
+        return 8;
+    const bool lps = a.model == kLPS || a.model == kLinLPS;
+    const int64_t four = a.precision == PDK_MIXED ? ( lps || a.splas ? 1536 : 1088 ) : ( rowFeatures( a ) ? 1792 : 2560 );
+    return nslices <= four ? 4 : 1;
+}
+
+ForcePick pickForce( const PDArgs& a, int64_t nslices )
+{
+    ForcePick p;
+    if ( !useRowWindows( a ) )
+    {
+        p.fn = a.exist ? pickForceForm<true>( a ) : pickForceForm<false>( a );
+        return p;
+    }
+    if ( rowFeatures( a ) )
+    {
+        p.waves = splitWaves( a, nslices );
+        p.fn = p.waves > 1 || a.hole_win ? splitForceRowsFeat( a, p.waves, a.hole_win != nullptr )
+                                         : pickForceRowsFeat( a );
+        return p;
+    }
+    const bool plain_model = a.model == kPMB || a.model == kLPS;
+    if ( plain_model && !rowsGeneral( a ) )
+        p.waves = splitWaves( a, nslices );
+    if ( p.waves > 1 || a.hole_win )
+    {
+        p.fn = splitForceRows( a, p.waves, a.hole_win != nullptr );
+        return p;
+    }
+    p.fn = pickForceRows( a );
+    return p;
 }
 
 thread_local char g_force_name[64];
@@ -3678,6 +1944,15 @@ static unsigned sliceBlocks( const PDArgs& a )
     return static_cast<unsigned>( ( a.nslices + kSlicesPerBlock - 1 ) / kSlicesPerBlock );
 }
 
+// Grid and block of a launch over nslices slices.
+static unsigned splitBlocks( int64_t nslices, int waves )
+{
+    return static_cast<unsigned>( waves > 1 ? nslices : ( nslices + kSlicesPerBlock - 1 ) / kSlicesPerBlock );
+}
+static unsigned splitThreads( int waves )
+{
+    return waves > 1 ? static_cast<unsigned>( waves ) * kSlice : kBlock;
+}
 void launchForce( const PDArgs* args_dev, const PDArgs& a, int32_t epilogue_mode, int32_t parity,
                   hipStream_t st )
 {
@@ -3685,13 +1960,12 @@ void launchForce( const PDArgs* args_dev, const PDArgs& a, int32_t epilogue_mode
         return;
     const int32_t accumulate = epilogue_mode < 0 ? 1 : 0;
     const int32_t epi = epilogue_mode < 0 ? kEpiStoreOnly : epilogue_mode;
-    ForceFn fn = pickForce( a );
-    hipLaunchKernelGGL( fn, dim3( sliceBlocks( a ) ), dim3( kBlock ), 0, st, args_dev, nullptr, nullptr, epi,
-                        parity, int64_t( 0 ), accumulate );
+    const ForcePick p = pickForce( a, a.nslices );
+    hipLaunchKernelGGL( p.fn, dim3( splitBlocks( a.nslices, p.waves ) ), dim3( splitThreads( p.waves ) ),
+                        0, st, args_dev, nullptr, nullptr, epi, parity,
+                        int64_t( 0 ), accumulate );
     PDK_HIP( hipGetLastError() );
 }
-
-using LpsFn = void ( * )( const PDArgs*, const int32_t*, const int64_t*, int32_t, int64_t, int32_t, int32_t );
 
 template <bool GEN>
 LpsFn pickLpsRows( const PDArgs& a )
@@ -3703,12 +1977,27 @@ LpsFn pickLpsRows( const PDArgs& a )
 
 // The LPS state pass follows the layout (row windows wherever a row table
 // exists), not the force-pass tuning knob; both kernels give the same results.
-LpsFn pickLps( const PDArgs& a )
+struct LpsPick
 {
+    LpsFn fn = nullptr;
+    int waves = 1;
+};
+LpsPick pickLps( const PDArgs& a, int64_t nslices )
+{
+    LpsPick p;
     if ( a.rows != nullptr && a.nrows > 0 )
-        return a.vol_uniform ? pickLpsRows<false>( a ) : pickLpsRows<true>( a );
-    return a.fracture ? ( a.precision == PDK_MIXED ? kLpsState<true, kMixed> : kLpsState<true, kF64> )
+    {
+        if ( a.vol_uniform )
+            p.waves = splitWaves( a, nslices );
+        if ( p.waves > 1 || a.hole_win )
+            p.fn = splitLpsRows( a, p.waves, a.hole_win != nullptr );
+        else
+            p.fn = a.vol_uniform ? pickLpsRows<false>( a ) : pickLpsRows<true>( a );
+        return p;
+    }
+    p.fn = a.fracture ? ( a.precision == PDK_MIXED ? kLpsState<true, kMixed> : kLpsState<true, kF64> )
                       : ( a.precision == PDK_MIXED ? kLpsState<false, kMixed> : kLpsState<false, kF64> );
+    return p;
 }
 
 void launchLpsState( const PDArgs* args_dev, const PDArgs& a, bool weighted_volume, bool dilatation,
@@ -3716,8 +2005,9 @@ void launchLpsState( const PDArgs* args_dev, const PDArgs& a, bool weighted_volu
 {
     if ( a.nslices == 0 )
         return;
-    LpsFn fn = pickLps( a );
-    hipLaunchKernelGGL( fn, dim3( sliceBlocks( a ) ), dim3( kBlock ), 0, st, args_dev, nullptr, nullptr, parity,
+    const LpsPick p = pickLps( a, a.nslices );
+    hipLaunchKernelGGL( p.fn, dim3( splitBlocks( a.nslices, p.waves ) ), dim3( splitThreads( p.waves ) ),
+                        0, st, args_dev, nullptr, nullptr, parity,
                         int64_t( 0 ), int32_t( weighted_volume ), int32_t( dilatation ) );
     PDK_HIP( hipGetLastError() );
 }
@@ -3753,8 +2043,9 @@ void launchForceBatched( const PDArgs* specs_dev, const PDArgs& variant, const i
 {
     if ( ntiles == 0 )
         return;
-    ForceFn fn = pickForce( variant );
-    hipLaunchKernelGGL( fn, dim3( static_cast<unsigned>( ntiles ) ), dim3( kBlock ), 0, st, specs_dev, tile_spec,
+    const ForcePick p = pickForce( variant, ntiles * kSlicesPerBlock );
+    hipLaunchKernelGGL( p.fn, dim3( splitBlocks( ntiles * kSlicesPerBlock, p.waves ) ), dim3( splitThreads( p.waves ) ),
+                        0, st, specs_dev, tile_spec,
                         tile_slice, int32_t( kEpiFinalInitial ), static_cast<int32_t>( launch_index & 1 ),
                         launch_index, int32_t( 0 ) );
     PDK_HIP( hipGetLastError() );
@@ -3765,8 +2056,9 @@ void launchLpsStateBatched( const PDArgs* specs_dev, const PDArgs& variant, cons
 {
     if ( ntiles == 0 )
         return;
-    LpsFn fn = pickLps( variant );
-    hipLaunchKernelGGL( fn, dim3( static_cast<unsigned>( ntiles ) ), dim3( kBlock ), 0, st, specs_dev, tile_spec,
+    const LpsPick p = pickLps( variant, ntiles * kSlicesPerBlock );
+    hipLaunchKernelGGL( p.fn, dim3( splitBlocks( ntiles * kSlicesPerBlock, p.waves ) ), dim3( splitThreads( p.waves ) ),
+                        0, st, specs_dev, tile_spec,
                         tile_slice, static_cast<int32_t>( launch_index & 1 ), launch_index,
                         int32_t( variant.fracture ? 1 : 0 ), int32_t( 1 ) );
     PDK_HIP( hipGetLastError() );

@@ -160,6 +160,10 @@ struct SlotForm
     DevBuf exist, soff, table, xi2d, xiv, rows, rowstart, aux, rec;
     int32_t slots = 0;
     int32_t nrows = 0; // row windows (0: the stencil does not split into <= kMaxRows rows)
+    int32_t row_max = 0; // slots of the longest row
+    // lattice with missing sites: neighbour windows per (slice, row) and each lane's place in them
+    bool hole = false;
+    DevBuf hole_win, hole_pos;
 };
 bool buildStencilSlots( const PDArgs& a, const int64_t dims[3], const double h[3], double rc,
                         const std::vector<int64_t>& perm_host, DevBuf& col, DevBuf& intact, int64_t* slice_ptr_dev,

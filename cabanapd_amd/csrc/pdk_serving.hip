@@ -143,7 +143,7 @@ struct BatchEngine::Impl
             // one kernel variant per group: model, fracture, precision, bond layout
             const int form = ( useRowWindows( *v.h ) ? 2 : ( v.h->exist ? 1 : 0 ) ) +
                              ( v.h->rows != nullptr ? 4 : 0 ) + ( v.h->vol_uniform ? 0 : 8 ) +
-                             ( v.h->any_nofail ? 16 : 0 );
+                             ( v.h->any_nofail ? 16 : 0 ) + ( v.h->hole_win != nullptr ? 32 : 0 );
             auto k = std::make_tuple( v.model, v.fracture, v.precision, form );
             auto it = key.find( k );
             size_t gi;
@@ -159,6 +159,7 @@ struct BatchEngine::Impl
                 gi = it->second;
             Group& g = ng[gi];
             PDArgs a = *v.h;
+            g.variant.row_max = std::max( g.variant.row_max, a.row_max ); // decides whether slices are split
             a.parity_offset = r.parity_offset;
             a.end_launch = r.end_launch;
             a.launch_ctr = ctr.as<int64_t>();

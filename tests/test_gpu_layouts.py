@@ -59,3 +59,38 @@ def test_whole_number_horizons_take_stencil_slots(model, m, precision):
     assert a["layout"]["stencil_slots"] and not b["layout"]["stencil_slots"]
     assert (a["bonds"][2] == 0).any()
     same(a, b, precision)
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("kind", ["pmb", "lps", "epp", "materials", "thermal"])
+def test_split_slices_match_gathers(kind, precision):
+    """Specimens of few slices share each slice's rows among the waves of a
+    block (8 up to 256 slices, 4 up to a limit, then one wave per slice):
+    the gathers' bits on both sides of the lines, a part-filled last slice
+    and one slice alone included."""
+    for dims in ((4, 5, 3), (9, 9, 9), (16, 32, 32), (17, 31, 32), (32, 33, 66), (41, 41, 41), (44, 51, 73)):
+        w = box("LPS" if kind in ("lps", "materials") else "PMB", dims, 3.01, True)
+        d = w["desc"]
+        n = w["x"].shape[0]
+        rng = np.random.default_rng(5)
+        if kind == "epp":
+            d.mechanics, d.sigma_y = 1, 2.5e7
+        if kind == "thermal":
+            d.thermal, d.alpha, d.temp0 = 1, 1e-6, 20.0
+            w["temperature"] = 20.0 + 40.0 * rng.random(n)
+        if kind == "materials":
+            w["materials"] = ([(4.3e10, 2.9e10, 3.8), (8e10, 5e10, 38.0)], (rng.random(n) < 0.4).astype(np.int32))
+        d.precision = precision
+        out = []
+        for variant in (0, 4):
+            s = engine.Spec(ctx(), d, n)
+            configs.upload(s, w)
+            configs.setup(s, w)
+            s.set_tuning(variant)
+            s.step(4)
+            out.append([s.get("u"), s.get("v"), s.get("f"), s.bonds()[2], s.kernel_name(0)])
+            s.close()
+        say(f"case: {kind} {dims} precision {precision}: {(n + 63) // 64} slices, {out[0][4]} vs {out[1][4]}")
+        assert "Rows" in out[0][4] and "Rows" not in out[1][4]
+        for a, b in zip(out[0][:4], out[1][:4]):
+            assert np.array_equal(a, b)
