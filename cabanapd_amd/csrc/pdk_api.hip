@@ -227,6 +227,7 @@ struct pdk_spec_s
     bool pair_tables = false; // particle types and pair tables on the device
     double mat_c[16] = {}, mat_bcc[16] = {}, mat_tc[4] = {}, mat_sc[4] = {};
     double lat_h[3] = { 0, 0, 0 }; // lattice spacing when lattice_rows
+    double lat_lo[3] = { 0, 0, 0 }; // position of lattice index (0, 0, 0)
     int64_t lat_dims[3] = { 0, 0, 0 };
     double lat_dev = 0.0;          // largest distance of a position from its lattice site / spacing
     int32_t nsten = 0;             // stencil entries (0 = no stencil)
@@ -423,7 +424,7 @@ struct pdk_spec_s
             h.rowstart = slot.nrows > 0 ? slot.rowstart.as<uint32_t>() : nullptr;
             h.nrows = slot.nrows;
             h.row_max = slot.row_max;
-            h.hole_win = slot.hole ? slot.hole_win.as<int2>() : nullptr;
+            h.hole_win = slot.hole ? slot.hole_win.as<int4>() : nullptr;
             h.hole_pos = slot.hole ? slot.hole_pos.as<uint8_t>() : nullptr;
             for ( int dd = 0; dd < 3; dd++ )
                 h.lat_n[dd] = static_cast<int32_t>( lat_dims[dd] );
@@ -1031,7 +1032,7 @@ int pdk_spec_upload( pdk_spec s, const double* x, const double* u, const double*
         std::vector<int64_t> lperm;
         bool lattice = false;
         if ( s->d.ordering != PDK_ORDER_MORTON )
-            lattice = latticeOrder( x, n, lperm, s->lat_h, s->lat_dims, &s->lat_dev );
+            lattice = latticeOrder( x, n, lperm, s->lat_lo, s->lat_h, s->lat_dims, &s->lat_dev );
         require( lattice || s->d.ordering != PDK_ORDER_LATTICE_ROWS, "positions do not form a lattice" );
         s->lattice_rows = lattice;
         s->vol_uniform = true;
@@ -1237,6 +1238,13 @@ int pdk_build_bonds( pdk_spec s )
                     if ( buildStencilSlots( s->h, s->lat_dims, s->lat_h, q.rc, s->h_perm, s->col, s->intact,
                                             s->slice_ptr.as<int64_t>(), s->total_rows, s->col_rows_cap, s->slot,
                                             s->scratch, s->acct(), s->st ) )
+                        s->nsten = s->slot.slots;
+                    // missing sites: the forms whose row passes take them
+                    // (equal volumes, no no-fail particles, PMB or LPS)
+                    else if ( s->vol_uniform && !( s->d.fracture && s->any_nofail ) && !isLinearModel( s->d.model ) &&
+                              buildHoleSlots( s->h, s->lat_dims, s->lat_lo, s->lat_h, q.rc, s->h_perm, s->col,
+                                              s->intact, s->slice_ptr.as<int64_t>(), s->total_rows, s->col_rows_cap,
+                                              s->slot, s->scratch, s->acct(), s->st ) )
                         s->nsten = s->slot.slots;
                 } );
             }
@@ -2121,7 +2129,7 @@ int pdk_spec_layout( pdk_spec s, int32_t* lattice_rows, int32_t* stencil_entries
         if ( stencil_entries )
             *stencil_entries = s->nsten;
         if ( stencil_slots )
-            *stencil_slots = s->slot.slots > 0 ? 1 : 0;
+            *stencil_slots = s->slot.slots > 0 && !s->slot.hole ? 1 : 0;
     } );
 }
 
@@ -2142,7 +2150,7 @@ int pdk_set_tuning( pdk_spec s, int32_t unroll )
                  "unroll must be 0 (row windows), 1, 2, 4 or 8" );
         require( unroll != 0 || s->rowsCover(),
                  "this combination of materials, EPP and temperature dependence uses the gather variant" );
-        require( unroll != 0 || !s->built || s->slot.nrows > 0,
+        require( unroll != 0 || !s->built || ( s->slot.nrows > 0 && !s->slot.hole ),
                  "row windows need the stencil-slot layout of a full lattice" );
         s->unroll = unroll;
         if ( s->uploaded )

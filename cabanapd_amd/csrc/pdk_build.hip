@@ -635,6 +635,176 @@ __global__ __launch_bounds__( kThreads ) void kFillStencilSlots( int64_t n, int6
     }
 }
 
+// ---- Stencil-slot form of lattices with missing sites ------------------------
+// Particles in lattice-row order, the ids counting only the sites that hold
+// one: site[p] is particle p's site (iz*ny + iy)*nx + ix, id[site] the particle
+// on a site or -1.  Slot q is still stencil entry q for every particle; its
+// neighbour is the particle on the site that the entry points to, if any.
+// Along one lattice row consecutive sites that exist have consecutive ids, so
+// the neighbours of a slice in one row of the stencil lie in one id window
+// (or two), and a lane's place in it moves on by one with every neighbour that exists.
+__global__ __launch_bounds__( kThreads ) void kSites( const double* __restrict__ x, int64_t n, double lo0, double lo1,
+                                                      double lo2, double h0, double h1, double h2, LatticeBox L,
+                                                      int32_t* __restrict__ site, int32_t* __restrict__ id,
+                                                      int32_t* __restrict__ flag )
+{
+    const int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if ( p >= n )
+        return;
+    const double lo[3] = { lo0, lo1, lo2 }, h[3] = { h0, h1, h2 };
+    const int32_t ext[3] = { L.nx, L.ny, L.nz };
+    int64_t k[3];
+    bool bad = false;
+    for ( int d = 0; d < 3; d++ )
+    {
+        k[d] = static_cast<int64_t>( rint( ( x[d * n + p] - lo[d] ) / h[d] ) );
+        bad = bad || k[d] < 0 || k[d] >= ext[d];
+    }
+    if ( bad )
+    {
+        *flag = 1;
+        site[p] = 0;
+        return;
+    }
+    const int32_t s = static_cast<int32_t>( ( k[2] * L.ny + k[1] ) * L.nx + k[0] );
+    site[p] = s;
+    id[s] = static_cast<int32_t>( p );
+}
+
+// The particle that entry t of particle p points to, or -1.
+__device__ __forceinline__ int32_t holeNeighbour( const int4 t, int32_t ix, int32_t iy, int32_t iz,
+                                                  const LatticeBox& L, const int32_t* __restrict__ id )
+{
+    if ( !inBox( t, ix, iy, iz, L ) )
+        return -1;
+    return id[( ( iz + t.z ) * L.ny + iy + t.y ) * L.nx + ix + t.x];
+}
+
+// Sites strictly ascending, and every compact row equal to its existing
+// stencil entries in slot order.
+__global__ __launch_bounds__( kThreads ) void kCheckHoleSlots( PDArgs a, LatticeBox L, const int4* __restrict__ ent,
+                                                               int32_t S, const int32_t* __restrict__ site,
+                                                               const int32_t* __restrict__ id,
+                                                               int32_t* __restrict__ flag )
+{
+    const int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if ( p >= a.n )
+        return;
+    int32_t ix, iy, iz;
+    latticeCoords( site[p], L, ix, iy, iz );
+    const int64_t slice = p / kSlice;
+    const int lane = static_cast<int>( p - slice * kSlice );
+    const int64_t base = a.slice_ptr[slice];
+    const int32_t cnt = a.cnt[p];
+    int32_t q = 0;
+    bool bad = p > 0 && site[p] <= site[p - 1];
+    for ( int32_t e = 0; e < S && !bad; e++ )
+    {
+        const int32_t j = holeNeighbour( ent[e], ix, iy, iz, L, id );
+        if ( j < 0 )
+            continue;
+        if ( q >= cnt || a.col[( base + q ) * kSlice + lane] != j )
+            bad = true;
+        q++;
+    }
+    if ( bad || q != cnt )
+        *flag = 1;
+}
+
+// The slot-form arrays and, per row of the row table, the slice's neighbour
+// window and each lane's place in it.  A window is one run of ids, or two
+// where the slice's own row has a gap that the neighbouring row fills (the
+// grips of a dogbone): place w holds id w + (w < y ? x : z) of its int4, w its
+// length.  Sets *flag where it is longer than the row passes stage (127 ids;
+// a place may reach one past the end).
+__global__ __launch_bounds__( kThreads ) void kFillHoleSlots( int64_t n, int64_t nslices, LatticeBox L,
+                                                              const int4* __restrict__ ent, int32_t S,
+                                                              const int4* __restrict__ rows, int32_t nrows,
+                                                              const int32_t* __restrict__ site,
+                                                              const int32_t* __restrict__ id, int32_t* __restrict__ col,
+                                                              uint64_t* __restrict__ exist,
+                                                              uint64_t* __restrict__ intact, int4* __restrict__ hole_win,
+                                                              uint8_t* __restrict__ hole_pos, int32_t* __restrict__ flag )
+{
+    const int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    const int64_t slice = p / kSlice;
+    if ( slice >= nslices )
+        return; // whole wavefront
+    const int lane = threadIdx.x & ( kSlice - 1 );
+    const bool valid = p < n;
+    int32_t ix = 0, iy = 0, iz = 0;
+    if ( valid )
+        latticeCoords( site[p], L, ix, iy, iz );
+    const int32_t self = static_cast<int32_t>( valid ? p : slice * kSlice );
+    constexpr int32_t kNone = 0x7fffffff;
+    for ( int32_t r = 0; r < nrows; r++ )
+    {
+        const int4 R = rows[r];
+        int32_t first = kNone, last = -1;
+        for ( int32_t t = 0; t < R.y; t++ )
+        {
+            const int32_t e = R.x + t;
+            const int32_t j = valid ? holeNeighbour( ent[e], ix, iy, iz, L, id ) : -1;
+            const bool ex = j >= 0;
+            col[( slice * S + e ) * kSlice + lane] = ex ? j : self;
+            const uint64_t m = __ballot( ex );
+            if ( lane == 0 )
+            {
+                exist[slice * S + e] = m;
+                intact[slice * S + e] = m;
+            }
+            if ( ex )
+            {
+                first = min( first, j );
+                last = max( last, j );
+            }
+        }
+        // the ids of the lanes before this one end at prev (ids ascend with
+        // the lane: sites do)
+        int32_t run = last;
+        for ( int off = 1; off < kSlice; off <<= 1 )
+        {
+            const int32_t o = __shfl_up( run, off );
+            if ( lane >= off )
+                run = max( run, o );
+        }
+        const int32_t end = __shfl( run, kSlice - 1 );
+        int32_t prev = __shfl_up( run, 1 );
+        if ( lane == 0 )
+            prev = -1;
+        int32_t g = first;
+        for ( int off = 32; off > 0; off >>= 1 )
+            g = min( g, __shfl_xor( g, off ) );
+        int32_t len1 = 2 * kSlice, g2 = 0, len = 0; // one segment
+        if ( end >= 0 )
+        {
+            len = end - g + 1;
+            if ( len > 2 * kSlice - 1 )
+            {
+                // the largest run of ids that no lane needs is left out
+                int32_t gap = first != kNone && prev >= 0 ? first - prev - 1 : 0;
+                int32_t best = gap;
+                for ( int off = 32; off > 0; off >>= 1 )
+                    best = max( best, __shfl_xor( best, off ) );
+                const int src = __builtin_ctzll( __ballot( gap == best ) );
+                len1 = __shfl( prev, src ) - g + 1;
+                g2 = __shfl( first, src );
+                len = len1 + ( end - g2 + 1 );
+                if ( ( best <= 0 || len > 2 * kSlice - 1 ) && lane == 0 )
+                    *flag = 1;
+            }
+        }
+        else
+            g = static_cast<int32_t>( slice * kSlice ); // no bond of the slice in this row
+        int32_t place = 0;
+        if ( first != kNone )
+            place = first - g < len1 ? first - g : first - g2 + len1;
+        hole_pos[( slice * nrows + r ) * kSlice + lane] = static_cast<uint8_t>( min( place, 2 * kSlice - 1 ) );
+        if ( lane == 0 )
+            hole_win[slice * nrows + r] = make_int4( g, len1, g2 - len1, len );
+    }
+}
+
 template <class T>
 void ensure( DevBuf& b, size_t count, MemAccount* acct )
 {
@@ -674,8 +844,8 @@ void launchInvertPerm( const int64_t* perm_dev, int64_t n, int64_t* inv_dev, hip
     PDK_HIP( hipGetLastError() );
 }
 
-bool latticeOrder( const double* x, int64_t n, std::vector<int64_t>& perm, double h_out[3], int64_t dims_out[3],
-                   double* dev_out )
+bool latticeOrder( const double* x, int64_t n, std::vector<int64_t>& perm, double lo_out[3], double h_out[3],
+                   int64_t dims_out[3], double* dev_out )
 {
     if ( n < 2 )
         return false;
@@ -715,6 +885,7 @@ bool latticeOrder( const double* x, int64_t n, std::vector<int64_t>& perm, doubl
             hi = std::max( hi, x[3 * p + d] );
         h_out[d] = nk[d] > 1 ? ( hi - lo[d] ) / static_cast<double>( nk[d] - 1 ) : h[d];
         dims_out[d] = nk[d];
+        lo_out[d] = lo[d];
     }
     double dev = 0.0;
     for ( int d = 0; d < 3; d++ )
@@ -1043,11 +1214,12 @@ struct SlotEntry
 // caller checks the entries against every row of the cell search (horizons of
 // a whole number of spacings plus 1e-10, as most input decks set them, have
 // lattice vectors within 1e-7 of the cutoff).
+// holes: sites may be missing (the caller order must then be the lattice order).
 bool slotStencil( int64_t n, const int64_t dims[3], const double h[3], double rc,
-                  const std::vector<int64_t>& perm_host, double margin, std::vector<SlotEntry>& es,
+                  const std::vector<int64_t>& perm_host, double margin, bool holes, std::vector<SlotEntry>& es,
                   LatticeBox& L, bool& identity )
 {
-    if ( dims[0] * dims[1] * dims[2] != n || static_cast<int64_t>( perm_host.size() ) != n )
+    if ( ( !holes && dims[0] * dims[1] * dims[2] != n ) || static_cast<int64_t>( perm_host.size() ) != n )
         return false;
     // Caller order equal to the lattice order: slots sorted by id offset are
     // sorted by caller id for every particle.  Otherwise the slot order is
@@ -1055,6 +1227,8 @@ bool slotStencil( int64_t n, const int64_t dims[3], const double h[3], double rc
     identity = true;
     for ( int64_t p = 0; p < n && identity; p++ )
         identity = perm_host[p] == p;
+    if ( holes && !identity )
+        return false;
     int32_t K[3];
     for ( int d = 0; d < 3; d++ )
     {
@@ -1111,24 +1285,16 @@ std::vector<int4> slotEntries( const std::vector<SlotEntry>& es )
 
 // Fill the slot arrays, the row table, offsets, the FP32 stencil table and
 // the FP64 |xi|^2 of each entry, and move them into place.
-void finishSlots( int64_t n, int64_t nslices, const LatticeBox& L, const std::vector<SlotEntry>& es,
+// With site and id (missing sites) also the windows; false, with nothing
+// moved, when they do not fit the row passes.
+bool finishSlots( int64_t n, int64_t nslices, const LatticeBox& L, const std::vector<SlotEntry>& es,
                   const int4* dent, const double h[3], DevBuf& col, DevBuf& intact, int64_t* slice_ptr_dev,
                   int64_t& total_rows, int64_t& col_capacity_rows, SlotForm& out, MemAccount* acct,
-                  hipStream_t st )
+                  hipStream_t st, const int32_t* site = nullptr, const int32_t* id = nullptr,
+                  int32_t* flag_dev = nullptr )
 {
     const int32_t S = static_cast<int32_t>( es.size() );
     const int64_t rows = nslices * S;
-    DevBuf ncol, nintact, nexist, dsoff, dtab;
-    ncol.alloc( static_cast<size_t>( rows ) * kSlice * sizeof( int32_t ), acct );
-    nintact.alloc( static_cast<size_t>( rows ) * sizeof( uint64_t ), acct );
-    nexist.alloc( static_cast<size_t>( rows ) * sizeof( uint64_t ), acct );
-    kFillStencilSlots<<<gridFor( nslices * kSlice ), kThreads, 0, st>>>( n, nslices, L, dent, S, ncol.as<int32_t>(),
-                                                                         nexist.as<uint64_t>(), nintact.as<uint64_t>() );
-    PDK_HIP( hipGetLastError() );
-    std::vector<int64_t> sp( nslices + 1 );
-    for ( int64_t k = 0; k <= nslices; k++ )
-        sp[k] = k * S;
-    PDK_HIP( hipMemcpyAsync( slice_ptr_dev, sp.data(), ( nslices + 1 ) * sizeof( int64_t ), hipMemcpyHostToDevice, st ) );
     // Row windows: maximal runs of slots with one (dy, dz) and consecutive dx.
     std::vector<int4> rtab;
     for ( int32_t e = 0; e < S; e++ )
@@ -1162,6 +1328,37 @@ void finishSlots( int64_t n, int64_t nslices, const LatticeBox& L, const std::ve
         drstart.alloc( 9 * sizeof( uint32_t ), acct );
         PDK_HIP( hipMemcpyAsync( drstart.as<uint32_t>(), rs.data(), 9 * sizeof( uint32_t ), hipMemcpyHostToDevice, st ) );
     }
+    if ( site && nrows == 0 )
+        return false;
+    DevBuf ncol, nintact, nexist, dsoff, dtab, nwin, npos;
+    ncol.alloc( static_cast<size_t>( rows ) * kSlice * sizeof( int32_t ), acct );
+    nintact.alloc( static_cast<size_t>( rows ) * sizeof( uint64_t ), acct );
+    nexist.alloc( static_cast<size_t>( rows ) * sizeof( uint64_t ), acct );
+    if ( site )
+    {
+        nwin.alloc( static_cast<size_t>( nslices ) * nrows * sizeof( int4 ), acct );
+        npos.alloc( static_cast<size_t>( nslices ) * nrows * kSlice, acct );
+        PDK_HIP( hipMemsetAsync( flag_dev, 0, sizeof( int32_t ), st ) );
+        kFillHoleSlots<<<gridFor( nslices * kSlice ), kThreads, 0, st>>>(
+            n, nslices, L, dent, S, drows.as<int4>(), nrows, site, id, ncol.as<int32_t>(), nexist.as<uint64_t>(),
+            nintact.as<uint64_t>(), nwin.as<int4>(), npos.as<uint8_t>(), flag_dev );
+        PDK_HIP( hipGetLastError() );
+        int32_t flag = 0;
+        PDK_HIP( hipMemcpyAsync( &flag, flag_dev, sizeof( int32_t ), hipMemcpyDeviceToHost, st ) );
+        PDK_HIP( hipStreamSynchronize( st ) );
+        if ( flag )
+            return false;
+    }
+    else
+    {
+        kFillStencilSlots<<<gridFor( nslices * kSlice ), kThreads, 0, st>>>(
+            n, nslices, L, dent, S, ncol.as<int32_t>(), nexist.as<uint64_t>(), nintact.as<uint64_t>() );
+        PDK_HIP( hipGetLastError() );
+    }
+    std::vector<int64_t> sp( nslices + 1 );
+    for ( int64_t k = 0; k <= nslices; k++ )
+        sp[k] = k * S;
+    PDK_HIP( hipMemcpyAsync( slice_ptr_dev, sp.data(), ( nslices + 1 ) * sizeof( int64_t ), hipMemcpyHostToDevice, st ) );
     std::vector<int32_t> soff( 256, 0 );
     std::vector<float4> tab( 256, make_float4( 0.f, 0.f, 0.f, 1.f ) );
     std::vector<double> tab2( 256, 1.0 );
@@ -1204,8 +1401,12 @@ void finishSlots( int64_t n, int64_t nslices, const LatticeBox& L, const std::ve
     for ( const int4& r : rtab )
         out.row_max = std::max( out.row_max, r.y );
     out.slots = S;
+    out.hole = site != nullptr;
+    out.hole_win = std::move( nwin );
+    out.hole_pos = std::move( npos );
     total_rows = rows;
     col_capacity_rows = rows;
+    return true;
 }
 
 // Direct build check: every in-box stencil bond passes the exact FP64 cutoff
@@ -1262,7 +1463,7 @@ bool buildStencilSlots( const PDArgs& a, const int64_t dims[3], const double h[3
     std::vector<SlotEntry> es;
     LatticeBox L{};
     bool identity = false;
-    if ( !slotStencil( n, dims, h, rc, perm_host, 0.0, es, L, identity ) )
+    if ( !slotStencil( n, dims, h, rc, perm_host, 0.0, false, es, L, identity ) )
         return false;
     const int32_t S = static_cast<int32_t>( es.size() );
     const std::vector<int4> ent = slotEntries( es );
@@ -1278,9 +1479,51 @@ bool buildStencilSlots( const PDArgs& a, const int64_t dims[3], const double h[3
     PDK_HIP( hipStreamSynchronize( st ) );
     if ( flag )
         return false;
-    finishSlots( n, a.nslices, L, es, dent.as<int4>(), h, col, intact, slice_ptr_dev, total_rows, col_capacity_rows,
-                 out, acct, st );
-    return true;
+    return finishSlots( n, a.nslices, L, es, dent.as<int4>(), h, col, intact, slice_ptr_dev, total_rows,
+                        col_capacity_rows, out, acct, st );
+}
+
+bool buildHoleSlots( const PDArgs& a, const int64_t dims[3], const double lo[3], const double h[3], double rc,
+                     const std::vector<int64_t>& perm_host, DevBuf& col, DevBuf& intact, int64_t* slice_ptr_dev,
+                     int64_t& total_rows, int64_t& col_capacity_rows, SlotForm& out, BuildScratch& s, MemAccount* acct,
+                     hipStream_t st )
+{
+    const int64_t n = a.n;
+    // a table of the box's sites: only where at least an eighth of them hold a
+    // particle (sparser ones would mostly stage empty windows anyway)
+    if ( dims[0] > n * 8 / dims[1] / dims[2] )
+        return false;
+    const int64_t box = dims[0] * dims[1] * dims[2];
+    if ( box <= n || box >= ( int64_t( 1 ) << 30 ) )
+        return false;
+    std::vector<SlotEntry> es;
+    LatticeBox L{};
+    bool identity = false;
+    if ( !slotStencil( n, dims, h, rc, perm_host, 0.0, true, es, L, identity ) )
+        return false;
+    const int32_t S = static_cast<int32_t>( es.size() );
+    const std::vector<int4> ent = slotEntries( es );
+    DevBuf dent, site, id;
+    dent.alloc( S * sizeof( int4 ), acct );
+    site.alloc( n * sizeof( int32_t ), acct );
+    id.alloc( box * sizeof( int32_t ), acct );
+    ensure<int32_t>( s.flag, 1, acct );
+    PDK_HIP( hipMemcpyAsync( dent.as<int4>(), ent.data(), S * sizeof( int4 ), hipMemcpyHostToDevice, st ) );
+    PDK_HIP( hipMemsetAsync( s.flag.as<int32_t>(), 0, sizeof( int32_t ), st ) );
+    PDK_HIP( hipMemsetAsync( id.as<int32_t>(), 0xff, box * sizeof( int32_t ), st ) );
+    kSites<<<gridFor( n ), kThreads, 0, st>>>( a.x, n, lo[0], lo[1], lo[2], h[0], h[1], h[2], L, site.as<int32_t>(),
+                                               id.as<int32_t>(), s.flag.as<int32_t>() );
+    kCheckHoleSlots<<<gridFor( n ), kThreads, 0, st>>>( a, L, dent.as<int4>(), S, site.as<int32_t>(),
+                                                        id.as<int32_t>(), s.flag.as<int32_t>() );
+    PDK_HIP( hipGetLastError() );
+    int32_t flag = 0;
+    PDK_HIP( hipMemcpyAsync( &flag, s.flag.as<int32_t>(), sizeof( int32_t ), hipMemcpyDeviceToHost, st ) );
+    PDK_HIP( hipStreamSynchronize( st ) );
+    if ( flag )
+        return false;
+    return finishSlots( n, a.nslices, L, es, dent.as<int4>(), h, col, intact, slice_ptr_dev, total_rows,
+                        col_capacity_rows, out, acct, st, site.as<int32_t>(), id.as<int32_t>(),
+                        s.flag.as<int32_t>() );
 }
 
 bool buildStencilSlotsDirect( const double* x_dev, int64_t n, const int64_t dims[3], const double h[3], double rc,
@@ -1296,7 +1539,7 @@ bool buildStencilSlotsDirect( const double* x_dev, int64_t n, const int64_t dims
     std::vector<SlotEntry> es;
     LatticeBox L{};
     bool identity = false;
-    if ( !slotStencil( n, dims, h, rc, perm_host, 2e-5, es, L, identity ) )
+    if ( !slotStencil( n, dims, h, rc, perm_host, 2e-5, false, es, L, identity ) )
         return false;
     const int32_t S = static_cast<int32_t>( es.size() );
     const std::vector<int4> ent = slotEntries( es );
@@ -1313,9 +1556,8 @@ bool buildStencilSlotsDirect( const double* x_dev, int64_t n, const int64_t dims
     PDK_HIP( hipStreamSynchronize( st ) );
     if ( flag )
         return false;
-    finishSlots( n, ( n + kSlice - 1 ) / kSlice, L, es, dent.as<int4>(), h, col, intact, slice_ptr_dev, total_rows,
-                 col_capacity_rows, out, acct, st );
-    return true;
+    return finishSlots( n, ( n + kSlice - 1 ) / kSlice, L, es, dent.as<int4>(), h, col, intact, slice_ptr_dev,
+                        total_rows, col_capacity_rows, out, acct, st );
 }
 
 void launchPrenotch( const PDArgs& a, int32_t nnotch, const double* notch_dev, hipStream_t st )

@@ -138,9 +138,10 @@ struct PDArgs
     int32_t nrows;          // 0: no row table
     int32_t lat_n[3];       // lattice extent (stencil-slot form)
     // Lattices with missing sites in the stencil-slot form: per slice and row
-    // of the row table the neighbour window (first id, length <= 127) and each
-    // lane's place in it ([slice][row][lane]); null on full lattices.
-    const int2* hole_win;
+    // of the row table the neighbour window (place k holds id k + (k < y ? x : z),
+    // w <= 127 places) and each lane's place in it ([slice][row][lane]); null
+    // on full lattices.
+    const int4* hole_win;
     const uint8_t* hole_pos;
     int32_t row_max;        // longest row of the row table, in slots
     // FP64 row passes: positions, volumes and constants are within the ranges

@@ -158,6 +158,7 @@ __global__ __launch_bounds__( kBlock ) __attribute__( ( amdgpu_waves_per_eu( ( P
     uint32_t elo = 0, ehi = 0, mlo = 0, mhi = 0; // existence words (stencil-slot form)
     const int32_t self = static_cast<int32_t>( pc );
     const uint64_t* __restrict__ exist = SLOTS ? A.exist + base : nullptr;
+    const bool holes = SLOTS && A.hole_win != nullptr;
     auto fetch = [&]( int32_t qb, int32_t( &dst )[SLOTS ? 1 : KB], uint32_t( &sdst )[KB / 4], uint32_t& lo,
                       uint32_t& hi, uint32_t& xlo, uint32_t& xhi ) {
         if constexpr ( SLOTS )
@@ -223,7 +224,8 @@ __global__ __launch_bounds__( kBlock ) __attribute__( ( amdgpu_waves_per_eu( ( P
                 const uint32_t h32 = __builtin_amdgcn_readlane( ehi, g + k );
                 const uint64_t e = ( static_cast<uint64_t>( h32 ) << 32 ) | l32;
                 ex[k] = ( e >> lane ) & 1ull;
-                jj[k] = ex[k] ? p + soffs[q0 + k] : pc;
+                // (missing sites: the stored neighbour id)
+                jj[k] = ex[k] ? ( holes ? static_cast<int64_t>( colp[( q0 + k ) * kSlice] ) : p + soffs[q0 + k] ) : pc;
             }
             else
             {
@@ -1900,7 +1902,7 @@ const char* lpsKernelName( const PDArgs& a )
 // stretch (the same results either way).
 static bool outputRows( const PDArgs& a )
 {
-    if ( a.rows == nullptr || a.nrows <= 0 || a.exist == nullptr )
+    if ( a.rows == nullptr || a.nrows <= 0 || a.exist == nullptr || a.hole_win != nullptr )
         return false;
     const bool lps = a.model == kLPS || a.model == kLinLPS;
     const int feat = ( a.mtype ? kFeatMT : 0 ) | ( !lps && a.temp ? kFeatTH : 0 ) | ( !lps && a.splas ? kFeatEP : 0 );
@@ -2147,7 +2149,7 @@ void launchHeatTransfer( const PDArgs* args_dev, const PDArgs& a, double dt, hip
     if ( a.nslices == 0 )
         return;
     auto fn = a.fracture ? kHeatConduction<true> : kHeatConduction<false>;
-    if ( a.rows != nullptr && a.nrows > 0 && a.exist != nullptr )
+    if ( a.rows != nullptr && a.nrows > 0 && a.exist != nullptr && a.hole_win == nullptr )
         fn = a.vol_uniform ? ( a.fracture ? kHeatConductionRows<true, false> : kHeatConductionRows<false, false> )
                            : ( a.fracture ? kHeatConductionRows<true, true> : kHeatConductionRows<false, true> );
     hipLaunchKernelGGL( fn, dim3( sliceBlocks( a ) ), dim3( kBlock ), 0, st, args_dev );

@@ -142,8 +142,8 @@ void launchMortonOrder( const double* x_aos_dev, int64_t n, const double lo[3], 
 // its site lo + k h along an axis, as a fraction of that axis' spacing, plus
 // the rounding of the site (stencil bond vectors differ from x_j - x_i by at
 // most twice that per axis).
-bool latticeOrder( const double* x_aos_host, int64_t n, std::vector<int64_t>& perm, double h_out[3],
-                   int64_t dims_out[3], double* dev_out );
+bool latticeOrder( const double* x_aos_host, int64_t n, std::vector<int64_t>& perm, double lo_out[3],
+                   double h_out[3], int64_t dims_out[3], double* dev_out );
 // Stencil ids of a lattice specimen's bonds (mixed form); false when some
 // bond is not a lattice vector or the stencil has more than 255 entries.
 bool buildStencil( const PDArgs& a, const double h[3], double rc, int64_t total_rows, DevBuf& sid, DevBuf& table,
@@ -169,6 +169,13 @@ bool buildStencilSlots( const PDArgs& a, const int64_t dims[3], const double h[3
                         const std::vector<int64_t>& perm_host, DevBuf& col, DevBuf& intact, int64_t* slice_ptr_dev,
                         int64_t& total_rows, int64_t& col_capacity_rows, SlotForm& out, BuildScratch& s,
                         MemAccount* acct, hipStream_t st );
+// The same form for a lattice with missing sites (rows checked against the
+// compact ones as above; caller order = lattice order); adds the neighbour
+// windows that the row passes stage.
+bool buildHoleSlots( const PDArgs& a, const int64_t dims[3], const double lo[3], const double h[3], double rc,
+                     const std::vector<int64_t>& perm_host, DevBuf& col, DevBuf& intact, int64_t* slice_ptr_dev,
+                     int64_t& total_rows, int64_t& col_capacity_rows, SlotForm& out, BuildScratch& s, MemAccount* acct,
+                     hipStream_t st );
 // The same form built without the cell search: every in-box stencil bond is
 // checked with the exact cutoff test; fills cnt.  False (nothing written but
 // cnt) when the lattice does not qualify.

@@ -585,7 +585,12 @@ __device__ __forceinline__ double addRound( const SplitTerms<W, ND, NF>& T, int 
 // W: waves per slice (1, or a split slice).  HOLE: a lattice with missing
 // sites: the neighbour window of (slice, row) and each lane's place in it come
 // from the build's tables (PDArgs::hole_win, hole_pos), and a lane's place
-// moves on by one with every neighbour that exists.
+// moves on by one with every neighbour that exists.  Two vector instructions
+// and a scalar load a slot more than on full lattices, where the gathers of the
+// compact form read 5 bytes of ids a bond and took a wavefront's neighbour
+// data from three to twelve scattered loads: 100 mixed steps of a 423k-particle
+// perforated plate 26.5 -> 11.0 ms, 100 FP64 elastic-plastic steps of a 29k
+// dogbone 14.2 -> 5.3 ms.
 // G: slots evaluated together (1: one after the other).
 template <int MODEL, bool FRAC, int PREC, bool GEN, int W = 1, bool HOLE = false, int G = 1>
 __global__ __launch_bounds__( W == 1 ? kBlock : W * kSlice ) __attribute__( ( amdgpu_waves_per_eu( ( MODEL == 1 || MODEL == 5 || G > 1 ) ? 1 : 6, 8 ) ) ) void
@@ -716,12 +721,7 @@ kForceRows( const PDArgs* __restrict__ specs,
     if constexpr ( GEN )
         rs[KV] = bufferOf( volp, nbytes );
     const uint32_t lane8 = static_cast<uint32_t>( lane ) * 8u;
-    // 64 window values starting at id g (uniform) into dst.
-    auto loadHalf = [&]( double* dst, int32_t g ) {
-        // g >= 0: lane offset + uniform start; g < 0: per-lane offsets, the
-        // negative ones wrap out of range and read 0
-        const uint32_t vo = g >= 0 ? lane8 : static_cast<uint32_t>( g + lane ) * 8u;
-        const uint32_t so = g >= 0 ? static_cast<uint32_t>( g ) * 8u : 0u;
+    auto loadAt = [&]( double* dst, uint32_t vo, uint32_t so ) {
 #pragma unroll
         for ( int k = 0; k < KV; k++ )
             dst[k] = bufferLoad64( rs[k], vo, so );
@@ -731,26 +731,36 @@ kForceRows( const PDArgs* __restrict__ specs,
             dst[KNF] = ( FRAC && bufferLoad8( rnf, vo >> 3, so >> 3 ) != 0 ) ? 1.0 : 0.0;
         }
     };
+    // 64 window values starting at id g (uniform) into dst.
+    auto loadHalf = [&]( double* dst, int32_t g ) {
+        // g >= 0: lane offset + uniform start; g < 0: per-lane offsets, the
+        // negative ones wrap out of range and read 0
+        loadAt( dst, g >= 0 ? lane8 : static_cast<uint32_t>( g + lane ) * 8u,
+                g >= 0 ? static_cast<uint32_t>( g ) * 8u : 0u );
+    };
+    auto loadIds = [&]( double* dst, int32_t id ) { loadAt( dst, static_cast<uint32_t>( id ) * 8u, 0u ); };
     // Window of row r: ids g .. g + 63 (every lane) and g + 64 .. g + 64 + c - 2
     // (lanes < c - 1); with holes, ids and length from the build's table.
     const int nrows = scalarLoad( &A.nrows );
     const int64_t hole0 = HOLE ? w.slice * nrows : 0;
-    const int2* __restrict__ hwin = HOLE ? scalarLoad( &A.hole_win ) + hole0 : nullptr;
+    const int4* __restrict__ hwin = HOLE ? scalarLoad( &A.hole_win ) + hole0 : nullptr;
     const uint8_t* __restrict__ hpos = HOLE ? scalarLoad( &A.hole_pos ) + hole0 * kSlice + lane : nullptr;
-    int32_t gnext = 0, pnext = 0; // window start and place of the row being loaded
+    int4 wnext{};      // (HOLE) window and place of the row being loaded
+    int32_t pnext = 0;
     auto loadRow = [&]( int r ) {
         const int4 R = scalarLoad4( rows + r );
-        int32_t g = p032 + R.z; // uniform
-        int32_t more = R.y - 1;
         if constexpr ( HOLE )
         {
-            g = scalarLoad( &hwin[r].x );
-            more = scalarLoad( &hwin[r].y ) - kSlice;
+            wnext = scalarLoad4( hwin + r );
             pnext = hpos[r * kSlice];
+            loadIds( v0, lane + ( lane < wnext.y ? wnext.x : wnext.z ) );
+            if ( lane + kSlice < wnext.w )
+                loadIds( v1, lane + kSlice + ( lane + kSlice < wnext.y ? wnext.x : wnext.z ) );
+            return;
         }
-        gnext = g;
+        const int32_t g = p032 + R.z; // uniform
         loadHalf( v0, g );
-        if ( lane < more )
+        if ( lane < R.y - 1 )
             loadHalf( v1, g + kSlice );
     };
 
@@ -804,7 +814,8 @@ kForceRows( const PDArgs* __restrict__ specs,
     auto evalRow = [&]( const int r ) __attribute__( ( always_inline ) ) {
         const int4 R = scalarLoad4( rows + r );
         double* __restrict__ wb = &win[wv][NBUF == 2 ? r & 1 : 0][0][0];
-        const int32_t gwin = gnext, pos0 = pnext;
+        const int4 hw = wnext;
+        const int32_t pos0 = pnext;
         if constexpr ( NBUF == 1 )
         {
             // the previous row's window reads stay above this row's stores
@@ -993,8 +1004,8 @@ kForceRows( const PDArgs* __restrict__ specs,
                             // whole pass), the displacements are the registers
                             // and the window
                             __asm__ volatile( "" ::: "memory" );
-                            // (with holes: window start + the lane's place)
-                            const int64_t jo = HOLE ? static_cast<int64_t>( gwin ) + ( pos - lane ) : p0 + R.z + t;
+                            // (with holes: the id at the lane's place)
+                            const int64_t jo = HOLE ? static_cast<int64_t>( pos - lane + ( pos < hw.y ? hw.x : hw.z ) ) : p0 + R.z + t;
                             const double* __restrict__ xj = x + jo;
                             const double* __restrict__ xp = x + p0;
                             Bond64 e;
@@ -1541,11 +1552,7 @@ __global__ __launch_bounds__( W == 1 ? kBlock : W * kSlice ) __attribute__( ( am
 #pragma unroll
     for ( int k = 0; k < NC; k++ )
         v1[k] = 0.0;
-    auto loadHalf = [&]( double* dst, int32_t g ) {
-        // g >= 0: lane offset + uniform start; g < 0: per-lane offsets, the
-        // negative ones wrap out of range and read 0
-        const uint32_t vo = g >= 0 ? lane8 : static_cast<uint32_t>( g + lane ) * 8u;
-        const uint32_t so = g >= 0 ? static_cast<uint32_t>( g ) * 8u : 0u;
+    auto loadAt = [&]( double* dst, uint32_t vo, uint32_t so ) {
 #pragma unroll
         for ( int k = 0; k <= KV; k++ )
             dst[k] = bufferLoad64( rs[k], vo, so );
@@ -1561,24 +1568,33 @@ __global__ __launch_bounds__( W == 1 ? kBlock : W * kSlice ) __attribute__( ( am
         if constexpr ( TH )
             dst[KH] = bufferLoad64( rth, vo, so );
     };
+    auto loadHalf = [&]( double* dst, int32_t g ) {
+        // g >= 0: lane offset + uniform start; g < 0: per-lane offsets, the
+        // negative ones wrap out of range and read 0
+        loadAt( dst, g >= 0 ? lane8 : static_cast<uint32_t>( g + lane ) * 8u,
+                g >= 0 ? static_cast<uint32_t>( g ) * 8u : 0u );
+    };
+    auto loadIds = [&]( double* dst, int32_t id ) { loadAt( dst, static_cast<uint32_t>( id ) * 8u, 0u ); };
     const int nrows = scalarLoad( &A.nrows );
     const int64_t hole0 = HOLE ? w.slice * nrows : 0;
-    const int2* __restrict__ hwin = HOLE ? scalarLoad( &A.hole_win ) + hole0 : nullptr;
+    const int4* __restrict__ hwin = HOLE ? scalarLoad( &A.hole_win ) + hole0 : nullptr;
     const uint8_t* __restrict__ hpos = HOLE ? scalarLoad( &A.hole_pos ) + hole0 * kSlice + lane : nullptr;
-    int32_t gnext = 0, pnext = 0; // window start and place of the row being loaded
+    int4 wnext{};      // (HOLE) window and place of the row being loaded
+    int32_t pnext = 0;
     auto loadRow = [&]( int r ) {
         const int4 R = scalarLoad4( rows + r );
-        int32_t g = p032 + R.z; // uniform
-        int32_t more = R.y - 1;
         if constexpr ( HOLE )
         {
-            g = scalarLoad( &hwin[r].x );
-            more = scalarLoad( &hwin[r].y ) - kSlice;
+            wnext = scalarLoad4( hwin + r );
             pnext = hpos[r * kSlice];
+            loadIds( v0, lane + ( lane < wnext.y ? wnext.x : wnext.z ) );
+            if ( lane + kSlice < wnext.w )
+                loadIds( v1, lane + kSlice + ( lane + kSlice < wnext.y ? wnext.x : wnext.z ) );
+            return;
         }
-        gnext = g;
+        const int32_t g = p032 + R.z; // uniform
         loadHalf( v0, g );
-        if ( lane < more )
+        if ( lane < R.y - 1 )
             loadHalf( v1, g + kSlice );
     };
 
@@ -1639,7 +1655,8 @@ __global__ __launch_bounds__( W == 1 ? kBlock : W * kSlice ) __attribute__( ( am
     };
     auto evalRow = [&]( const int r ) __attribute__( ( always_inline ) ) {
         const int4 R = scalarLoad4( rows + r );
-        const int32_t gwin = gnext, pos0 = pnext;
+        const int4 hw = wnext;
+        const int32_t pos0 = pnext;
         // the previous row's window reads stay above this row's stores (a
         // lane's read of a position another lane overwrites)
         __builtin_amdgcn_fence( __ATOMIC_RELEASE, "wavefront" );
@@ -1794,7 +1811,7 @@ __global__ __launch_bounds__( W == 1 ? kBlock : W * kSlice ) __attribute__( ( am
                             // x_i from being hoisted into registers held for
                             // the whole pass)
                             __asm__ volatile( "" ::: "memory" );
-                            const int64_t j = HOLE ? static_cast<int64_t>( gwin ) + pos : p + R.z + t;
+                            const int64_t j = HOLE ? static_cast<int64_t>( pos + ( pos < hw.y ? hw.x : hw.z ) ) : p + R.z + t;
                             Bond64 e;
                             getDistance64( x[p], x[n + p], x[2 * n + p], ui0, ui1, ui2, x[j], x[n + j], x[2 * n + j],
                                            uj0, uj1, uj2, e );
@@ -2093,31 +2110,36 @@ __global__ __launch_bounds__( W == 1 ? kBlock : W * kSlice ) void kLpsStateRows(
     if constexpr ( GEN )
         rs[KV] = bufferOf( volp, nbytes );
     const uint32_t lane8 = static_cast<uint32_t>( lane ) * 8u;
-    auto loadHalf = [&]( double* dst, int32_t g ) {
-        const uint32_t vo = g >= 0 ? lane8 : static_cast<uint32_t>( g + lane ) * 8u;
-        const uint32_t so = g >= 0 ? static_cast<uint32_t>( g ) * 8u : 0u;
+    auto loadAt = [&]( double* dst, uint32_t vo, uint32_t so ) {
 #pragma unroll
         for ( int k = 0; k < NC; k++ )
             dst[k] = bufferLoad64( rs[k], vo, so );
     };
+    auto loadHalf = [&]( double* dst, int32_t g ) {
+        loadAt( dst, g >= 0 ? lane8 : static_cast<uint32_t>( g + lane ) * 8u,
+                g >= 0 ? static_cast<uint32_t>( g ) * 8u : 0u );
+    };
+    auto loadIds = [&]( double* dst, int32_t id ) { loadAt( dst, static_cast<uint32_t>( id ) * 8u, 0u ); };
     const int nrows = scalarLoad( &A.nrows );
     const int64_t hole0 = HOLE ? w.slice * nrows : 0;
-    const int2* __restrict__ hwin = HOLE ? scalarLoad( &A.hole_win ) + hole0 : nullptr;
+    const int4* __restrict__ hwin = HOLE ? scalarLoad( &A.hole_win ) + hole0 : nullptr;
     const uint8_t* __restrict__ hpos = HOLE ? scalarLoad( &A.hole_pos ) + hole0 * kSlice + lane : nullptr;
     const uint64_t* __restrict__ exw = HOLE ? scalarLoad( &A.exist ) + row0 : nullptr;
     int32_t pnext = 0; // place in the window of the row being loaded
     auto loadRow = [&]( int r ) {
         const int4 R = scalarLoad4( rows + r );
-        int32_t g = p032 + R.z; // uniform
-        int32_t more = R.y - 1;
         if constexpr ( HOLE )
         {
-            g = scalarLoad( &hwin[r].x );
-            more = scalarLoad( &hwin[r].y ) - kSlice;
+            const int4 wnext = scalarLoad4( hwin + r );
             pnext = hpos[r * kSlice];
+            loadIds( v0, lane + ( lane < wnext.y ? wnext.x : wnext.z ) );
+            if ( lane + kSlice < wnext.w )
+                loadIds( v1, lane + kSlice + ( lane + kSlice < wnext.y ? wnext.x : wnext.z ) );
+            return;
         }
+        const int32_t g = p032 + R.z; // uniform
         loadHalf( v0, g );
-        if ( lane < more )
+        if ( lane < R.y - 1 )
             loadHalf( v1, g + kSlice );
     };
     // split: a bond's terms -- FP64: the one of the sum being formed; mixed:

@@ -94,3 +94,104 @@ def test_split_slices_match_gathers(kind, precision):
         assert "Rows" in out[0][4] and "Rows" not in out[1][4]
         for a, b in zip(out[0][:4], out[1][:4]):
             assert np.array_equal(a, b)
+
+
+def cut(w, dims, keep):
+    """Keep the particles of a box (x fastest) where keep(i, j, k)."""
+    k, j, i = np.meshgrid(*(np.arange(d) for d in dims[::-1]), indexing="ij")
+    m = keep(i.ravel(), j.ravel(), k.ravel())
+    for key in ("x", "vol", "rho", "u", "v"):
+        w[key] = np.ascontiguousarray(w[key][m])
+    return w
+
+
+SHAPES = {
+    "hole": ((40, 31, 6), lambda i, j, k: (i - 20) ** 2 + (j - 13) ** 2 > 49),
+    "waist": ((251, 17, 5), lambda i, j, k: np.abs(j - 8) <= np.where(np.abs(i - 125) < 50, 3, 8)),
+    "random": ((23, 19, 11), lambda i, j, k: np.random.default_rng(3).random(i.size) < 0.8),
+    "sparse": ((25, 25, 9), lambda i, j, k: np.random.default_rng(4).random(i.size) < 0.2),
+    "corner": ((33, 20, 12), lambda i, j, k: ~((i > 15) & (j > 8))),
+    "comb": ((64, 20, 6), lambda i, j, k: (j % 5 > 1) | (i % 9 == 0)),
+    "steps": ((150, 12, 4), lambda i, j, k: i < np.where(j < 6, 9, 150)),
+}
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("kind", ["pmb", "pmb_elastic", "lps", "lps_elastic", "epp", "materials", "thermal"])
+def test_missing_sites_match_compact(kind, precision):
+    """Lattices with missing sites on row windows, one wave per slice and
+    split, against the compact form and against the gathers over the same
+    layout: the same bonds, bits (FP64) and output passes.  (steps, comb: windows
+    longer than the passes stage; the build keeps the compact form.)"""
+    big = ((120, 81, 20), lambda i, j, k: (i - 60) ** 2 + (j - 30) ** 2 > 400)
+    for name, (dims, keep) in dict(SHAPES, big=big).items():
+        w = box("LPS" if kind in ("lps", "lps_elastic", "materials") else "PMB", dims, 3.01,
+                kind not in ("pmb_elastic", "lps_elastic", "thermal"))
+        cut(w, dims, keep)
+        d = w["desc"]
+        n = w["x"].shape[0]
+        rng = np.random.default_rng(6)
+        if kind == "epp":
+            d.mechanics, d.sigma_y = 1, 2.5e7
+        if kind == "thermal":
+            d.thermal, d.alpha, d.temp0, d.kappa, d.cp, d.thermal_subcycle = 2, 1e-6, 20.0, 10.0, 1.0, 2
+            w["temperature"] = 20.0 + 40.0 * rng.random(n)
+        if kind == "materials":
+            w["materials"] = ([(4.3e10, 2.9e10, 3.8), (8e10, 5e10, 38.0)], (rng.random(n) < 0.4).astype(np.int32))
+        d.precision = precision
+        out = []
+        for layout, variant in ((0, None), (PDK_BONDS_COMPACT, None), (0, 4)):
+            d.bond_layout = layout
+            s = engine.Spec(ctx(), d, n)
+            configs.upload(s, w)
+            configs.setup(s, w)
+            if variant is not None:
+                s.set_tuning(variant)
+            s.step(5)
+            s.compute_energy()
+            s.compute_stress()
+            out.append(dict(bonds=s.bonds(), name=s.kernel_name(0), lay=s.layout(),
+                            **{f: s.get(f) for f in ("u", "v", "f", "W", "stress")}))
+            s.close()
+        say(f"case: {kind} {name} precision {precision}: {n} particles, {out[0]['name']}")
+        assert ("Rows" in out[0]["name"]) == (name not in ("steps", "comb"))
+        assert not out[0]["lay"]["stencil_slots"]
+        for o in out[1:]:
+            for b in range(3):
+                assert np.array_equal(out[0]["bonds"][b], o["bonds"][b])
+            for f in ("u", "v", "f", "W", "stress"):
+                if precision == 0 or o is out[2]:
+                    assert np.array_equal(out[0][f], o[f], equal_nan=True), f
+                else:
+                    assert rel_err(np.nan_to_num(out[0][f]), np.nan_to_num(o[f])) <= 1e-6, f
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+def test_missing_sites_in_the_batch(precision):
+    """Specimens with missing sites beside full ones in one batch: each as alone."""
+    ws = []
+    for name in ("hole", "corner", "random"):
+        dims, keep = SHAPES[name]
+        ws.append(cut(box("PMB", dims, 3.01, True), dims, keep))
+    ws.append(box("PMB", (20, 21, 9), 3.01, True))
+    ws.append(cut(box("LPS", (21, 20, 9), 3.01, True), (21, 20, 9), lambda i, j, k: i + j > 6))
+    specs, alone = [], []
+    for w in ws:
+        w["desc"].precision = precision
+        pair = []
+        for _ in range(2):
+            s = engine.Spec(ctx(), w["desc"], w["x"].shape[0])
+            configs.upload(s, w)
+            configs.setup(s, w)
+            pair.append(s)
+        pair[1].step(12)
+        alone.append([pair[1].get(f) for f in ("u", "v", "f")])
+        pair[1].close()
+        specs.append(pair[0])
+    for s in specs:
+        ctx().submit(s, 12)
+    ctx().progress()
+    for s, ref in zip(specs, alone):
+        for f, r in zip(("u", "v", "f"), ref):
+            assert np.array_equal(s.get(f), r, equal_nan=True)
+        s.close()
