@@ -198,7 +198,7 @@ struct pdk_spec_s
     DevBuf x, U0, U1, v, f, vol, rho, nofail, bcflag, body, m, theta, lpsA, lpsB, W, phi, perm, inv, cnt,
         slice_ptr, col, intact, radius, u_neigh, partial, args, notch, staging, sid, stab, stab_xi2d, stab_xiv, stress, mtype,
         splas,
-        temp, cond;
+        temp, cond, pair_rec;
     // Prescribed values (force_update == false conditions): members (device
     // ids), a and b ([count][ncomp]); one set for U and one for TEMPERATURE.
     struct Prescribed
@@ -252,10 +252,11 @@ struct pdk_spec_s
     // contact bookkeeping
     int64_t steps_since_build = 0;
     double max_disp = 0.0;
-    // contact step: pinned host copy of the largest displacement since the
-    // last build, and the event after its copy (the host waits on that, not
-    // on the stream)
+    // contact step: the largest displacement since the last build, in pinned
+    // host memory that the device writes, and the event after that (the host
+    // waits on it, not on the stream)
     double* disp_pinned = nullptr;
+    double* disp_dev = nullptr; // its device address
     hipEvent_t disp_ready = nullptr;
     double radius_max = 0.0; // largest per-particle radius (polydisperse contact)
     // timing
@@ -404,6 +405,9 @@ struct pdk_spec_s
         h.stress = stress.as<double>();
         h.radius = radius ? radius.as<double>() : nullptr;
         h.u_neigh = u_neigh ? u_neigh.as<double>() : nullptr;
+        h.rec_x = pair_rec.as<double4>();
+        h.rec_u = pair_rec ? h.rec_x + n : nullptr;
+        h.rec_v = pair_rec ? h.rec_x + 2 * n : nullptr;
         h.sid = sid ? sid.as<uint8_t>() : nullptr;
         h.stencil = stab ? stab.as<float4>() : nullptr;
         h.stencil_xi2d = stab_xi2d ? stab_xi2d.as<double>() : nullptr;
@@ -892,6 +896,7 @@ int pdk_spec_create( pdk_ctx ctx, const pdk_model_desc* desc, int64_t n, pdk_spe
         if ( isContact( *desc ) )
         {
             s->u_neigh.alloc( d3, a );
+            s->pair_rec.alloc( 3 * n * sizeof( double4 ), a );
             if ( desc->polydisperse )
                 s->radius.alloc( d1, a );
         }
@@ -1180,7 +1185,7 @@ int pdk_spec_bytes( pdk_spec s, uint64_t* bytes )
         for ( const DevBuf* b : { &s->x, &s->U0, &s->U1, &s->v, &s->f, &s->vol, &s->rho, &s->nofail, &s->bcflag,
                                   &s->body, &s->m, &s->theta, &s->lpsA, &s->lpsB, &s->W, &s->phi, &s->perm, &s->inv,
                                   &s->cnt, &s->slice_ptr, &s->col, &s->intact, &s->radius, &s->u_neigh,
-                                  &s->partial, &s->args, &s->sid, &s->stab, &s->stab_xi2d, &s->stab_xiv } )
+                                  &s->pair_rec, &s->partial, &s->args, &s->sid, &s->stab, &s->stab_xi2d, &s->stab_xiv } )
             t += b->bytes();
         *bytes = t;
     } );
@@ -2328,9 +2333,11 @@ ContactState contactState( pdk_spec s )
     if ( !s->disp_pinned )
     {
         PDK_HIP( hipHostMalloc( reinterpret_cast<void**>( &s->disp_pinned ), sizeof( double ), hipHostMallocDefault ) );
+        PDK_HIP( hipHostGetDevicePointer( reinterpret_cast<void**>( &s->disp_dev ), s->disp_pinned, 0 ) );
         PDK_HIP( hipEventCreateWithFlags( &s->disp_ready, hipEventDisableTiming ) );
     }
     c.disp_pinned = s->disp_pinned;
+    c.disp_dev = s->disp_dev;
     c.disp_ready = s->disp_ready;
     return c;
 }

@@ -99,6 +99,9 @@ struct PDArgs
     double* stress;         // [9][n], component 3 a + b (null until the first stress pass)
     const double* radius;   // contact: per-particle radius or null
     double* u_neigh;        // contact: u at last list build [3][n]
+    double4* rec_x;         // contact: pair records (x, radius), (u, rho V), (v, 0) per particle
+    double4* rec_u;
+    double4* rec_v;
     double* block_partial;  // energy / max-displacement partials
     // model constants
     double c, bcc, s0, theta_coeff, s_coeff;

@@ -15,6 +15,7 @@
 #include <cmath>
 #include <vector>
 
+#include "pdk_rows.hpp"
 #include "pdk_serving.hpp"
 
 namespace pdk
@@ -195,9 +196,43 @@ __device__ double normalForce( const PDArgs& A, const PairK& pk, double r, doubl
     }
 }
 
+// ---------------------------------------------------------------------------
+// Pair records: what a pair force reads of its neighbour, in three 32-byte
+// records (position and radius; displacement and mass; velocity) instead of
+// twelve gathered doubles.  The neighbours of a wavefront are scattered, so a
+// gather costs one cache line a lane and array: 64 lanes touched about 300
+// lines per slot.  rec_x follows the upload; rec_u and rec_v are written by the
+// pass that advances u and v.  The mass is the product rho V that the pair
+// formed before.
+// ---------------------------------------------------------------------------
+__global__ __launch_bounds__( 256 ) void kContactPack( const PDArgs* __restrict__ specs, int32_t parity )
+{
+#pragma clang fp contract( off )
+    const PDArgs& A = *specs;
+    const int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    const int64_t n = A.n;
+    if ( p >= n )
+        return;
+    const double* u = A.U[parity];
+    A.rec_x[p] = make_double4( A.x[p], A.x[n + p], A.x[2 * n + p], A.radius ? A.radius[p] : 0.0 );
+    A.rec_u[p] = make_double4( u[p], u[n + p], u[2 * n + p], A.rho[p] * A.vol[p] );
+    A.rec_v[p] = make_double4( A.v[p], A.v[n + p], A.v[2 * n + p], 0.0 );
+}
+
+// Hertz-JKR: a listed pair farther apart than its tear distance exerts
+// nothing, and the patch radius (a cube root, four square roots, a dozen
+// divisions) is most of the pass (VALU bound, 71 % of its cycles).  Each lane
+// first marks the pairs that may reach (a squared distance against a bound),
+// then evaluates the marked ones in list order: a wavefront runs the patch as
+// often as its busiest lane has touching neighbours, not once per listed slot.  A skipped pair adds zero times its unit normal, which
+// leaves the sum as it is (pairs that are not at a finite distance are not
+// skipped).  Undamped or not, Hertz evaluates every listed pair: its zero
+// depends on the velocities being finite.
+// (Hertz-JKR, 442k polydisperse spheres, 12 listed neighbours of which about
+// 3 touch: 139 -> 127 us; 71 % of the cycles issue VALU work.  Marking by the
+// estimated tear distance of each pair instead of the bound: 140.)
 template <bool POLY, bool JKR>
-__global__ __launch_bounds__( kBlock ) void kContact( const PDArgs* __restrict__ specs, int32_t epi,
-                                                      int32_t parity )
+__global__ __launch_bounds__( kBlock ) void kContact( const PDArgs* __restrict__ specs, int32_t epi )
 {
 #pragma clang fp contract( off )
     const PDArgs& A = *specs;
@@ -209,15 +244,14 @@ __global__ __launch_bounds__( kBlock ) void kContact( const PDArgs* __restrict__
     const int64_t p = slice * kSlice + lane;
     if ( p >= n )
         return; // no cross-lane operations in this kernel
-    const double* __restrict__ x = A.x;
-    const double* __restrict__ u = A.U[parity];
-    const double* __restrict__ v = A.v;
-    const double xi0 = x[p], xi1 = x[n + p], xi2 = x[2 * n + p];
-    const double ui0 = u[p], ui1 = u[n + p], ui2 = u[2 * n + p];
-    const double vi0 = v[p], vi1 = v[n + p], vi2 = v[2 * n + p];
+    const double4* __restrict__ rec_x = A.rec_x;
+    const double4* __restrict__ rec_u = A.rec_u;
+    const double4* __restrict__ rec_v = A.rec_v;
+    const double4 xi = rec_x[p], ui = rec_u[p], vi = rec_v[p];
     const double vol_i = A.vol[p];
     const double rho_i = A.rho[p];
-    const double Ri = POLY ? A.radius[p] : 0.0;
+    const double mi = ui.w;
+    const double Ri = xi.w;
     const int32_t mycnt = A.cnt[p];
     const int64_t base = A.slice_ptr[slice];
     const int32_t* __restrict__ colp = A.col + base * kSlice + lane;
@@ -228,36 +262,53 @@ __global__ __launch_bounds__( kBlock ) void kContact( const PDArgs* __restrict__
     pk.two_r = A.two_r;
     pk.ms = ( rho_i * vol_i ) / 2.0;
     double fx = 0.0, fy = 0.0, fz = 0.0;
-    for ( int32_t q = 0; q < mycnt; q++ )
-    {
-        const int64_t j = colp[q * kSlice];
-        const double rx = ( x[j] - xi0 ) + ( u[j] - ui0 );
-        const double ry = ( x[n + j] - xi1 ) + ( u[n + j] - ui1 );
-        const double rz = ( x[2 * n + j] - xi2 ) + ( u[2 * n + j] - ui2 );
-        const double r = sqrt( rx * rx + ry * ry + rz * rz );
-        const double nx = rx / r, ny = ry / r, nz = rz / r;
-        const double vx = v[j] - vi0, vy = v[n + j] - vi1, vz = v[2 * n + j] - vi2;
+    // The estimated tear distance of a polydisperse JKR pair and whether it
+    // decides on which side of it dn lies: an estimate within 3e-4 relative
+    // decides unless dn lies within 1e-3 of it.
+    auto tearEstimate = [&]( double Rs, double dn, double& xa, double& dte ) {
+        xa = 9.0 / 2.0 * A.Gamma * kPi / A.Es * crSq( Rs );
+        // (pow(6, -1/3) of the host's libm, as the oracle evaluates it)
+        const double a0e = cbrtEstimate( xa );
+        dte = -1.0 / 2.0 * A.jkr_c6 * crSq( a0e ) / Rs;
+        return xa > 0.0 && xa < 1e300 && fabs( dte ) > 1e-290 && fabs( dte ) < 1e290 &&
+               fabs( dn - dte ) > 1e-3 * fabs( dte );
+    };
+    auto pairForce = [&]( const double4 xj, const double4 uj, const double4 vj ) {
+        const double rx = ( xj.x - xi.x ) + ( uj.x - ui.x );
+        const double ry = ( xj.y - xi.y ) + ( uj.y - ui.y );
+        const double rz = ( xj.z - xi.z ) + ( uj.z - ui.z );
+        // |r| and the normal from one reciprocal root where that gives the
+        // general code's bits (pdk_rows.hpp: ordinary magnitudes, and not the
+        // one mantissa whose reciprocal it misses)
+        const double r2 = rx * rx + ry * ry + rz * rz;
+        const Root64 rr = rootRecip( r2 );
+        double r = rr.r, nx = divBy( rx, r, rr.y ), ny = divBy( ry, r, rr.y ), nz = divBy( rz, r, rr.y );
+        auto plain = []( double a ) { return a == 0.0 || fabs( a ) >= 0x1p-300; };
+        if ( !( r2 >= 0x1p-400 && r2 <= 0x1p400 ) || !plain( rx ) || !plain( ry ) || !plain( rz ) ||
+             lowWord( r ) == 0xffffffffu )
+        {
+            r = sqrt( r2 );
+            nx = rx / r;
+            ny = ry / r;
+            nz = rz / r;
+        }
+        const double vx = vj.x - vi.x, vy = vj.y - vi.y, vz = vj.z - vi.z;
         const double vn = vx * nx + vy * ny + vz * nz;
         if constexpr ( POLY )
         {
-            const double Rj = A.radius[j];
+            const double Rj = xj.w;
             pk.Rs = Ri * Rj / ( Ri + Rj );
             pk.two_r = Ri + Rj;
             if constexpr ( JKR )
             {
                 pk.coeff_h_n = 4.0 / 3.0 * A.Es / pk.Rs;
-                const double xa = 9.0 / 2.0 * A.Gamma * kPi / A.Es * crSq( pk.Rs );
                 // The tear distance only places delta_n = 2R - r on one side
-                // of it (normalForce): an estimate within 3e-4 relative
-                // decides unless delta_n lies within 1e-3 of it, and only
-                // then is the correctly rounded value formed.  The decision,
-                // and with it every force, is that of the exact value.
-                // (pow(6, -1/3) of the host's libm, as the oracle evaluates it)
-                const double a0e = cbrtEstimate( xa );
-                const double dte = -1.0 / 2.0 * A.jkr_c6 * crSq( a0e ) / pk.Rs;
+                // of it (normalForce): only where the estimate does not
+                // decide is the correctly rounded value formed.  The
+                // decision, and with it every force, is that of the exact value.
                 const double dn = pk.two_r - r;
-                if ( xa > 0.0 && xa < 1e300 && fabs( dte ) > 1e-290 && fabs( dte ) < 1e290 &&
-                     fabs( dn - dte ) > 1e-3 * fabs( dte ) )
+                double xa, dte;
+                if ( tearEstimate( pk.Rs, dn, xa, dte ) )
                     pk.delta_tear = dn >= dte ? -INFINITY : INFINITY;
                 else
                 {
@@ -267,7 +318,7 @@ __global__ __launch_bounds__( kBlock ) void kContact( const PDArgs* __restrict__
             }
             else
                 pk.coeff_h_n = 4.0 / 3.0 * A.Es * sqrt( pk.Rs );
-            const double mi = rho_i * vol_i, mj = A.rho[j] * A.vol[j];
+            const double mj = uj.w;
             pk.ms = mi * mj / ( mi + mj );
         }
         const double fn = normalForce<JKR>( A, pk, r, vn, vol_i );
@@ -294,7 +345,69 @@ __global__ __launch_bounds__( kBlock ) void kContact( const PDArgs* __restrict__
         fx += ftx;
         fy += fty;
         fz += ftz;
+    };
+    if constexpr ( JKR )
+    {
+        // Beyond contact a pair reaches as far as its tear distance, at most
+        // that of R* = R_i (it grows with R*, and R* = R_i R_j / (R_i + R_j) <
+        // R_i); with a margin over every rounding of the distances.
+        double reach = -pk.delta_tear;
+        if constexpr ( POLY )
+        {
+            const double a0e = cbrtEstimate( 9.0 / 2.0 * A.Gamma * kPi / A.Es * crSq( Ri ) );
+            reach = 1.0 / 2.0 * A.jkr_c6 * crSq( a0e ) / Ri;
+        }
+        reach = fabs( reach ) * 1.01 + 0x1p-30 * ( POLY ? Ri : pk.two_r );
+        // the ids of the marked pairs, kNear a lane
+        constexpr int kNear = 16;
+        __shared__ int32_t near[kNear][kBlock];
+        int32_t q = 0;
+        while ( q < mycnt )
+        {
+            int marked = 0;
+            while ( q < mycnt && marked <= kNear - 4 )
+            {
+                // four slots at a time: their loads in flight together
+                int32_t j[4];
+                double4 xj[4], uj[4];
+                const int c = mycnt - q < 4 ? mycnt - q : 4;
+#pragma unroll
+                for ( int k = 0; k < 4; k++ )
+                    j[k] = colp[( q + ( k < c ? k : 0 ) ) * kSlice];
+#pragma unroll
+                for ( int k = 0; k < 4; k++ )
+                {
+                    xj[k] = rec_x[j[k]];
+                    uj[k] = rec_u[j[k]];
+                }
+#pragma unroll
+                for ( int k = 0; k < 4; k++ )
+                {
+                    const double rx = ( xj[k].x - xi.x ) + ( uj[k].x - ui.x );
+                    const double ry = ( xj[k].y - xi.y ) + ( uj[k].y - ui.y );
+                    const double rz = ( xj[k].z - xi.z ) + ( uj[k].z - ui.z );
+                    const double r2 = rx * rx + ry * ry + rz * rz;
+                    // (comparisons that are false for NaN keep the pair)
+                    const double far = ( POLY ? Ri + xj[k].w : pk.two_r ) + reach;
+                    const bool skip = r2 > far * far && r2 < 1e300;
+                    if ( k < c && !skip )
+                        near[marked++][threadIdx.x] = j[k];
+                }
+                q += c;
+            }
+            for ( int m = 0; m < marked; m++ )
+            {
+                const int32_t j = near[m][threadIdx.x];
+                pairForce( rec_x[j], rec_u[j], rec_v[j] );
+            }
+        }
     }
+    else
+        for ( int32_t q = 0; q < mycnt; q++ )
+        {
+            const int32_t j = colp[q * kSlice];
+            pairForce( rec_x[j], rec_u[j], rec_v[j] );
+        }
     if ( epi != kEpiStoreOnly )
     {
         if ( A.body )
@@ -315,25 +428,19 @@ __global__ __launch_bounds__( kBlock ) void kContact( const PDArgs* __restrict__
             }
         }
     }
+    // (the velocities are left alone: other waves of this launch read those of
+    // their neighbours)
     A.f[p] = fx;
     A.f[n + p] = fy;
     A.f[2 * n + p] = fz;
-    if ( epi != kEpiFinal )
-        return;
-    // final half step (CabanaPD_Integrate.hpp:128-134); only when the pair
-    // force does not read velocities, since other waves of this launch read
-    // v of their neighbors
-    
-    const double half_dt_m = A.half_dt / rho_i;
-    A.v[p] = vi0 + half_dt_m * fx;
-    A.v[n + p] = vi1 + half_dt_m * fy;
-    A.v[2 * n + p] = vi2 + half_dt_m * fz;
 }
 
-// VelocityVerlet<Contact>::initialHalfStep (CabanaPD_Integrate.hpp:154-193):
-// the half kick, the drift into the other displacement buffer, and the block
-// maxima of |u - u_build|.
-__global__ __launch_bounds__( 256 ) void kContactInitial( const PDArgs* __restrict__ specs, int32_t parity,
+// VelocityVerlet<Contact>::initialHalfStep (CabanaPD_Integrate.hpp:154-193),
+// with FINAL preceded by the final half step of the step before (:128-134):
+// the half kicks, the drift into the other displacement buffer, the pair
+// records and the block maxima of |u - u_build|.
+template <bool FINAL>
+__global__ __launch_bounds__( 256 ) void kContactAdvance( const PDArgs* __restrict__ specs, int32_t parity,
                                                           double* __restrict__ partial )
 {
 #pragma clang fp contract( off )
@@ -347,17 +454,23 @@ __global__ __launch_bounds__( 256 ) void kContactInitial( const PDArgs* __restri
         const double half_dt_m = A.half_dt / A.rho[p];
         const double* u = A.U[parity];
         double* un = A.U[parity ^ 1];
-        double dd[3];
+        double dd[3], uu[3], vv[3];
+#pragma unroll
         for ( int d = 0; d < 3; d++ )
         {
-            double vv = A.v[d * n + p];
-            vv = vv + half_dt_m * A.f[d * n + p];
-            A.v[d * n + p] = vv;
-            const double nu = u[d * n + p] + A.dt * vv;
-            un[d * n + p] = nu;
-            dd[d] = nu - A.u_neigh[d * n + p];
+            const double f = A.f[d * n + p];
+            vv[d] = A.v[d * n + p];
+            if constexpr ( FINAL )
+                vv[d] = vv[d] + half_dt_m * f;
+            vv[d] = vv[d] + half_dt_m * f;
+            A.v[d * n + p] = vv[d];
+            uu[d] = u[d * n + p] + A.dt * vv[d];
+            un[d * n + p] = uu[d];
+            dd[d] = uu[d] - A.u_neigh[d * n + p];
         }
         mx = sqrt( dd[0] * dd[0] + dd[1] * dd[1] + dd[2] * dd[2] );
+        A.rec_u[p] = make_double4( uu[0], uu[1], uu[2], A.rho[p] * A.vol[p] );
+        A.rec_v[p] = make_double4( vv[0], vv[1], vv[2], 0.0 );
     }
     red[threadIdx.x] = mx;
     __syncthreads();
@@ -369,6 +482,28 @@ __global__ __launch_bounds__( 256 ) void kContactInitial( const PDArgs* __restri
     }
     if ( threadIdx.x == 0 )
         partial[blockIdx.x] = red[0];
+}
+
+// Maximum of the per-block maxima, written to pinned host memory (one block;
+// a launch of its own: finishing in the last block of kContactAdvance needs a
+// device-wide release per block, which took that pass from 14 to 88 us).
+__global__ __launch_bounds__( 1024 ) void kMaxReduce( const double* __restrict__ partial, int64_t nb,
+                                                      double* __restrict__ out )
+{
+    __shared__ double red[1024];
+    double mx = 0.0;
+    for ( int64_t b = threadIdx.x; b < nb; b += 1024 )
+        mx = fmax( mx, partial[b] );
+    red[threadIdx.x] = mx;
+    __syncthreads();
+    for ( int w = 512; w > 0; w >>= 1 )
+    {
+        if ( (int)threadIdx.x < w )
+            red[threadIdx.x] = fmax( red[threadIdx.x], red[threadIdx.x + w] );
+        __syncthreads();
+    }
+    if ( threadIdx.x == 0 )
+        *out = red[0];
 }
 
 // VelocityVerlet::finalHalfStep (CabanaPD_Integrate.hpp:128-134) as its own
@@ -386,27 +521,7 @@ __global__ __launch_bounds__( 256 ) void kContactFinal( const PDArgs* __restrict
         A.v[d * n + p] = A.v[d * n + p] + half_dt_m * A.f[d * n + p];
 }
 
-// Maximum of the per-block maxima, written to out (one block).
-__global__ __launch_bounds__( 256 ) void kMaxReduce( const double* __restrict__ partial, int64_t nb,
-                                                     double* __restrict__ out )
-{
-    __shared__ double red[256];
-    double mx = 0.0;
-    for ( int64_t b = threadIdx.x; b < nb; b += 256 )
-        mx = fmax( mx, partial[b] );
-    red[threadIdx.x] = mx;
-    __syncthreads();
-    for ( int w = 128; w > 0; w >>= 1 )
-    {
-        if ( (int)threadIdx.x < w )
-            red[threadIdx.x] = fmax( red[threadIdx.x], red[threadIdx.x + w] );
-        __syncthreads();
-    }
-    if ( threadIdx.x == 0 )
-        *out = red[0];
-}
-
-using ContactFn = void ( * )( const PDArgs*, int32_t, int32_t );
+using ContactFn = void ( * )( const PDArgs*, int32_t );
 ContactFn pickContact( const PDArgs& a )
 {
     const bool jkr = a.model == PDK_MODEL_HERTZ_JKR;
@@ -425,25 +540,22 @@ const char* contactKernelName( const PDArgs& a )
     return jkr ? "kContact<false, true>" : "kContact<false, false>";
 }
 
-// Whether the pair force reads the velocities: the damping term (restitution
-// below 1) and, for Hertz-JKR, the approach/recede switch and the friction
-// (force_models/CabanaPD_Hertzian.hpp:74-80, CabanaPD_HertzianJKR.hpp:96-129).
-// Undamped Hertz reads them only through a zero term.
-bool contactReadsVelocity( const PDArgs& a )
+// The pair records of the current state.
+void launchContactPack( const PDArgs* args_dev, const PDArgs& a, int32_t parity, hipStream_t st )
 {
-    return a.model == PDK_MODEL_HERTZ_JKR || a.coeff_h_d != 0.0;
+    if ( a.n == 0 )
+        return;
+    hipLaunchKernelGGL( kContactPack, dim3( static_cast<unsigned>( ( a.n + 255 ) / 256 ) ), dim3( 256 ), 0, st,
+                        args_dev, parity );
+    PDK_HIP( hipGetLastError() );
 }
 
-void launchContactForce( const PDArgs* args_dev, const PDArgs& a, int32_t epilogue_mode, int32_t parity,
-                         hipStream_t st )
+void launchContactForce( const PDArgs* args_dev, const PDArgs& a, int32_t epilogue_mode, hipStream_t st )
 {
     if ( a.nslices == 0 )
         return;
-    // a velocity-dependent pass must not update v while other waves read it
-    if ( epilogue_mode == kEpiFinal && contactReadsVelocity( a ) )
-        throw Error( "internal: velocity-dependent contact needs the split final half step" );
     const unsigned g = static_cast<unsigned>( ( a.nslices + kSlicesPerBlock - 1 ) / kSlicesPerBlock );
-    hipLaunchKernelGGL( pickContact( a ), dim3( g ), dim3( kBlock ), 0, st, args_dev, epilogue_mode, parity );
+    hipLaunchKernelGGL( pickContact( a ), dim3( g ), dim3( kBlock ), 0, st, args_dev, epilogue_mode );
     PDK_HIP( hipGetLastError() );
 }
 
@@ -453,14 +565,6 @@ void launchContactFinal( const PDArgs* args_dev, const PDArgs& a, hipStream_t st
         return;
     hipLaunchKernelGGL( kContactFinal, dim3( static_cast<unsigned>( ( a.n + 255 ) / 256 ) ), dim3( 256 ), 0, st,
                         args_dev );
-    PDK_HIP( hipGetLastError() );
-}
-
-void launchContactInitialHalfStep( const PDArgs* args_dev, const PDArgs& a, int32_t parity, double* partial_dev,
-                                   int64_t nblocks, hipStream_t st )
-{
-    hipLaunchKernelGGL( kContactInitial, dim3( static_cast<unsigned>( nblocks ) ), dim3( 256 ), 0, st, args_dev,
-                        parity, partial_dev );
     PDK_HIP( hipGetLastError() );
 }
 
@@ -478,7 +582,10 @@ void contactForceStore( pdk_spec_s* s )
     if ( *cs.max_disp > cs.extend )
         specTimed( s, 3, [&] { contactBuildImpl( s, false, cs.max_disp, cs.since_build ); } );
     v = view( s );
-    specTimed( s, 0, [&] { launchContactForce( v.dargs, *v.h, kEpiStoreOnly, *v.cur, v.st ); } );
+    specTimed( s, 0, [&] {
+        launchContactPack( v.dargs, *v.h, *v.cur, v.st );
+        launchContactForce( v.dargs, *v.h, kEpiStoreOnly, v.st );
+    } );
 }
 
 void contactStep( pdk_spec_s* s, int32_t nsteps )
@@ -488,30 +595,32 @@ void contactStep( pdk_spec_s* s, int32_t nsteps )
     {
         SpecView v = view( s );
         const int64_t nb = ( v.n + 255 ) / 256;
-        if ( cs.partial->bytes() < static_cast<size_t>( nb + 1 ) * sizeof( double ) )
-            cs.partial->alloc( ( nb + 1 ) * sizeof( double ), cs.acct );
+        if ( cs.partial->bytes() < static_cast<size_t>( nb ) * sizeof( double ) )
+            cs.partial->alloc( nb * sizeof( double ), cs.acct );
         double* part = cs.partial->as<double>();
         specTimed( s, 4, [&] {
-            launchContactInitialHalfStep( v.dargs, *v.h, *v.cur, part, nb, v.st );
-            hipLaunchKernelGGL( kMaxReduce, dim3( 1 ), dim3( 256 ), 0, v.st, part, nb, part + nb );
+            const dim3 g( static_cast<unsigned>( nb ) );
+            // the final half step of the step before rides along
+            hipLaunchKernelGGL( k == 0 ? kContactAdvance<false> : kContactAdvance<true>, g, dim3( 256 ), 0, v.st,
+                                v.dargs, *v.cur, part );
+            hipLaunchKernelGGL( kMaxReduce, dim3( 1 ), dim3( 1024 ), 0, v.st, part, nb, cs.disp_dev );
             PDK_HIP( hipGetLastError() );
         } );
         *v.cur ^= 1;
         // The host decides on a rebuild (CabanaPD_Neighbor.hpp:116-119) from
-        // the largest displacement, copied to pinned memory.  Unless the
-        // periodic rebuild is due, the force pass (which writes f only; the
-        // final half step is its own pass) is launched with the current list
-        // before the host waits for that copy, so the GPU is not left idle
-        // meanwhile; if the displacement calls for a rebuild, the list is
-        // rebuilt and the force pass runs again over the new list, which
-        // overwrites f.  The results are those of deciding first.
-        PDK_HIP( hipMemcpyAsync( cs.disp_pinned, part + nb, sizeof( double ), hipMemcpyDeviceToHost, v.st ) );
+        // the largest displacement, which the pass wrote to pinned memory.
+        // Unless the periodic rebuild is due, the force pass (which writes f
+        // only) is launched with the current list before the host waits for
+        // that value, so the GPU is not left idle meanwhile; if the
+        // displacement calls for a rebuild, the list is rebuilt and the force
+        // pass runs again over the new list, which overwrites f.  The results
+        // are those of deciding first.
         PDK_HIP( hipEventRecord( cs.disp_ready, v.st ) );
         *cs.since_build += 1;
         const bool periodic = cs.rebuild_every > 0 && *cs.since_build >= cs.rebuild_every;
         auto force = [&] {
             v = view( s );
-            specTimed( s, 0, [&] { launchContactForce( v.dargs, *v.h, kEpiApplyOnly, *v.cur, v.st ); } );
+            specTimed( s, 0, [&] { launchContactForce( v.dargs, *v.h, kEpiApplyOnly, v.st ); } );
         };
         if ( !periodic )
             force();
@@ -523,8 +632,9 @@ void contactStep( pdk_spec_s* s, int32_t nsteps )
             specTimed( s, 3, [&] { contactBuildImpl( s, false, cs.max_disp, cs.since_build ); } );
             force();
         }
-        specTimed( s, 4, [&] { launchContactFinal( v.dargs, *v.h, v.st ); } );
     }
+    SpecView v = view( s );
+    specTimed( s, 4, [&] { launchContactFinal( v.dargs, *v.h, v.st ); } );
 }
 
 } // namespace pdk

@@ -283,10 +283,7 @@ const char* lpsKernelName( const PDArgs& a );
 const char* energyKernelName( const PDArgs& a );
 
 // ---- contact (pdk_contact.hip) -----------------------------------------------
-void launchContactForce( const PDArgs* args_dev, const PDArgs& a, int32_t epilogue, int32_t parity,
-                         hipStream_t st );
-void launchContactInitialHalfStep( const PDArgs* args_dev, const PDArgs& a, int32_t parity,
-                                   double* partial_dev, int64_t nblocks, hipStream_t st );
+void launchContactForce( const PDArgs* args_dev, const PDArgs& a, int32_t epilogue_mode, hipStream_t st );
 const char* contactKernelName( const PDArgs& a );
 
 // ---- region outputs (pdk_output.hip) ----------------------------------------

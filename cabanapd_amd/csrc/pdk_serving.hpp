@@ -39,7 +39,8 @@ struct ContactState
     int32_t rebuild_every;
     DevBuf* partial;
     MemAccount* acct;
-    double* disp_pinned;   // pinned host copy of the largest displacement
+    double* disp_pinned;   // largest displacement, in pinned host memory
+    double* disp_dev;      // its device address
     hipEvent_t disp_ready; // recorded after that copy
 };
 ContactState contactState( pdk_spec_s* s );

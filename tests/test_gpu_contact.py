@@ -182,3 +182,47 @@ def test_gpu_random_packing_reaches_solid_fraction():
         worst = max(worst, float(ov.max()))
     say(f"  largest pair overlap {worst:.3e} m (negative: a gap)")
     assert worst <= 0.0
+
+
+def pair_of(w):
+    g = engine.Spec(ctx(), w["desc"], w["x"].shape[0])
+    configs.upload(g, w)
+    configs.setup(g, w)
+    o = oracle_spec(w)
+    configs.setup(o, w)
+    return g, o
+
+
+@pytest.mark.parametrize("polydisperse", [False, True])
+@pytest.mark.parametrize("model", ["HERTZ", "HERTZ_JKR"])
+def test_gpu_crowded_contacts_bitwise(model, polydisperse):
+    """Clusters in which a sphere touches far more neighbours than a lane
+    marks at a time (16), beside isolated ones, pairs just in and out of reach
+    and a pair at exactly the contact distance: the oracle's bits."""
+    rng = np.random.default_rng(12)
+    r = 1e-3
+    x = rng.uniform(0.0, 2.6 * r, size=(67, 3))
+    d = 2.0 * r * (1.0 + np.array([-1e-6, -1e-12, 0.0, 1e-12, 1e-9, 1e-6, 2e-6, 3e-6, 1e-4, 0.02, 0.09]))
+    pairs = np.zeros((2 * d.size, 3))
+    pairs[0::2] = np.arange(d.size)[:, None] * np.array([0.0, 5.0 * r, 0.0]) + [20 * r, 0, 0]
+    pairs[1::2] = pairs[0::2] + np.stack([d, 0 * d, 0 * d], axis=1)
+    x = np.concatenate([x, pairs, [[-40 * r, 0, 0]]])
+    n = x.shape[0]
+    rad = np.full(n, r)
+    if polydisperse:
+        rad[:67] *= rng.uniform(0.8, 1.2, size=67)
+    desc = configs.make_desc(model, radius=r, radius_extend=0.1 * r, nu=0.25, E=7e6, restitution=0.5, gamma=0.05,
+                             dt=1e-9, rebuild_every=3, polydisperse=polydisperse)
+    w = configs._base(desc, x, 4.0 / 3.0 * np.pi * rad ** 3, 2600.0, "crowd", r, 8)
+    w["radius"] = rad if polydisperse else None
+    w["v"] = rng.normal(0.0, 0.5, size=(n, 3))
+    g, o = pair_of(w)
+    off = g.bonds()[0]
+    say(f"case: {model} polydisperse={polydisperse}: {n} spheres, longest row {np.diff(off).max()}")
+    assert np.diff(off).max() > 40
+    assert np.array_equal(g.get("f"), o.get("f"))
+    g.step(8)
+    o.step(8)
+    for fld in ("u", "v", "f"):
+        assert np.array_equal(g.get(fld), o.get(fld)), fld
+    g.close()
