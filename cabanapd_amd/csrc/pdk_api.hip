@@ -13,6 +13,7 @@
 
 #include "pdk_internal.hpp"
 #include "pdk_serving.hpp"
+#include "pdk_transfer.hpp"
 
 using namespace pdk;
 
@@ -183,6 +184,7 @@ struct pdk_ctx_s
     int device = 0;
     MemAccount acct;
     std::unique_ptr<BatchEngine> batch;
+    std::unique_ptr<HostTransfer> transfer;
     std::atomic<int64_t> live_specs{ 0 };
 };
 
@@ -818,6 +820,7 @@ int pdk_ctx_create( int device, uint64_t hbm_budget, pdk_ctx* out )
         PDK_HIP( hipMemGetInfo( &freeb, &total ) );
         c->acct.budget = hbm_budget ? hbm_budget : static_cast<uint64_t>( 0.9 * freeb );
         c->batch = std::make_unique<BatchEngine>( c.get() );
+        c->transfer = std::make_unique<HostTransfer>( device );
         *out = c.release();
     } );
 }
@@ -1933,8 +1936,7 @@ int pdk_download( pdk_spec s, int32_t field, double* out )
             launchScatterScalar( src, s->perm.as<int64_t>(), s->staging.as<double>(), n, s->st );
         else
             launchScatterRows( src, s->perm.as<int64_t>(), s->staging.as<double>(), n, nc, s->st );
-        PDK_HIP( hipMemcpyAsync( out, s->staging.as<double>(), bytes, hipMemcpyDeviceToHost, s->st ) );
-        PDK_HIP( hipStreamSynchronize( s->st ) );
+        s->ctx->transfer->out( out, s->staging.as<double>(), bytes, s->st );
     } );
 }
 
