@@ -1243,17 +1243,28 @@ int pdk_build_bonds( pdk_spec s )
             {
                 s->pushArgs();
                 s->timed( kClsBuild, [&] {
-                    if ( buildStencilSlots( s->h, s->lat_dims, s->lat_h, q.rc, s->h_perm, s->col, s->intact,
-                                            s->slice_ptr.as<int64_t>(), s->total_rows, s->col_rows_cap, s->slot,
-                                            s->scratch, s->acct(), s->st ) )
-                        s->nsten = s->slot.slots;
-                    // missing sites: the forms whose row passes take them
-                    // (equal volumes, no no-fail particles, PMB or LPS)
-                    else if ( s->vol_uniform && !( s->d.fracture && s->any_nofail ) && !isLinearModel( s->d.model ) &&
-                              buildHoleSlots( s->h, s->lat_dims, s->lat_lo, s->lat_h, q.rc, s->h_perm, s->col,
-                                              s->intact, s->slice_ptr.as<int64_t>(), s->total_rows, s->col_rows_cap,
-                                              s->slot, s->scratch, s->acct(), s->st ) )
-                        s->nsten = s->slot.slots;
+                    try
+                    {
+                        // full lattices; else missing sites, for the forms whose row
+                        // passes take them (equal volumes, no no-fail particles, PMB
+                        // or LPS)
+                        const bool holes =
+                            s->vol_uniform && !( s->d.fracture && s->any_nofail ) && !isLinearModel( s->d.model );
+                        if ( buildStencilSlots( s->h, s->lat_dims, s->lat_h, q.rc, s->h_perm, s->col, s->intact,
+                                                s->slice_ptr.as<int64_t>(), s->total_rows, s->col_rows_cap, s->slot,
+                                                s->scratch, s->acct(), s->st ) ||
+                             ( holes && buildHoleSlots( s->h, s->lat_dims, s->lat_lo, s->lat_h, q.rc, s->h_perm,
+                                                        s->col, s->intact, s->slice_ptr.as<int64_t>(), s->total_rows,
+                                                        s->col_rows_cap, s->slot, s->scratch, s->acct(), s->st ) ) )
+                            s->nsten = s->slot.slots;
+                    }
+                    catch ( const MemError& )
+                    {
+                        // no room for both forms at once: the compact one, which is
+                        // complete and untouched until the slot form is, stays
+                        PDK_HIP( hipStreamSynchronize( s->st ) );
+                        s->slot = SlotForm{};
+                    }
                 } );
             }
             // Mixed form on other lattices: one stencil id per bond replaces the x_j gather.

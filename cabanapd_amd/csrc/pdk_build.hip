@@ -1355,10 +1355,6 @@ bool finishSlots( int64_t n, int64_t nslices, const LatticeBox& L, const std::ve
             n, nslices, L, dent, S, ncol.as<int32_t>(), nexist.as<uint64_t>(), nintact.as<uint64_t>() );
         PDK_HIP( hipGetLastError() );
     }
-    std::vector<int64_t> sp( nslices + 1 );
-    for ( int64_t k = 0; k <= nslices; k++ )
-        sp[k] = k * S;
-    PDK_HIP( hipMemcpyAsync( slice_ptr_dev, sp.data(), ( nslices + 1 ) * sizeof( int64_t ), hipMemcpyHostToDevice, st ) );
     std::vector<int32_t> soff( 256, 0 );
     std::vector<float4> tab( 256, make_float4( 0.f, 0.f, 0.f, 1.f ) );
     std::vector<double> tab2( 256, 1.0 );
@@ -1386,6 +1382,11 @@ bool finishSlots( int64_t n, int64_t nslices, const LatticeBox& L, const std::ve
     PDK_HIP( hipMemcpyAsync( dsoff.as<int32_t>(), soff.data(), 256 * sizeof( int32_t ), hipMemcpyHostToDevice, st ) );
     PDK_HIP( hipMemcpyAsync( dtab.as<float4>(), tab.data(), 256 * sizeof( float4 ), hipMemcpyHostToDevice, st ) );
     PDK_HIP( hipMemcpyAsync( dxi2.as<double>(), tab2.data(), 256 * sizeof( double ), hipMemcpyHostToDevice, st ) );
+    // every allocation is done: from here on the compact form is replaced
+    std::vector<int64_t> sp( nslices + 1 );
+    for ( int64_t k = 0; k <= nslices; k++ )
+        sp[k] = k * S;
+    PDK_HIP( hipMemcpyAsync( slice_ptr_dev, sp.data(), ( nslices + 1 ) * sizeof( int64_t ), hipMemcpyHostToDevice, st ) );
     PDK_HIP( hipStreamSynchronize( st ) );
     col = std::move( ncol );
     intact = std::move( nintact );

@@ -21,6 +21,12 @@ struct Error : std::runtime_error
     using std::runtime_error::runtime_error;
 };
 
+// Device memory that the budget or the device does not have.
+struct MemError : Error
+{
+    using Error::Error;
+};
+
 #define PDK_HIP( call )                                                                        \
     do                                                                                         \
     {                                                                                          \
@@ -43,7 +49,7 @@ struct MemAccount
     {
         std::lock_guard<std::mutex> g( mu );
         if ( budget && in_use + bytes > budget )
-            throw Error( "HBM budget exceeded: need " + std::to_string( bytes ) + " B more, " +
+            throw MemError( "HBM budget exceeded: need " + std::to_string( bytes ) + " B more, " +
                          std::to_string( budget - in_use ) + " B left" );
         in_use += bytes;
     }
@@ -88,6 +94,11 @@ class DevBuf
             ptr_ = nullptr;
             if ( acct )
                 acct->unreserve( bytes );
+            if ( e == hipErrorOutOfMemory )
+            {
+                (void)hipGetLastError();
+                throw MemError( "hipMalloc failed: out of memory" );
+            }
             PDK_HIP( e );
         }
         bytes_ = bytes;

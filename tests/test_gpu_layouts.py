@@ -195,3 +195,43 @@ def test_missing_sites_in_the_batch(precision):
         for f, r in zip(("u", "v", "f"), ref):
             assert np.array_equal(s.get(f), r, equal_nan=True)
         s.close()
+
+
+@pytest.mark.parametrize("shape", ["hole", "whole horizon"])
+def test_tight_budgets_keep_the_compact_form(shape):
+    """Where the HBM budget holds the compact form but not both forms at
+    once, the build keeps the compact one instead of failing."""
+    if shape == "hole":
+        dims, keep = SHAPES["hole"]
+        w = cut(box("PMB", dims, 3.01, True), dims, keep)
+    else:
+        w = box("PMB", (40, 31, 6), 3, True)
+    n = w["x"].shape[0]
+
+    def build(budget, layout):
+        d = type(w["desc"]).from_buffer_copy(w["desc"])
+        d.bond_layout = layout
+        with engine.Context(0, budget) as c:
+            s = None
+            try:
+                s = engine.Spec(c, d, n)
+                configs.upload(s, w)
+                configs.setup(s, w)
+                s.step(3)
+                return s.get("u"), s.kernel_name(0)
+            except engine.PdkError:
+                return None
+            finally:
+                if s is not None:
+                    s.close()
+
+    seen = set()
+    for budget in np.geomspace(4e6, 4e7, 40).astype(int):
+        compact, auto = build(int(budget), PDK_BONDS_COMPACT), build(int(budget), 0)
+        if compact is None:
+            continue
+        assert auto is not None, f"budget {budget}"
+        assert np.array_equal(auto[0], compact[0])
+        seen.add("Rows" in auto[1])
+    say(f"case: {shape}: row windows chosen over the budgets: {sorted(seen)}")
+    assert seen == {False, True}
