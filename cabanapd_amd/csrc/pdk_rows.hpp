@@ -1952,6 +1952,98 @@ __global__ __launch_bounds__( W == 1 ? kBlock : W * kSlice ) __attribute__( ( am
             }
             return __ballot( gen );
         };
+        // slotFast over NG slots at once, every lane evaluating (as kForceRows'
+        // group): NG independent chains overlap in a split launch, which has
+        // few waves per SIMD
+        auto groupFast = [&]( auto ng, const int t0, const double lim ) __attribute__( ( always_inline ) ) {
+            constexpr int NG = decltype( ng )::value;
+            uint64_t ww[NG], brkm[NG], bad = 0;
+            const double* wr[NG];
+            double spv[NG];
+            Fast64 b[NG];
+            double temp_avg[NG];
+            bool gen[NG];
+#pragma unroll
+            for ( int g = 0; g < NG; g++ )
+            {
+                ww[g] = scalarLoad( mwords + R.x + t0 + g );
+                brkm[g] = 0;
+                wr[g] = window( t0 + g );
+                moveOn( t0 + g );
+                spv[g] = 0.0;
+                if constexpr ( EP )
+                    spv[g] = spl[( R.x + t0 + g ) * kSlice];
+            }
+#pragma unroll
+            for ( int g = 0; g < NG; g++ )
+            {
+                getDistanceFast( xi0, xi1, xi2, ui0, ui1, ui2, wr[g][3 * kW], wr[g][4 * kW], wr[g][5 * kW], wr[g][0],
+                                 wr[g][kW], wr[g][2 * kW], b[g] );
+                temp_avg[g] = 0.0;
+                if constexpr ( TH )
+                {
+                    temp_avg[g] = thermalAvg( A, Ti, wr[g][KH * kW] );
+                    b[g].s = b[g].s - ( A.alpha * temp_avg[g] );
+                }
+                gen[g] =
+                    !( fabs( b[g].s ) <= 0x1p600 ) || max( lowWord( b[g].r ), lowWord( b[g].xi ) ) == 0xffffffffu;
+            }
+#pragma unroll
+            for ( int g = 0; g < NG; g++ )
+            {
+                int mj = 0;
+                bool nf_j = nf_i;
+                if constexpr ( TAG )
+                {
+                    const int tag = static_cast<int>( wr[g][KT * kW] );
+                    mj = tag >> 1;
+                    if constexpr ( !kIsLps<MODEL> )
+                        nf_j = ( tag & 1 ) != 0;
+                }
+                if constexpr ( FRAC )
+                {
+                    const double bcc_ij = TH ? thermalBcc( A, temp_avg[g] ) : ( MT ? tab_bcc[ti4 + mj] : bcc );
+                    brkm[g] = __ballot( !gen[g] && criticalStretch64( b[g].r, b[g].xi, bcc_ij ) && !nf_i && !nf_j ) &
+                              ww[g];
+                }
+                const bool live = __builtin_amdgcn_inverse_ballot_w64( ww[g] & ~brkm[g] );
+                const double vj = wr[g][KV * kW];
+                double coeff;
+                if constexpr ( !kIsLps<MODEL> )
+                {
+                    double sd = b[g].s;
+                    if constexpr ( EP )
+                    {
+                        if ( live && !gen[g] )
+                            sd = plasticStretchAt( spl + ( R.x + t0 + g ) * kSlice, spv[g], b[g].s, A.sY );
+                    }
+                    coeff = ( MT ? tab_c[ti4 + mj] : c ) * sd * vj;
+                }
+                else
+                {
+                    const double infl = infl1 ? 1.0 / b[g].xi : 1.0;
+                    coeff = ( Ai + wr[g][( 3 + NX ) * kW] + b[g].s * ( Bi + wr[g][( 4 + NX ) * kW] ) ) * infl * b[g].xi *
+                            vj;
+                }
+                // (a bond that breaks needs no coefficient)
+                bad |= __ballot( gen[g] || ( live && !( fabs( coeff ) <= lim ) ) ) & ww[g];
+                const double cx = divBy( coeff * b[g].rx, b[g].r, b[g].yr );
+                const double cy = divBy( coeff * b[g].ry, b[g].r, b[g].yr );
+                const double cz = divBy( coeff * b[g].rz, b[g].r, b[g].yr );
+                put( t0 + g, live ? cx : -0.0, live ? cy : -0.0, live ? cz : -0.0 );
+            }
+            if constexpr ( FRAC )
+            {
+#pragma unroll
+                for ( int g = 0; g < NG; g++ )
+                    if ( __builtin_expect( brkm[g] != 0, 0 ) )
+                    {
+                        if ( lane == 0 )
+                            bits[R.x + t0 + g] = ww[g] & ~brkm[g];
+                    }
+            }
+            return bad;
+        };
         if constexpr ( PREC == kMixed )
         {
 #pragma unroll
@@ -1965,8 +2057,19 @@ __global__ __launch_bounds__( W == 1 ? kBlock : W * kSlice ) __attribute__( ( am
             {
                 const double fx0 = fx, fy0 = fy, fz0 = fz;
                 uint64_t bad = 0;
-                for ( int t = 0; t < R.y; t++ )
-                    bad |= slotFast( t, limit );
+                if constexpr ( W > 1 )
+                {
+                    int t = 0;
+                    for ( ; t + 5 <= R.y; t += 5 )
+                        bad |= groupFast( std::integral_constant<int, 5>{}, t, limit );
+                    for ( ; t + 3 <= R.y; t += 3 )
+                        bad |= groupFast( std::integral_constant<int, 3>{}, t, limit );
+                    for ( ; t < R.y; t++ )
+                        bad |= groupFast( std::integral_constant<int, 1>{}, t, limit );
+                }
+                else
+                    for ( int t = 0; t < R.y; t++ )
+                        bad |= slotFast( t, limit );
                 if ( __builtin_expect( bad == 0, 1 ) )
                     return;
                 fx = fx0;
