@@ -1801,12 +1801,16 @@ ForceFn pickForceRowsFeat( const PDArgs& a )
 //   slices                  200            512           1077          2197
 //   FP64 PMB fracture   55/ 20/ 15    56/ 25/ 28    71/ 48/ 66    91/ 80/118
 //   FP64 LPS fracture  148/ 54/ 39   150/ 68/ 75   189/128/181   242/210/328
-//   FP64 two materials 168/ 62/ 45   168/ 75/ 85   205/163/205   256/271/371
+//   FP64 two materials 168/ 60/ 44   168/ 73/ 83   204/156/199   256/261/361
+//   FP64 temperature    61/ 26/ 20    61/ 32/ 34    76/ 58/ 77    97/ 94/135
+//   FP64 plastic        95/ 30/ 21   115/ 38/ 42   130/ 71/ 99   148/116/178
 //   mixed PMB fracture  32/ 16/ 12    32/ 18/ 21    33/ 33/ 47    37/ 54/ 82
 //   mixed LPS fracture  81/ 35/ 25    81/ 38/ 38    82/ 63/ 85    95/106/153
 //   mixed plastic       75/ 25/ 17    88/ 32/ 36   102/ 60/ 85   114/ 97/152
 // Eight waves (up to 89 KB of LDS) fit once on a CU, so they serve up to 256
-// slices.
+// slices.  With temperature the line stays below what the cube suggests: 40
+// steps of a heated 49^3 block (1839 slices) took 4.09 ms with one wave per
+// slice, 4.38 with four.
 int splitWaves( const PDArgs& a, int64_t nslices )
 {
     if ( a.row_max > kSplitSlots )
@@ -1814,7 +1818,8 @@ int splitWaves( const PDArgs& a, int64_t nslices )
     if ( nslices <= 256 )
         return 8;
     const bool lps = a.model == kLPS || a.model == kLinLPS;
-    const int64_t four = a.precision == PDK_MIXED ? ( lps || a.splas ? 1536 : 1088 ) : ( rowFeatures( a ) ? 1792 : 2560 );
+    const int64_t four = a.precision == PDK_MIXED ? ( lps || a.splas ? 1536 : 1088 )
+                                                  : ( a.mtype || a.temp ? 1792 : 2560 );
     return nslices <= four ? 4 : 1;
 }
 

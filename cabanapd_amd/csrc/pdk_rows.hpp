@@ -590,8 +590,10 @@ __device__ __forceinline__ double addRound( const SplitTerms<W, ND, NF>& T, int 
 // compact form read 5 bytes of ids a bond and took a wavefront's neighbour
 // data from three to twelve scattered loads: 100 mixed steps of a 423k-particle
 // perforated plate 26.5 -> 11.0 ms, 100 FP64 elastic-plastic steps of a 29k
-// dogbone 14.2 -> 5.3 ms.
-// G: slots evaluated together (1: one after the other).
+// dogbone 14.2 -> 5.3 ms (4.3 with slots together).
+// G: slots evaluated together (1: one after the other).  Five in split launches
+// in FP64.  With one wave per slice five gave 47 -> 41 us on small specimens and
+// nothing from 2000 slices on; the mixed form got slower.
 template <int MODEL, bool FRAC, int PREC, bool GEN, int W = 1, bool HOLE = false, int G = 1>
 __global__ __launch_bounds__( W == 1 ? kBlock : W * kSlice ) __attribute__( ( amdgpu_waves_per_eu( ( MODEL == 1 || MODEL == 5 || G > 1 ) ? 1 : 6, 8 ) ) ) void
 kForceRows( const PDArgs* __restrict__ specs,
