@@ -243,7 +243,7 @@ struct pdk_spec_s
     bool lattice_rows = false; // device order is lattice rows (else Morton)
     int32_t unroll = -1;       // force-pass variant (tuning knob): -1 default, 0 row windows, 1/2/4/8 gathers
     bool coords_plain = false; // every coordinate is zero or within [2^-100, 2^100)
-    bool vols_plain = false;   // every volume is within [2^-150, 2^150)
+    double vol_min = 0.0, vol_max = 0.0;
     bool vol_uniform = false;  // every particle has volume vol_value
     double vol_value = 0.0;
     bool any_nofail = false;
@@ -351,31 +351,79 @@ struct pdk_spec_s
         return step_graph[c];
     }
 
-    // Whether the FP64 row passes may take the shared-reciprocal arithmetic
-    // (rootRecip, divBy): with lattice vectors within [2^-60, 2^60], volumes,
-    // c V and the LPS coefficients as tested here, u, x and T zero or within
-    // [2^-100, 2^100) and lpsA, lpsB zero or within [2^-200, 2^200), a bond's
-    // nonzero terms satisfy |s| >= 2^-54 (2^-266 with a thermal strain),
-    // |r_k| >= 2^-205, coeff >= 2^-570, so every quotient and remainder is
-    // above 2^-930 and, with |coeff| <= 2^600, below 2^930.
-    bool plainRange() const
+    // The FP64 row passes may take the shared-reciprocal arithmetic (rootRecip,
+    // divBy) where every quotient and every remainder of a bond stays above
+    // 2^-960 (1074 less the 106 bits that a remainder's last bit lies below
+    // its dividend), or is zero.  Returned is the largest L up to 400 for which
+    // u, x and T that are zero or at least 2^-L in magnitude see to that with
+    // this specimen's constants; 0 where the lattice or the constants are outside
+    // the ranges tested here.  400: squares of displacement differences, at least 2^-(L + 54)
+    // each, then stay above 2^-960 too.  A bond's nonzero terms, as powers of two:
+    //   r_k    >= -(L + 54)      (the last bit of a staged value)
+    //   s      >= -55            ((r - xi) / xi of two doubles)
+    //          >= min(-108, alpha - L - 56, alpha + temp0 - 54) with a thermal strain
+    //   s - sp >= min(-108, s - 53, sY - 54) with a plastic stretch
+    //   coeff  >= c + V + s - 2, LPS: V - 364 (lpsA, lpsB zero or >= -200,
+    //             their sum with s times the other cancels to its last bit) + xi, + infl
+    // and the quotient by r < 2^102 is smaller than coeff r_k by that much.
+    // (Lattices that start at rest hold values down to about 2^-340 ahead of a
+    // front.  With 2^-100 for L, the limit for the largest ranges allowed here, up to a
+    // third of the rows that carry force were evaluated twice: 27 % on a struck
+    // 180k plate at 60 steps, 35 % on the 79k regression plate at 100.)
+    int plainLow() const
     {
         auto within = []( double a, double lo, double hi ) { return std::fabs( a ) >= lo && std::fabs( a ) < hi; };
         auto zeroOr = [&]( double a, double lo, double hi ) { return a == 0.0 || within( a, lo, hi ); };
-        if ( !coords_plain || !vols_plain || slot.slots <= 0 )
-            return false;
+        if ( !coords_plain || !( vol_min >= 0x1p-150 && vol_max < 0x1p150 ) || slot.slots <= 0 )
+            return 0;
+        double h_min = d.horizon;
         for ( int dd = 0; dd < 3; dd++ )
-            if ( !within( lat_h[dd], 0x1p-60, 0x1p60 ) && lat_dims[dd] > 1 )
-                return false;
+            if ( lat_dims[dd] > 1 )
+            {
+                if ( !within( lat_h[dd], 0x1p-60, 0x1p60 ) )
+                    return 0;
+                h_min = std::min( h_min, lat_h[dd] );
+            }
         if ( !within( d.horizon, 0x1p-60, 0x1p60 ) )
-            return false;
+            return 0;
         bool ok = lps() || within( k.c, 0x1p-150, 0x1p150 );
         ok = ok && zeroOr( k.theta_coeff, 0x1p-150, 0x1p150 ) && zeroOr( k.s_coeff, 0x1p-150, 0x1p150 );
         ok = ok && zeroOr( d.alpha, 0x1p-60, 0x1p60 ) && zeroOr( d.temp0, 0x1p-100, 0x1p100 );
         ok = ok && zeroOr( k.thermal_coeff, 0x1p-150, 0x1p150 );
+        const bool plastic = d.mechanics == PDK_MECH_EPP;
+        ok = ok && ( !plastic || zeroOr( k.s_Y, 0x1p-150, 0x1p150 ) );
+        double c_min = lps() ? 1.0 : std::fabs( k.c );
         for ( int t = 0; pair_tables && t < 16; t++ )
+        {
             ok = ok && zeroOr( mat_c[t], 0x1p-150, 0x1p150 );
-        return ok;
+            if ( !lps() && mat_c[t] != 0.0 )
+                c_min = std::min( c_min, std::fabs( mat_c[t] ) );
+        }
+        if ( !ok )
+            return 0;
+        const int ev = std::ilogb( vol_min ), eh = std::min( std::ilogb( h_min ), 0 );
+        const bool thermal = d.thermal != PDK_TEMP_INDEPENDENT && d.alpha != 0.0;
+        int low = 400;
+        for ( ; low > 0; low-- )
+        {
+            int es = -55;
+            if ( thermal )
+            {
+                es = std::min( -108, std::ilogb( d.alpha ) - low - 56 );
+                if ( d.temp0 != 0.0 )
+                    es = std::min( es, std::ilogb( d.alpha ) + std::ilogb( d.temp0 ) - 54 );
+            }
+            if ( plastic )
+            {
+                es = std::min( -108, es - 53 );
+                if ( k.s_Y != 0.0 )
+                    es = std::min( es, std::ilogb( k.s_Y ) - 54 );
+            }
+            const int ecoeff = lps() ? ev - 364 + 2 * eh : std::ilogb( c_min ) + ev + es - 2;
+            if ( ecoeff - ( low + 54 ) - 102 >= -960 )
+                break;
+        }
+        return low;
     }
 
     void pushArgs()
@@ -390,7 +438,7 @@ struct pdk_spec_s
         h.f = f.as<double>();
         h.vol = vol.as<double>();
         h.rho = rho.as<double>();
-        h.plain_range = plainRange() ? 1 : 0;
+        h.plain_low = plainLow();
         h.nofail = nofail.as<uint8_t>();
         h.bcflag = bcflag.as<uint8_t>();
         h.body = body ? body.as<double>() : nullptr;
@@ -1013,7 +1061,7 @@ int pdk_spec_upload( pdk_spec s, const double* x, const double* u, const double*
         // particle spacing (cube root of the mean volume).
         double lo[3] = { x[0], x[1], x[2] };
         double vsum = 0.0;
-        // magnitudes, for the FP64 row passes' arithmetic (plainRange)
+        // magnitudes, for the FP64 row passes' arithmetic (plainLow)
         double cmin = 1.0, cmax = 1.0, vmin = vol[0], vmax = vol[0];
         for ( int64_t i = 0; i < n; i++ )
         {
@@ -1030,7 +1078,8 @@ int pdk_spec_upload( pdk_spec s, const double* x, const double* u, const double*
             vmax = std::max( vmax, vol[i] );
         }
         s->coords_plain = cmin >= 0x1p-100 && cmax < 0x1p100;
-        s->vols_plain = vmin >= 0x1p-150 && vmax < 0x1p150;
+        s->vol_min = vmin;
+        s->vol_max = vmax;
         double h = std::cbrt( vsum / n );
         if ( !( h > 0 ) || !std::isfinite( h ) )
             h = 1.0;

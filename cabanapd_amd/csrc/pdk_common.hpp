@@ -147,10 +147,11 @@ struct PDArgs
     const int4* hole_win;
     const uint8_t* hole_pos;
     int32_t row_max;        // longest row of the row table, in slots
-    // FP64 row passes: positions, volumes and constants are within the ranges
-    // for which the shared-reciprocal bond arithmetic gives the general
-    // code's bits (the rows test displacements themselves)
-    int32_t plain_range;
+    // FP64 row passes: 0, or the L for which the shared-reciprocal bond
+    // arithmetic gives the general code's bits where u and T are zero or at
+    // least 2^-L (the rows test that) with this specimen's positions, volumes
+    // and constants
+    int32_t plain_low;
     // Multi-material specimens (FP64 gather passes): material of each
     // particle (null: one material), the PMB coefficient and the critical
     // stretch coefficient of each material pair [4 a + b], and each

@@ -1129,7 +1129,7 @@ __global__ __launch_bounds__( kBlock ) void kEnergyRows( const PDArgs* __restric
         };
         // (no division by |r|: any displacement goes through the shared
         // reciprocal of |xi|, except where the stretch is not a number)
-        const bool plain = !kIsLin<MODEL> && scalarLoad( &A.plain_range ) != 0;
+        const bool plain = !kIsLin<MODEL> && scalarLoad( &A.plain_low ) != 0;
         rw.walk(
             &win[wv][0][0][0], plain, []( const double*, const double* ) { return false; }, S,
             [&]( int32_t q, const double* __restrict__ wr, int32_t g ) {
@@ -1303,7 +1303,8 @@ __global__ __launch_bounds__( kBlock ) void kStressRows( const PDArgs* __restric
         S.s12 += fy * xi_z;
         S.s21 += fz * xi_y;
     };
-    const bool plain = !kIsLin<MODEL> && scalarLoad( &A.plain_range ) != 0;
+    const int plain_low = kIsLin<MODEL> ? 0 : scalarLoad( &A.plain_low );
+    const bool plain = plain_low != 0;
     int own_lo = 0, own_hi = 0, own_la = 0, own_ha = 0;
     expRange( ui0, own_lo, own_hi );
     expRange( ui1, own_lo, own_hi );
@@ -1332,7 +1333,7 @@ __global__ __launch_bounds__( kBlock ) void kStressRows( const PDArgs* __restric
                 expRange( v0[q], la, ha );
                 expRange( v1[q], la, ha );
             }
-            return lo < -kPlainExp || hi > kPlainExp || la < -kPlainExpAB || ha > kPlainExpAB;
+            return lo < -plain_low || hi > kPlainHigh || la < -kPlainExpAB || ha > kPlainExpAB;
         },
         S,
         [&]( int32_t q, const double* __restrict__ wr, int32_t g ) {
@@ -1474,17 +1475,18 @@ __global__ __launch_bounds__( kBlock ) void kHeatConductionRows( const PDArgs* _
     const int lin = A.lin_micro;
     const double volu = A.vol_value;
     double conduction = 0.0;
+    const int plain_low = scalarLoad( &A.plain_low );
     int own_lo = 0, own_hi = 0;
     expRange( Ti, own_lo, own_hi );
     // (intact bonds under fracture, a subset of the existing ones; the linear
     // microconductivity keeps the general code)
     rw.walk(
-        &win[wv][0][0][0], lin == 0 && scalarLoad( &A.plain_range ) != 0,
+        &win[wv][0][0][0], lin == 0 && plain_low != 0,
         [&]( const double* v0, const double* v1 ) {
             int lo = own_lo, hi = own_hi;
             expRange( v0[3], lo, hi );
             expRange( v1[3], lo, hi );
-            return lo < -kPlainExp || hi > kPlainExp;
+            return lo < -plain_low || hi > kPlainHigh;
         },
         conduction,
         [&]( int32_t q, const double* __restrict__ wr, int32_t g ) {

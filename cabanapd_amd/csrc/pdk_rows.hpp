@@ -293,14 +293,14 @@ __device__ __forceinline__ void linearized32g( double xi0, double xi1, double xi
 // the same iterations, so the results are the correctly rounded ones, the
 // same bits.  That holds
 //   - for operands whose intermediate values neither overflow nor lose bits
-//     to underflow: PDArgs::plain_range (lattice, constants) and the rows'
-//     own test of the staged values (kPlainExp) see to that, together with
-//     the coefficient's bound plainLimit;
+//     to underflow: PDArgs::plain_low (lattice, constants) and the rows'
+//     own test of the staged values (rowPlain) see to that, together with
+//     the coefficient's bound of 2^600;
 //   - for roots that are neither zero, infinite nor NaN: those make the
 //     stretch NaN, and with it the coefficient;
 //   - for divisors other than 2^k (2 - 2^-52), the one mantissa whose
-//     reciprocal Newton's iteration misses by an ulp: lastBits finds every
-//     divisor whose low word is all ones.
+//     reciprocal Newton's iteration misses by an ulp: lowWord
+//     finds every divisor whose low word is all ones.
 // A row in which a lane fails one of them is evaluated again by the general
 // code, from the sums as they were before the row.
 // (checked on the GPU against IEEE results: 1e8 roots and quotients, half of
@@ -309,7 +309,7 @@ __device__ __forceinline__ void linearized32g( double xi0, double xi1, double xi
 // 25 steps of the 1.44M-particle plate with their download 28.2 -> 23.6 ms,
 // 50 steps of a 41^3 cube 4.23 -> 3.52 ms, with the LPS model 8.50 -> 7.48.)
 // ---------------------------------------------------------------------------
-constexpr int kPlainExp = 100;   // staged u, x and T: zero or 2^-100 <= |.| < 2^100
+constexpr int kPlainHigh = 100;  // staged u and T: zero or 2^-plain_low <= |.| < 2^100
 constexpr int kPlainExpAB = 200; // staged lpsA, lpsB: zero or 2^-200 <= |.| < 2^200
 
 struct Root64
@@ -767,7 +767,8 @@ kForceRows( const PDArgs* __restrict__ specs,
     };
 
     // FAST: the range test of a row's staged values and of particle i's own
-    const bool plain = FAST && scalarLoad( &A.plain_range ) != 0;
+    const int plain_low = FAST ? scalarLoad( &A.plain_low ) : 0;
+    const bool plain = plain_low != 0;
     int own_lo = 0, own_hi = 0;
     if constexpr ( FAST )
     {
@@ -783,7 +784,7 @@ kForceRows( const PDArgs* __restrict__ specs,
             expRange( v0[q], lo, hi );
             expRange( v1[q], lo, hi );
         }
-        bool out = lo < -kPlainExp || hi > kPlainExp;
+        bool out = lo < -plain_low || hi > kPlainHigh;
         if constexpr ( NAB )
         {
             int la = 0, ha = 0;
@@ -1602,7 +1603,8 @@ __global__ __launch_bounds__( W == 1 ? kBlock : W * kSlice ) __attribute__( ( am
 
     // FP64: rows of ordinary values take the shared reciprocals (see kForceRows)
     constexpr bool FAST = ( PREC == kF64 );
-    const bool plain = FAST && scalarLoad( &A.plain_range ) != 0;
+    const int plain_low = FAST ? scalarLoad( &A.plain_low ) : 0;
+    const bool plain = plain_low != 0;
     int own_lo = 0, own_hi = 0;
     if constexpr ( FAST )
     {
@@ -1624,7 +1626,7 @@ __global__ __launch_bounds__( W == 1 ? kBlock : W * kSlice ) __attribute__( ( am
             expRange( v0[KH], lo, hi );
             expRange( v1[KH], lo, hi );
         }
-        bool out = lo < -kPlainExp || hi > kPlainExp;
+        bool out = lo < -plain_low || hi > kPlainHigh;
         if constexpr ( NAB )
         {
             int la = 0, ha = 0;
@@ -2262,7 +2264,7 @@ __global__ __launch_bounds__( W == 1 ? kBlock : W * kSlice ) void kLpsStateRows(
     // the lanes that need the general code; then the row is evaluated again
     // by bond, from the sum as it was.  Terms of absent bonds are -0.0, which
     // leave every sum as it is.
-    const bool plain = PREC == kF64 && scalarLoad( &A.plain_range ) != 0;
+    const bool plain = PREC == kF64 && scalarLoad( &A.plain_low ) != 0;
     auto walk = [&]( auto&& bond, auto&& fast, double& sum, double& sum2 ) {
         auto evalRow = [&]( const int r ) __attribute__( ( always_inline ) ) {
             const int4 R = scalarLoad4( rows + r );

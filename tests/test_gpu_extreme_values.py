@@ -8,9 +8,9 @@ has NaN)."""
 import numpy as np
 import pytest
 
-from cabanapd_amd import configs
+from cabanapd_amd import configs, engine
 from cabanapd_amd._abi import make_desc
-from tests.parity import pair, say
+from tests.parity import ctx, pair, say
 
 pytestmark = pytest.mark.gpu
 
@@ -78,3 +78,71 @@ def test_extreme_displacements_match_oracle(kind, wild):
         same(g.get(fld), o.get(fld), fld)
     assert np.array_equal(g.bonds()[2], o.bonds()[2])
     g.close()
+
+
+@pytest.mark.parametrize("kind", ["pmb", "pmb_fracture", "lps", "lps_influence1", "lps_fracture", "epp", "epp_tiny",
+                                  "materials", "heat"])
+def test_fading_displacements_match_oracle(kind):
+    """A front's tail: displacements (and temperatures) that fade from 1e-7 of
+    the spacing through both sides of the limit of the fast form (2^-400 = 4e-121
+    at most) to subnormal, one component far smaller than the others; with
+    epp_tiny a yield stretch below the fast form's range."""
+    say(f"case: {kind}, {N}^3 FP64, displacements fading over 300 powers of ten")
+    w = workload("epp" if kind == "epp_tiny" else kind, 5, False)
+    rng = np.random.default_rng(8)
+    n = w["x"].shape[0]
+    fade = 10.0 ** -np.interp(np.arange(n), [0, n // 3, n - 1], [9, 130, 322])
+    scale = rng.choice([1.0, 1e-3, 1e-60, 0.0], size=(n, 3), p=[0.5, 0.2, 0.2, 0.1])
+    w["u"] = rng.uniform(-1, 1, size=(n, 3)) * fade[:, None] * scale
+    w["u"][:, 0] += 1e-6 * H * rng.uniform(-1, 1, size=n)  # every bond along x carries force
+    if kind == "epp_tiny":
+        w["desc"].sigma_y = 1e-290
+    if kind == "heat":
+        w["temperature"] = rng.uniform(-1, 1, size=n) * fade[::-1]
+    g, o = pair(w)
+    for fld in ("f", "W"):
+        same(g.get(fld), o.get(fld), fld + " at init")
+    g.compute_stress()
+    o.compute_stress()
+    same(g.get("stress"), o.get("stress"), "stress")
+    g.step(3)
+    o.step(3)
+    for fld in ("u", "v", "f") + (("m", "theta") if kind.startswith("lps") else ()) + (
+            ("temperature",) if kind == "heat" else ()):
+        same(g.get(fld), o.get(fld), fld)
+    assert np.array_equal(g.bonds()[2], o.bonds()[2])
+    g.close()
+
+
+@pytest.mark.parametrize("model", ["PMB", "LPS"])
+def test_fading_displacements_keep_the_fast_rows(model):
+    """Small values that a front leaves ahead of it (down to 1e-100) in rows
+    that carry force do not send them through the general code: the force pass
+    takes the time that it takes without them (evaluating the rows twice took
+    1.6 times as long)."""
+    h = 5e-4
+    x, vol, _ = configs.grid_cell_centred([0, 0, 0], [64 * h, 64 * h, 64 * h], (64, 64, 64))
+    kw = dict(horizon=3.01 * h, K=4.3e10, dt=1e-9, fracture=True, G0=3.8e3)
+    if model == "LPS":
+        kw.update(G=2.9e10, influence=0)
+    w = configs._base(make_desc(model, **kw), x, vol, 2440.0, "fading", h, 25)
+    n = x.shape[0]
+    rng = np.random.default_rng(2)
+    full = rng.uniform(-1, 1, size=(n, 3)) * 1e-6 * h
+    tails = full.copy()
+    tails[:, 1:] *= 10.0 ** -rng.uniform(40, 90, size=(n, 1))
+    s = engine.Spec(ctx(), w["desc"], n)
+    best = {}
+    for name, u in (("full", full), ("tails", tails)):
+        w["u"] = u
+        configs.upload(s, w)
+        configs.setup(s, w)
+        best[name] = np.inf
+        for _ in range(5):
+            s.timing(True)
+            s.compute_force()
+            best[name] = min(best[name], s.kernel_time(0)[0])
+        s.timing(False)
+    say(f"case: {model}, {n} particles, force pass {best['full']:.4f} ms, with tails {best['tails']:.4f} ms")
+    assert best["tails"] < 1.25 * best["full"]
+    s.close()
