@@ -1871,39 +1871,6 @@ bool rowFeaturesSupported( int32_t model, bool pair_tables, bool thermal, bool p
     return model == kPMB || !( thermal || plastic );
 }
 
-const char* forceKernelName( const PDArgs& a )
-{
-    if ( useRowWindows( a ) && rowFeatures( a ) )
-    {
-        std::snprintf( g_force_name, sizeof( g_force_name ), "kForceRowsF<%d, %s, %d, %d>", a.model,
-                       a.fracture ? "true" : "false", a.precision == PDK_MIXED ? 1 : 0, rowFeatures( a ) );
-        return g_force_name;
-    }
-    if ( useRowWindows( a ) )
-    {
-        std::snprintf( g_force_name, sizeof( g_force_name ), "kForceRows<%d, %s, %d, %s>", a.model,
-                       a.fracture ? "true" : "false", a.precision == PDK_MIXED ? 1 : 0,
-                       rowsGeneral( a ) ? "true" : "false" );
-        return g_force_name;
-    }
-    const bool mm = a.precision == PDK_MIXED && a.mtype != nullptr && ( a.model == kPMB || a.model == kLPS );
-    std::snprintf( g_force_name, sizeof( g_force_name ), "kForce<%d, %s, %d, %d, %s%s>", a.model,
-                   a.fracture ? "true" : "false", a.precision == PDK_MIXED ? 1 : 0, normalizeUnroll( a.unroll ),
-                   a.exist ? "true" : "false", mm ? ", true" : "" );
-    return g_force_name;
-}
-const char* lpsKernelName( const PDArgs& a )
-{
-    if ( a.rows != nullptr && a.nrows > 0 )
-    {
-        std::snprintf( g_lps_name, sizeof( g_lps_name ), "kLpsStateRows<%s, %d, %s>",
-                       a.fracture ? "true" : "false", a.precision == PDK_MIXED ? 1 : 0,
-                       a.vol_uniform ? "false" : "true" );
-        return g_lps_name;
-    }
-    return a.fracture ? ( a.precision == PDK_MIXED ? "kLpsState<true, 1>" : "kLpsState<true, 0>" )
-                      : ( a.precision == PDK_MIXED ? "kLpsState<false, 1>" : "kLpsState<false, 0>" );
-}
 // The output passes take the row windows wherever the layout has a row table
 // and the specimen has no per-particle material type, temperature or plastic
 // stretch (the same results either way).
@@ -2007,6 +1974,41 @@ LpsPick pickLps( const PDArgs& a, int64_t nslices )
     p.fn = a.fracture ? ( a.precision == PDK_MIXED ? kLpsState<true, kMixed> : kLpsState<true, kF64> )
                       : ( a.precision == PDK_MIXED ? kLpsState<false, kMixed> : kLpsState<false, kF64> );
     return p;
+}
+
+const char* forceKernelName( const PDArgs& a )
+{
+    const char* frac = a.fracture ? "true" : "false";
+    const int prec = a.precision == PDK_MIXED ? 1 : 0;
+    if ( !useRowWindows( a ) )
+    {
+        const bool mm = prec == 1 && a.mtype != nullptr && ( a.model == kPMB || a.model == kLPS );
+        std::snprintf( g_force_name, sizeof( g_force_name ), "kForce<%d, %s, %d, %d, %s%s>", a.model, frac, prec,
+                       normalizeUnroll( a.unroll ), a.exist ? "true" : "false", mm ? ", true" : "" );
+        return g_force_name;
+    }
+    const int waves = pickForce( a, a.nslices ).waves;
+    const char* hole = a.hole_win ? "true" : "false";
+    if ( rowFeatures( a ) )
+        std::snprintf( g_force_name, sizeof( g_force_name ), "kForceRowsF<%d, %s, %d, %d, %d, %s>", a.model, frac,
+                       prec, rowFeatures( a ), waves, hole );
+    else
+        std::snprintf( g_force_name, sizeof( g_force_name ), "kForceRows<%d, %s, %d, %s, %d, %s, %d>", a.model, frac,
+                       prec, rowsGeneral( a ) ? "true" : "false", waves, hole, waves > 1 ? kSplitSlots : 1 );
+    return g_force_name;
+}
+const char* lpsKernelName( const PDArgs& a )
+{
+    if ( a.rows != nullptr && a.nrows > 0 )
+    {
+        std::snprintf( g_lps_name, sizeof( g_lps_name ), "kLpsStateRows<%s, %d, %s, %d, %s>",
+                       a.fracture ? "true" : "false", a.precision == PDK_MIXED ? 1 : 0,
+                       a.vol_uniform ? "false" : "true", pickLps( a, a.nslices ).waves,
+                       a.hole_win ? "true" : "false" );
+        return g_lps_name;
+    }
+    return a.fracture ? ( a.precision == PDK_MIXED ? "kLpsState<true, 1>" : "kLpsState<true, 0>" )
+                      : ( a.precision == PDK_MIXED ? "kLpsState<false, 1>" : "kLpsState<false, 0>" );
 }
 
 void launchLpsState( const PDArgs* args_dev, const PDArgs& a, bool weighted_volume, bool dilatation,

@@ -461,8 +461,8 @@ int pdk_set_graph(pdk_spec spec, int32_t enable);
 int pdk_kernel_timing(pdk_spec spec, int32_t enable);
 int pdk_kernel_time(pdk_spec spec, int32_t kernel_class, double* total_ms, int64_t* launches);
 /* Name of the device function behind a kernel class for the spec's current
- * configuration (rocprofv3 adds the instance's further template arguments:
- * waves per slice, missing sites, slots together). */
+ * configuration, as rocprofv3 reports it.  The row-window passes end in waves per
+ * slice, missing sites and (kForceRows) slots together. */
 int pdk_kernel_name(pdk_spec spec, int32_t kernel_class, char* buf, int32_t buflen);
 
 /* ---- serving: continuous batching ---------------------------------------------

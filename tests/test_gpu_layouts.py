@@ -235,3 +235,27 @@ def test_tight_budgets_keep_the_compact_form(shape):
         seen.add("Rows" in auto[1])
     say(f"case: {shape}: row windows chosen over the budgets: {sorted(seen)}")
     assert seen == {False, True}
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("model", ["PMB", "LPS"])
+def test_kernel_names_tell_the_instance(model, precision):
+    """Waves per slice and missing sites are part of the reported names: 8 up
+    to 256 slices, 4 above, 1 on large specimens."""
+    hole = lambda i, j, k: (i - 16) ** 2 + (j - 15) ** 2 > 49
+    for dims, keep, waves in (((16, 32, 32), None, 8), ((17, 31, 32), None, 4), ((60, 60, 60), None, 1),
+                              ((33, 30, 10), hole, 8), ((33, 30, 33), hole, 4), ((60, 60, 60), hole, 1)):
+        w = box(model, dims, 3.01, True)
+        if keep:
+            cut(w, dims, keep)
+        w["desc"].precision = precision
+        s = engine.Spec(ctx(), w["desc"], w["x"].shape[0])
+        configs.upload(s, w)
+        configs.setup(s, w)
+        tail = f"{waves}, {'true' if keep else 'false'}"
+        m = {"PMB": 0, "LPS": 1}[model]
+        say(f"case: {model} {dims} precision {precision}: {s.kernel_name(0)} {s.kernel_name(1)}")
+        assert s.kernel_name(0) == f"kForceRows<{m}, true, {precision}, false, {tail}, {5 if waves > 1 else 1}>"
+        if model == "LPS":
+            assert s.kernel_name(1) == f"kLpsStateRows<true, {precision}, false, {tail}>"
+        s.close()
