@@ -1797,32 +1797,53 @@ ForceFn pickForceRowsFeat( const PDArgs& a )
 
 // Waves per slice of a launch over nslices slices.  With one wave per slice a
 // launch of fewer than about four waves per SIMD (1024 SIMDs) lasts as long
-// as one wave's chain of slots; the split form (pdk_rows.hpp) shortens that
-// chain but leaves waves waiting at its barriers, so it loses once the SIMDs
-// are full.  Measured, one step of a cube, 1 / 4 / 8 waves per slice, in us:
+// as one wave's chain of slots, and its time steps up at every further 1024
+// slices; the split form (pdk_rows.hpp) shortens that chain but leaves waves
+// waiting at its barriers and adds five slots of every row, however short, so
+// it loses once the SIMDs are full, and on short rows sooner.  Its time steps
+// up with every 256 slices (a block per CU), so the lines are multiples of 256.
+// Measured, one step of a cube, 1 / 4 / 8 waves per slice, in us:
 //   slices                  200            512           1077          2197
-//   FP64 PMB fracture   55/ 20/ 15    56/ 25/ 28    71/ 48/ 66    91/ 80/118
+//   FP64 PMB fracture   55/ 20/ 15    56/ 25/ 28    71/ 48/ 66    92/ 80/118
 //   FP64 LPS fracture  148/ 54/ 39   150/ 68/ 75   189/128/181   242/210/328
-//   FP64 two materials 168/ 60/ 44   168/ 73/ 83   204/156/199   256/261/361
-//   FP64 temperature    61/ 26/ 20    61/ 32/ 34    76/ 58/ 77    97/ 94/135
-//   FP64 plastic        95/ 30/ 21   115/ 38/ 42   130/ 71/ 99   148/116/178
-//   mixed PMB fracture  32/ 16/ 12    32/ 18/ 21    33/ 33/ 47    37/ 54/ 82
-//   mixed LPS fracture  81/ 35/ 25    81/ 38/ 38    82/ 63/ 85    95/106/153
-//   mixed plastic       75/ 25/ 17    88/ 32/ 36   102/ 60/ 85   114/ 97/152
-// Eight waves (up to 89 KB of LDS) fit once on a CU, so they serve up to 256
-// slices.  With temperature the line stays below what the cube suggests: 40
-// steps of a heated 49^3 block (1839 slices) took 4.09 ms with one wave per
-// slice, 4.38 with four.
+//   FP64 two materials  76/ 27/ 20    75/ 32/ 37    89/ 62/ 87   109/104/158
+//   FP64 temperature    56/ 22/ 16    57/ 28/ 30    71/ 53/ 72    90/ 88/129
+//   FP64 plastic        94/ 29/ 21   114/ 36/ 41   129/ 69/ 98   146/114/176
+//   mixed PMB fracture  32/ 16/ 11    32/ 17/ 20    33/ 33/ 46    38/ 53/ 81
+//   mixed LPS fracture  81/ 34/ 24    81/ 36/ 37    82/ 61/ 84    92/105/149
+//   mixed two materials 57/ 23/ 15    56/ 24/ 27    58/ 45/ 64    67/ 74/113
+//   mixed temperature   39/ 17/ 13    39/ 19/ 23    40/ 37/ 53    50/ 62/ 96
+//   mixed plastic       74/ 25/ 17    87/ 31/ 35   101/ 60/ 84   114/ 96/152
+//   rows of 1 to 3 slots (horizon 1.5 spacings):
+//   FP64 PMB fracture   14/  8/  7    14/  9/ 12    17/ 17/ 28    22/ 26/ 49
+//   mixed PMB fracture  10/  7/  6    10/  8/ 11    11/ 14/ 23    12/ 22/ 40
+//   mixed LPS fracture  22/ 14/ 13    22/ 16/ 19    23/ 26/ 42    26/ 41/ 71
+//   missing sites (a hole; 185, 510, 1054 and 2201 slices):
+//   FP64 PMB fracture   58/ 20/ 15    58/ 25/ 28    74/ 59/ 67    98/106/127
+//   mixed LPS fracture  82/ 35/ 25    82/ 38/ 38    84/ 84/ 88   104/148/164
+// Eight waves take a CU's LDS once (38 to 140 KB), so they serve up to 256
+// slices, where they won in every form.
 int splitWaves( const PDArgs& a, int64_t nslices )
 {
     if ( a.row_max > kSplitSlots )
         return 1;
     if ( nslices <= 256 )
         return 8;
+    // the last multiple of 256 up to which four waves measured faster, but for
+    // sizes just past a multiple of 1024, where one wave's step comes first:
+    // PMB, LPS, several materials, temperature, plastic
+    static constexpr int16_t kFour[2][2][2][5] = {
+        // rows of three slots and more on average: FP64, mixed; the same with missing sites
+        { { { 2560, 2560, 1792, 1792, 2560 }, { 1024, 1536, 1536, 1280, 2304 } },
+          { { 1536, 1792, 1536, 1280, 1792 }, { 1280, 1024, 1024, 1024, 1536 } } },
+        // shorter ones: 2 spacings decide (at 1.5, four waves lose up to 12 %
+        // in the last 512 slices before a line)
+        { { { 1536, 1536, 1536, 1536, 1792 }, { 768, 1024, 1024, 768, 1536 } },
+          { { 1024, 1280, 768, 768, 1280 }, { 768, 1024, 768, 512, 1280 } } } };
     const bool lps = a.model == kLPS || a.model == kLinLPS;
-    const int64_t four = a.precision == PDK_MIXED ? ( lps || a.splas ? 1536 : 1088 )
-                                                  : ( a.mtype || a.temp ? 1792 : 2560 );
-    return nslices <= four ? 4 : 1;
+    const int kind = a.mtype ? 2 : ( a.splas ? 4 : ( a.temp && !lps ? 3 : ( lps ? 1 : 0 ) ) );
+    const bool short_rows = a.stencil_slots < 3 * a.nrows;
+    return nslices <= kFour[short_rows][a.hole_win != nullptr][a.precision == PDK_MIXED][kind] ? 4 : 1;
 }
 
 ForcePick pickForce( const PDArgs& a, int64_t nslices )

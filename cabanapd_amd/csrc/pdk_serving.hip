@@ -159,7 +159,12 @@ struct BatchEngine::Impl
                 gi = it->second;
             Group& g = ng[gi];
             PDArgs a = *v.h;
-            g.variant.row_max = std::max( g.variant.row_max, a.row_max ); // decides whether slices are split
+            if ( a.row_max > g.variant.row_max ) // the longest rows decide whether slices are split
+            {
+                g.variant.row_max = a.row_max;
+                g.variant.nrows = a.nrows;
+                g.variant.stencil_slots = a.stencil_slots;
+            }
             a.parity_offset = r.parity_offset;
             a.end_launch = r.end_launch;
             a.launch_ctr = ctr.as<int64_t>();

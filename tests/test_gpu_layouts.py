@@ -259,3 +259,58 @@ def test_kernel_names_tell_the_instance(model, precision):
         if model == "LPS":
             assert s.kernel_name(1) == f"kLpsStateRows<true, {precision}, false, {tail}>"
         s.close()
+
+
+def waves_of(s):
+    return int(s.kernel_name(0).split("<")[1].split(",")[4])
+
+
+LINES = {  # (kind, rows of a 1.5-spacing horizon, missing sites): four waves up to, FP64 and mixed
+    ("pmb", False, False): (2560, 1024), ("pmb", True, False): (1536, 768), ("pmb", False, True): (1536, 1280),
+    ("lps", False, False): (2560, 1536), ("lps", True, False): (1536, 1024), ("lps", False, True): (1792, 1024),
+    ("materials", True, False): (1536, 1024), ("thermal", False, False): (1792, 1280),
+    ("thermal", True, True): (768, 512), ("epp", False, True): (1792, 1536), ("epp", True, False): (1792, 1536),
+}
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("kind,short,hole", list(LINES))
+def test_lines_of_split_launches(kind, short, hole, precision):
+    """The size up to which four waves share a slice depends on the rows, the
+    form and the precision: on both sides of each line, the gathers' bits."""
+    line = LINES[kind, short, hole][precision]
+    for slices, waves in ((line, 4), (line + 1, 1)):
+        # layers of 8 x 8 = 64 particles; the holes' layers have 4 sites more
+        dims = (9, 8, slices) if hole else (8, 8, slices)
+        w = box("LPS" if kind in ("lps", "materials") else "PMB", dims, 1.5 if short else 3.01, True)
+        if hole:
+            cut(w, dims, lambda i, j, k: (i != 4) | (j == 0))
+            for key in ("x", "vol", "rho", "u", "v"):
+                w[key] = np.ascontiguousarray(w[key][:64 * slices])
+        d = w["desc"]
+        n = w["x"].shape[0]
+        assert n == 64 * slices
+        rng = np.random.default_rng(5)
+        if kind == "epp":
+            d.mechanics, d.sigma_y = 1, 2.5e7
+        if kind == "thermal":
+            d.thermal, d.alpha, d.temp0 = 1, 1e-6, 20.0
+            w["temperature"] = 20.0 + 40.0 * rng.random(n)
+        if kind == "materials":
+            w["materials"] = ([(4.3e10, 2.9e10, 3.8), (8e10, 5e10, 38.0)], (rng.random(n) < 0.4).astype(np.int32))
+        d.precision = precision
+        out = []
+        for variant in (None, 4):
+            s = engine.Spec(ctx(), d, n)
+            configs.upload(s, w)
+            configs.setup(s, w)
+            if variant is None:
+                say(f"case: {kind} {slices} slices precision {precision}: {s.kernel_name(0)}")
+                assert waves_of(s) == waves
+            else:
+                s.set_tuning(variant)
+            s.step(3)
+            out.append([s.get("u"), s.get("v"), s.get("f"), s.bonds()[2]])
+            s.close()
+        for a, b in zip(*out):
+            assert np.array_equal(a, b)
