@@ -1248,6 +1248,8 @@ int pdk_build_bonds( pdk_spec s )
     return guarded( [&] {
         require( s && s->uploaded, "spec not uploaded" );
         require( !s->in_batch, "spec is running in the batch engine" );
+        s->built = false; // until this build is complete
+        s->inited = false;
         if ( isContact( s->d ) )
         {
             s->timed( kClsBuild, [&] { contactBuild( s, true ); } );
@@ -1267,6 +1269,7 @@ int pdk_build_bonds( pdk_spec s )
             s->stab_xiv.release();
             s->nsten = 0;
             s->slot = SlotForm{};
+            s->splas.release();
             // Full lattice: slot q of every row is stencil entry q, so the
             // force pass computes neighbor ids instead of streaming them.
             // Built straight from the lattice where the stencil is clear of
@@ -1291,6 +1294,8 @@ int pdk_build_bonds( pdk_spec s )
             if ( !direct && s->lattice_rows && s->d.bond_layout != PDK_BONDS_COMPACT )
             {
                 s->pushArgs();
+                // a plastic stretch per bond slot goes with the form
+                DevBuf* state = s->d.mechanics == PDK_MECH_EPP ? &s->splas : nullptr;
                 s->timed( kClsBuild, [&] {
                     try
                     {
@@ -1301,10 +1306,11 @@ int pdk_build_bonds( pdk_spec s )
                             s->vol_uniform && !( s->d.fracture && s->any_nofail ) && !isLinearModel( s->d.model );
                         if ( buildStencilSlots( s->h, s->lat_dims, s->lat_h, q.rc, s->h_perm, s->col, s->intact,
                                                 s->slice_ptr.as<int64_t>(), s->total_rows, s->col_rows_cap, s->slot,
-                                                s->scratch, s->acct(), s->st ) ||
+                                                s->scratch, s->acct(), s->st, state ) ||
                              ( holes && buildHoleSlots( s->h, s->lat_dims, s->lat_lo, s->lat_h, q.rc, s->h_perm,
                                                         s->col, s->intact, s->slice_ptr.as<int64_t>(), s->total_rows,
-                                                        s->col_rows_cap, s->slot, s->scratch, s->acct(), s->st ) ) )
+                                                        s->col_rows_cap, s->slot, s->scratch, s->acct(), s->st,
+                                                        state ) ) )
                             s->nsten = s->slot.slots;
                     }
                     catch ( const MemError& )
@@ -1331,7 +1337,8 @@ int pdk_build_bonds( pdk_spec s )
             // BasePlasticity::updateBonds after the neighbor list: zero s_p
             // per bond (CabanaPD_Solver.hpp:183-185, CabanaPD_ForceModels.hpp:157-161)
             const size_t b = static_cast<size_t>( std::max<int64_t>( s->total_rows, 1 ) ) * kSlice * sizeof( double );
-            s->splas.alloc( b, s->acct() );
+            if ( s->splas.bytes() != b )
+                s->splas.alloc( b, s->acct() );
             PDK_HIP( hipMemsetAsync( s->splas.as<double>(), 0, b, s->st ) );
         }
         s->built = true;

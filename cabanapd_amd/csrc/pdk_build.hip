@@ -1287,11 +1287,15 @@ std::vector<int4> slotEntries( const std::vector<SlotEntry>& es )
 // the FP64 |xi|^2 of each entry, and move them into place.
 // With site and id (missing sites) also the windows; false, with nothing
 // moved, when they do not fit the row passes.
+// With bond_state also one double per bond slot.  keep_room (a compact form is
+// there and would do): MemError, with nothing moved, unless the budget then
+// still has what later calls on this specimen may allocate (stress tensors and
+// their download, 144 B a particle, and a body force, 24 B).
 bool finishSlots( int64_t n, int64_t nslices, const LatticeBox& L, const std::vector<SlotEntry>& es,
                   const int4* dent, const double h[3], DevBuf& col, DevBuf& intact, int64_t* slice_ptr_dev,
                   int64_t& total_rows, int64_t& col_capacity_rows, SlotForm& out, MemAccount* acct,
                   hipStream_t st, const int32_t* site = nullptr, const int32_t* id = nullptr,
-                  int32_t* flag_dev = nullptr )
+                  int32_t* flag_dev = nullptr, DevBuf* bond_state = nullptr, bool keep_room = false )
 {
     const int32_t S = static_cast<int32_t>( es.size() );
     const int64_t rows = nslices * S;
@@ -1382,6 +1386,19 @@ bool finishSlots( int64_t n, int64_t nslices, const LatticeBox& L, const std::ve
     PDK_HIP( hipMemcpyAsync( dsoff.as<int32_t>(), soff.data(), 256 * sizeof( int32_t ), hipMemcpyHostToDevice, st ) );
     PDK_HIP( hipMemcpyAsync( dtab.as<float4>(), tab.data(), 256 * sizeof( float4 ), hipMemcpyHostToDevice, st ) );
     PDK_HIP( hipMemcpyAsync( dxi2.as<double>(), tab2.data(), 256 * sizeof( double ), hipMemcpyHostToDevice, st ) );
+    DevBuf nstate;
+    if ( bond_state )
+        nstate.alloc( static_cast<size_t>( rows ) * kSlice * sizeof( double ), acct );
+    if ( keep_room && acct )
+    {
+        // (the compact form's arrays are given back below)
+        const uint64_t later = static_cast<uint64_t>( n ) * 168, back = col.bytes() + intact.bytes();
+        if ( later > back )
+        {
+            acct->reserve( later - back );
+            acct->unreserve( later - back );
+        }
+    }
     // every allocation is done: from here on the compact form is replaced
     std::vector<int64_t> sp( nslices + 1 );
     for ( int64_t k = 0; k <= nslices; k++ )
@@ -1390,6 +1407,8 @@ bool finishSlots( int64_t n, int64_t nslices, const LatticeBox& L, const std::ve
     PDK_HIP( hipStreamSynchronize( st ) );
     col = std::move( ncol );
     intact = std::move( nintact );
+    if ( bond_state )
+        *bond_state = std::move( nstate );
     out.exist = std::move( nexist );
     out.soff = std::move( dsoff );
     out.table = std::move( dtab );
@@ -1458,7 +1477,7 @@ __global__ __launch_bounds__( kThreads ) void kDirectSlotCheck( const double* __
 bool buildStencilSlots( const PDArgs& a, const int64_t dims[3], const double h[3], double rc,
                         const std::vector<int64_t>& perm_host, DevBuf& col, DevBuf& intact, int64_t* slice_ptr_dev,
                         int64_t& total_rows, int64_t& col_capacity_rows, SlotForm& out, BuildScratch& s,
-                        MemAccount* acct, hipStream_t st )
+                        MemAccount* acct, hipStream_t st, DevBuf* bond_state )
 {
     const int64_t n = a.n;
     std::vector<SlotEntry> es;
@@ -1481,13 +1500,13 @@ bool buildStencilSlots( const PDArgs& a, const int64_t dims[3], const double h[3
     if ( flag )
         return false;
     return finishSlots( n, a.nslices, L, es, dent.as<int4>(), h, col, intact, slice_ptr_dev, total_rows,
-                        col_capacity_rows, out, acct, st );
+                        col_capacity_rows, out, acct, st, nullptr, nullptr, nullptr, bond_state, true );
 }
 
 bool buildHoleSlots( const PDArgs& a, const int64_t dims[3], const double lo[3], const double h[3], double rc,
                      const std::vector<int64_t>& perm_host, DevBuf& col, DevBuf& intact, int64_t* slice_ptr_dev,
                      int64_t& total_rows, int64_t& col_capacity_rows, SlotForm& out, BuildScratch& s, MemAccount* acct,
-                     hipStream_t st )
+                     hipStream_t st, DevBuf* bond_state )
 {
     const int64_t n = a.n;
     // a table of the box's sites: only where at least an eighth of them hold a
@@ -1524,7 +1543,7 @@ bool buildHoleSlots( const PDArgs& a, const int64_t dims[3], const double lo[3],
         return false;
     return finishSlots( n, a.nslices, L, es, dent.as<int4>(), h, col, intact, slice_ptr_dev, total_rows,
                         col_capacity_rows, out, acct, st, site.as<int32_t>(), id.as<int32_t>(),
-                        s.flag.as<int32_t>() );
+                        s.flag.as<int32_t>(), bond_state, true );
 }
 
 bool buildStencilSlotsDirect( const double* x_dev, int64_t n, const int64_t dims[3], const double h[3], double rc,

@@ -179,14 +179,14 @@ struct SlotForm
 bool buildStencilSlots( const PDArgs& a, const int64_t dims[3], const double h[3], double rc,
                         const std::vector<int64_t>& perm_host, DevBuf& col, DevBuf& intact, int64_t* slice_ptr_dev,
                         int64_t& total_rows, int64_t& col_capacity_rows, SlotForm& out, BuildScratch& s,
-                        MemAccount* acct, hipStream_t st );
+                        MemAccount* acct, hipStream_t st, DevBuf* bond_state );
 // The same form for a lattice with missing sites (rows checked against the
 // compact ones as above; caller order = lattice order); adds the neighbour
 // windows that the row passes stage.
 bool buildHoleSlots( const PDArgs& a, const int64_t dims[3], const double lo[3], const double h[3], double rc,
                      const std::vector<int64_t>& perm_host, DevBuf& col, DevBuf& intact, int64_t* slice_ptr_dev,
                      int64_t& total_rows, int64_t& col_capacity_rows, SlotForm& out, BuildScratch& s, MemAccount* acct,
-                     hipStream_t st );
+                     hipStream_t st, DevBuf* bond_state );
 // The same form built without the cell search: every in-box stencil bond is
 // checked with the exact cutoff test; fills cnt.  False (nothing written but
 // cnt) when the lattice does not qualify.

@@ -314,3 +314,50 @@ def test_lines_of_split_launches(kind, short, hole, precision):
             s.close()
         for a, b in zip(*out):
             assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("shape,kind", [("hole", "epp"), ("whole horizon", "epp"), ("sparse", "epp"), ("sparse", "pmb"),
+                                        ("hole", "pmb")])
+def test_tight_budgets_hold_the_whole_run(shape, kind):
+    """Wherever the HBM budget holds build, steps, stress and downloads over
+    the compact form, the form that the build chooses gets through them too:
+    the plastic stretches of its slots and the buffers of later calls count."""
+    if shape == "whole horizon":
+        w = box("PMB", (40, 31, 6), 3, True)
+    else:
+        dims, keep = SHAPES["hole"] if shape == "hole" else (
+            (60, 50, 20), lambda i, j, k: np.random.default_rng(4).random(i.size) < 0.2)
+        w = cut(box("PMB", dims, 3.01, True), dims, keep)
+    d = type(w["desc"]).from_buffer_copy(w["desc"])
+    if kind == "epp":
+        d.mechanics, d.sigma_y = 1, 2.5e7
+    n = w["x"].shape[0]
+
+    def run(budget, layout):
+        d.bond_layout = layout
+        with engine.Context(0, budget) as c:
+            s = None
+            try:
+                s = engine.Spec(c, d, n)
+                configs.upload(s, w)
+                configs.setup(s, w)
+                s.step(3)
+                s.compute_stress()
+                s.set_body_force(np.zeros((n, 3)))
+                return s.get("u"), s.get("stress"), s.kernel_name(0)
+            except engine.PdkError:
+                return None
+            finally:
+                if s is not None:
+                    s.close()
+
+    seen = set()
+    for budget in np.geomspace(3e6, 6e7, 60).astype(int):
+        compact, auto = run(int(budget), PDK_BONDS_COMPACT), run(int(budget), 0)
+        if compact is None:
+            continue
+        assert auto is not None, f"budget {budget}"
+        assert np.array_equal(auto[0], compact[0]) and np.array_equal(auto[1], compact[1], equal_nan=True)
+        seen.add("Rows" in auto[2])
+    say(f"case: {shape} {kind}, {n} particles: row windows chosen over the budgets: {sorted(seen)}")
+    assert seen == {False, True}
