@@ -57,13 +57,11 @@ class HostTransfer
     // dst (host) <- src (device) after the work queued on st; complete on return.
     void out( void* dst, const void* src, size_t bytes, hipStream_t st )
     {
-        if ( bytes < kDirect )
-        {
-            PDK_HIP( hipMemcpyAsync( dst, src, bytes, hipMemcpyDeviceToHost, st ) );
+        // The work queued on st is waited for here, before the context's
+        // slots are taken: other specimens' copies go on meanwhile.
+        if ( bytes >= kDirect )
             PDK_HIP( hipStreamSynchronize( st ) );
-            return;
-        }
-        run( bytes, [=]( Slot& s, size_t off, size_t len ) {
+        if ( bytes < kDirect || !run( bytes, [=]( Slot& s, size_t off, size_t len ) {
             hipError_t e = hipMemcpyAsync( s.mem, static_cast<const char*>( src ) + off, len, hipMemcpyDeviceToHost, st );
             if ( e == hipSuccess )
                 e = hipEventRecord( s.done, st );
@@ -72,7 +70,11 @@ class HostTransfer
             if ( e == hipSuccess )
                 std::memcpy( static_cast<char*>( dst ) + off, s.mem, len );
             return e;
-        } );
+        } ) )
+        {
+            PDK_HIP( hipMemcpyAsync( dst, src, bytes, hipMemcpyDeviceToHost, st ) );
+            PDK_HIP( hipStreamSynchronize( st ) );
+        }
     }
 
   private:
@@ -137,16 +139,37 @@ class HostTransfer
         }
     }
 
-    void run( size_t bytes, std::function<hipError_t( Slot&, size_t, size_t )> chunk )
+    // The pinned slots and their events; false where they cannot be had.
+    bool ready()
     {
-        std::lock_guard<std::mutex> one( mu_ ); // one copy at a time
         for ( Slot& s : slots_ )
         {
+            hipError_t e = hipSuccess;
             if ( !s.mem )
-                PDK_HIP( hipHostMalloc( reinterpret_cast<void**>( &s.mem ), kChunk, hipHostMallocDefault ) );
-            if ( !s.done )
-                PDK_HIP( hipEventCreateWithFlags( &s.done, hipEventDisableTiming ) );
+                e = hipHostMalloc( reinterpret_cast<void**>( &s.mem ), kChunk, hipHostMallocDefault );
+            if ( e != hipSuccess )
+                s.mem = nullptr;
+            else if ( !s.done )
+            {
+                e = hipEventCreateWithFlags( &s.done, hipEventDisableTiming );
+                if ( e != hipSuccess )
+                    s.done = nullptr;
+            }
+            if ( e != hipSuccess )
+            {
+                (void)hipGetLastError();
+                return false;
+            }
         }
+        return true;
+    }
+
+    // False, with nothing copied, where there are no slots.
+    bool run( size_t bytes, std::function<hipError_t( Slot&, size_t, size_t )> chunk )
+    {
+        std::lock_guard<std::mutex> one( mu_ ); // one copy at a time
+        if ( !ready() )
+            return false;
         try
         {
             while ( workers_.size() + 1 < kSlots )
@@ -176,6 +199,7 @@ class HostTransfer
             job_.reset();
         }
         PDK_HIP( static_cast<hipError_t>( j->err.load() ) );
+        return true;
     }
 
     int device_;
