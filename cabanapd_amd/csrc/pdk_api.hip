@@ -2,6 +2,7 @@
 // host orchestration of the reference's Solver step order.
 #include <algorithm>
 #include <atomic>
+#include <chrono>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -9,6 +10,7 @@
 #include <memory>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "pdk_internal.hpp"
@@ -186,6 +188,11 @@ struct pdk_ctx_s
     std::unique_ptr<BatchEngine> batch;
     std::unique_ptr<HostTransfer> transfer;
     std::atomic<int64_t> live_specs{ 0 };
+    std::mutex rec_mu;
+    std::vector<pdk_spec> rec_holders; // contact specimens with pair records (under rec_mu)
+    std::atomic<int> rec_wanted{ 0 };  // allocations waiting for them
+    bool reclaimRecords( const std::function<bool()>& fits );
+    void releaseRecords( pdk_spec s ); // by whoever set its rec_busy
 };
 
 struct pdk_series_s;
@@ -254,6 +261,11 @@ struct pdk_spec_s
     // contact bookkeeping
     int64_t steps_since_build = 0;
     double max_disp = 0.0;
+    // pair_rec belongs to whoever set rec_busy: a call that uses it, or
+    // reclaimRecords releasing it.  The launch arguments hold its address as the
+    // last such call left it; PairRecords renews them before any launch.
+    std::atomic<bool> rec_busy{ false };
+    std::atomic<uint64_t> rec_bytes{ 0 };
     // contact step: the largest displacement since the last build, in pinned
     // host memory that the device writes, and the event after that (the host
     // waits on it, not on the stream)
@@ -455,9 +467,6 @@ struct pdk_spec_s
         h.stress = stress.as<double>();
         h.radius = radius ? radius.as<double>() : nullptr;
         h.u_neigh = u_neigh ? u_neigh.as<double>() : nullptr;
-        h.rec_x = pair_rec.as<double4>();
-        h.rec_u = pair_rec ? h.rec_x + n : nullptr;
-        h.rec_v = pair_rec ? h.rec_x + 2 * n : nullptr;
         h.sid = sid ? sid.as<uint8_t>() : nullptr;
         h.stencil = stab ? stab.as<float4>() : nullptr;
         h.stencil_xi2d = stab_xi2d ? stab_xi2d.as<double>() : nullptr;
@@ -759,6 +768,58 @@ void contactStep( pdk_spec s, int32_t nsteps );
 void contactForceStore( pdk_spec s );
 } // namespace pdk
 
+namespace
+{
+thread_local int t_records_held = 0; // specimens with records that a call on this thread uses
+}
+
+void pdk_ctx_s::releaseRecords( pdk_spec s )
+{
+    std::lock_guard<std::mutex> g( rec_mu );
+    s->pair_rec.release();
+    s->rec_bytes = 0;
+    rec_holders.erase( std::remove( rec_holders.begin(), rec_holders.end(), s ), rec_holders.end() );
+}
+
+// The pair records of contact specimens, one after the other.  Those that a
+// call is using on another thread are waited for (contactStep gives them up
+// between two steps), unless this thread uses some itself: it gives those up first
+// (rebuildList), so no two wait for each other.
+bool pdk_ctx_s::reclaimRecords( const std::function<bool()>& fits )
+{
+    for ( bool waiting = false;; )
+    {
+        bool again = false;
+        {
+            std::lock_guard<std::mutex> g( rec_mu );
+            const bool ok = fits();
+            for ( size_t k = 0; !ok && !again && k < rec_holders.size(); k++ )
+            {
+                pdk_spec s = rec_holders[k];
+                if ( s->rec_busy.exchange( true ) )
+                    continue;
+                // (every call that uses them waits for its launches before it returns)
+                s->pair_rec.release();
+                s->rec_bytes = 0;
+                rec_holders.erase( rec_holders.begin() + k );
+                s->rec_busy = false;
+                again = true;
+            }
+            if ( ok || ( !again && ( rec_holders.empty() || t_records_held > 0 ) ) )
+            {
+                if ( waiting )
+                    rec_wanted--;
+                return ok;
+            }
+            if ( !waiting )
+                rec_wanted++;
+            waiting = true;
+        }
+        if ( !again )
+            std::this_thread::sleep_for( std::chrono::microseconds( 20 ) );
+    }
+}
+
 extern "C" {
 
 const char* pdk_last_error( void )
@@ -869,6 +930,7 @@ int pdk_ctx_create( int device, uint64_t hbm_budget, pdk_ctx* out )
         c->acct.budget = hbm_budget ? hbm_budget : static_cast<uint64_t>( 0.9 * freeb );
         c->batch = std::make_unique<BatchEngine>( c.get() );
         c->transfer = std::make_unique<HostTransfer>( device );
+        c->acct.reclaim = [p = c.get()]( const std::function<bool()>& fits ) { return p->reclaimRecords( fits ); };
         *out = c.release();
     } );
 }
@@ -947,7 +1009,6 @@ int pdk_spec_create( pdk_ctx ctx, const pdk_model_desc* desc, int64_t n, pdk_spe
         if ( isContact( *desc ) )
         {
             s->u_neigh.alloc( d3, a );
-            s->pair_rec.alloc( 3 * n * sizeof( double4 ), a );
             if ( desc->polydisperse )
                 s->radius.alloc( d1, a );
         }
@@ -1038,6 +1099,12 @@ int pdk_spec_destroy( pdk_spec s )
             (void)hipStreamSynchronize( s->st );
         s->dropGraphs();
         detachSeries( s );
+        if ( s->ctx )
+        {
+            while ( s->rec_busy.exchange( true ) )
+                std::this_thread::yield(); // being released
+            s->ctx->releaseRecords( s );
+        }
         if ( s->disp_ready )
             (void)hipEventDestroy( s->disp_ready );
         if ( s->disp_pinned )
@@ -1237,8 +1304,9 @@ int pdk_spec_bytes( pdk_spec s, uint64_t* bytes )
         for ( const DevBuf* b : { &s->x, &s->U0, &s->U1, &s->v, &s->f, &s->vol, &s->rho, &s->nofail, &s->bcflag,
                                   &s->body, &s->m, &s->theta, &s->lpsA, &s->lpsB, &s->W, &s->phi, &s->perm, &s->inv,
                                   &s->cnt, &s->slice_ptr, &s->col, &s->intact, &s->radius, &s->u_neigh,
-                                  &s->pair_rec, &s->partial, &s->args, &s->sid, &s->stab, &s->stab_xi2d, &s->stab_xiv } )
+                                  &s->partial, &s->args, &s->sid, &s->stab, &s->stab_xi2d, &s->stab_xiv } )
             t += b->bytes();
+        t += s->rec_bytes;
         *bytes = t;
     } );
 }
@@ -2409,6 +2477,63 @@ ContactState contactState( pdk_spec s )
     c.disp_dev = s->disp_dev;
     c.disp_ready = s->disp_ready;
     return c;
+}
+
+PairRecords::PairRecords( pdk_spec s ) : s_( s )
+{
+    while ( s->rec_busy.exchange( true ) )
+        std::this_thread::yield(); // being released
+    try
+    {
+        if ( !s->pair_rec && !wanted() )
+        {
+            std::lock_guard<std::mutex> g( s->ctx->rec_mu );
+            fresh_ = s->pair_rec.allocIfRoom( 3 * s->n * sizeof( double4 ), s->acct() );
+            if ( fresh_ )
+            {
+                s->rec_bytes = s->pair_rec.bytes();
+                s->ctx->rec_holders.push_back( s );
+            }
+        }
+        setArgs();
+    }
+    catch ( ... )
+    {
+        s->rec_busy = false;
+        throw;
+    }
+    if ( s->pair_rec )
+        t_records_held++;
+}
+PairRecords::~PairRecords()
+{
+    if ( s_->pair_rec )
+        t_records_held--;
+    s_->rec_busy = false;
+}
+bool PairRecords::wanted() const
+{
+    return s_->ctx->rec_wanted > 0;
+}
+bool PairRecords::drop()
+{
+    if ( !s_->pair_rec )
+        return false;
+    PDK_HIP( hipStreamSynchronize( s_->st ) );
+    t_records_held--;
+    s_->ctx->releaseRecords( s_ );
+    setArgs();
+    return true;
+}
+void PairRecords::setArgs()
+{
+    double4* r = s_->pair_rec.as<double4>();
+    if ( s_->h.rec_x == r )
+        return;
+    s_->h.rec_x = r;
+    s_->h.rec_u = r ? r + s_->n : nullptr;
+    s_->h.rec_v = r ? r + 2 * s_->n : nullptr;
+    s_->pushArgs();
 }
 
 void specTimed( pdk_spec s, int cls, const std::function<void()>& fn )

@@ -203,7 +203,8 @@ __device__ double normalForce( const PDArgs& A, const PairK& pk, double r, doubl
 // gather costs one cache line a lane and array: 64 lanes touched about 300
 // lines per slot.  rec_x follows the upload; rec_u and rec_v are written by the
 // pass that advances u and v.  The mass is the product rho V that the pair
-// formed before.
+// formed before.  Where memory has no room for them (PairRecords) the arrays
+// are gathered (REC = false), with the same results.
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__( 256 ) void kContactPack( const PDArgs* __restrict__ specs, int32_t parity )
 {
@@ -231,8 +232,8 @@ __global__ __launch_bounds__( 256 ) void kContactPack( const PDArgs* __restrict_
 // (Hertz-JKR, 442k polydisperse spheres, 12 listed neighbours of which about
 // 3 touch: 139 -> 127 us; 71 % of the cycles issue VALU work.  Marking by the
 // estimated tear distance of each pair instead of the bound: 140.)
-template <bool POLY, bool JKR>
-__global__ __launch_bounds__( kBlock ) void kContact( const PDArgs* __restrict__ specs, int32_t epi )
+template <bool POLY, bool JKR, bool REC>
+__global__ __launch_bounds__( kBlock ) void kContact( const PDArgs* __restrict__ specs, int32_t epi, int32_t parity )
 {
 #pragma clang fp contract( off )
     const PDArgs& A = *specs;
@@ -247,7 +248,28 @@ __global__ __launch_bounds__( kBlock ) void kContact( const PDArgs* __restrict__
     const double4* __restrict__ rec_x = A.rec_x;
     const double4* __restrict__ rec_u = A.rec_u;
     const double4* __restrict__ rec_v = A.rec_v;
-    const double4 xi = rec_x[p], ui = rec_u[p], vi = rec_v[p];
+    const double* __restrict__ x = A.x;
+    const double* __restrict__ u = A.U[parity];
+    const double* __restrict__ v = A.v;
+    auto loadX = [&]( int64_t j ) {
+        if constexpr ( REC )
+            return rec_x[j];
+        else
+            return make_double4( x[j], x[n + j], x[2 * n + j], POLY ? A.radius[j] : 0.0 );
+    };
+    auto loadU = [&]( int64_t j ) {
+        if constexpr ( REC )
+            return rec_u[j];
+        else
+            return make_double4( u[j], u[n + j], u[2 * n + j], POLY ? A.rho[j] * A.vol[j] : 0.0 );
+    };
+    auto loadV = [&]( int64_t j ) {
+        if constexpr ( REC )
+            return rec_v[j];
+        else
+            return make_double4( v[j], v[n + j], v[2 * n + j], 0.0 );
+    };
+    const double4 xi = loadX( p ), ui = loadU( p ), vi = loadV( p );
     const double vol_i = A.vol[p];
     const double rho_i = A.rho[p];
     const double mi = ui.w;
@@ -377,8 +399,8 @@ __global__ __launch_bounds__( kBlock ) void kContact( const PDArgs* __restrict__
 #pragma unroll
                 for ( int k = 0; k < 4; k++ )
                 {
-                    xj[k] = rec_x[j[k]];
-                    uj[k] = rec_u[j[k]];
+                    xj[k] = loadX( j[k] );
+                    uj[k] = loadU( j[k] );
                 }
 #pragma unroll
                 for ( int k = 0; k < 4; k++ )
@@ -398,7 +420,7 @@ __global__ __launch_bounds__( kBlock ) void kContact( const PDArgs* __restrict__
             for ( int m = 0; m < marked; m++ )
             {
                 const int32_t j = near[m][threadIdx.x];
-                pairForce( rec_x[j], rec_u[j], rec_v[j] );
+                pairForce( loadX( j ), loadU( j ), loadV( j ) );
             }
         }
     }
@@ -406,7 +428,7 @@ __global__ __launch_bounds__( kBlock ) void kContact( const PDArgs* __restrict__
         for ( int32_t q = 0; q < mycnt; q++ )
         {
             const int32_t j = colp[q * kSlice];
-            pairForce( rec_x[j], rec_u[j], rec_v[j] );
+            pairForce( loadX( j ), loadU( j ), loadV( j ) );
         }
     if ( epi != kEpiStoreOnly )
     {
@@ -469,8 +491,11 @@ __global__ __launch_bounds__( 256 ) void kContactAdvance( const PDArgs* __restri
             dd[d] = uu[d] - A.u_neigh[d * n + p];
         }
         mx = sqrt( dd[0] * dd[0] + dd[1] * dd[1] + dd[2] * dd[2] );
-        A.rec_u[p] = make_double4( uu[0], uu[1], uu[2], A.rho[p] * A.vol[p] );
-        A.rec_v[p] = make_double4( vv[0], vv[1], vv[2], 0.0 );
+        if ( A.rec_u )
+        {
+            A.rec_u[p] = make_double4( uu[0], uu[1], uu[2], A.rho[p] * A.vol[p] );
+            A.rec_v[p] = make_double4( vv[0], vv[1], vv[2], 0.0 );
+        }
     }
     red[threadIdx.x] = mx;
     __syncthreads();
@@ -521,41 +546,49 @@ __global__ __launch_bounds__( 256 ) void kContactFinal( const PDArgs* __restrict
         A.v[d * n + p] = A.v[d * n + p] + half_dt_m * A.f[d * n + p];
 }
 
-using ContactFn = void ( * )( const PDArgs*, int32_t );
-ContactFn pickContact( const PDArgs& a )
+using ContactFn = void ( * )( const PDArgs*, int32_t, int32_t );
+template <bool REC>
+ContactFn pickContactForm( const PDArgs& a )
 {
     const bool jkr = a.model == PDK_MODEL_HERTZ_JKR;
     if ( a.polydisperse )
-        return jkr ? kContact<true, true> : kContact<true, false>;
-    return jkr ? kContact<false, true> : kContact<false, false>;
+        return jkr ? kContact<true, true, REC> : kContact<true, false, REC>;
+    return jkr ? kContact<false, true, REC> : kContact<false, false, REC>;
 }
+ContactFn pickContact( const PDArgs& a )
+{
+    return a.rec_x ? pickContactForm<true>( a ) : pickContactForm<false>( a );
+}
+thread_local char g_contact_name[64];
 
 } // namespace
 
 const char* contactKernelName( const PDArgs& a )
 {
-    const bool jkr = a.model == PDK_MODEL_HERTZ_JKR;
-    if ( a.polydisperse )
-        return jkr ? "kContact<true, true>" : "kContact<true, false>";
-    return jkr ? "kContact<false, true>" : "kContact<false, false>";
+    auto text = []( bool b ) { return b ? "true" : "false"; };
+    std::snprintf( g_contact_name, sizeof( g_contact_name ), "kContact<%s, %s, %s>", text( a.polydisperse != 0 ),
+                   text( a.model == PDK_MODEL_HERTZ_JKR ), text( a.rec_x != nullptr ) );
+    return g_contact_name;
 }
 
-// The pair records of the current state.
+// The pair records (if any) of the current state.
 void launchContactPack( const PDArgs* args_dev, const PDArgs& a, int32_t parity, hipStream_t st )
 {
-    if ( a.n == 0 )
+    if ( a.n == 0 || !a.rec_x )
         return;
     hipLaunchKernelGGL( kContactPack, dim3( static_cast<unsigned>( ( a.n + 255 ) / 256 ) ), dim3( 256 ), 0, st,
                         args_dev, parity );
     PDK_HIP( hipGetLastError() );
 }
 
-void launchContactForce( const PDArgs* args_dev, const PDArgs& a, int32_t epilogue_mode, hipStream_t st )
+void launchContactForce( const PDArgs* args_dev, const PDArgs& a, int32_t epilogue_mode, int32_t parity,
+                         hipStream_t st )
 {
     if ( a.nslices == 0 )
         return;
     const unsigned g = static_cast<unsigned>( ( a.nslices + kSlicesPerBlock - 1 ) / kSlicesPerBlock );
-    hipLaunchKernelGGL( pickContact( a ), dim3( g ), dim3( kBlock ), 0, st, args_dev, epilogue_mode );
+    hipLaunchKernelGGL( pickContact( a ), dim3( g ), dim3( kBlock ), 0, st, args_dev, epilogue_mode,
+                        parity );
     PDK_HIP( hipGetLastError() );
 }
 
@@ -574,25 +607,55 @@ void contactBuild( pdk_spec_s* s, bool initial )
     contactBuildImpl( s, initial, cs.max_disp, cs.since_build );
 }
 
+namespace
+{
+// The list rebuilt between steps; short of memory, without the pair records.
+void rebuildList( pdk_spec_s* s, const ContactState& cs, PairRecords& rec )
+{
+    specTimed( s, 3, [&] {
+        try
+        {
+            contactBuildImpl( s, false, cs.max_disp, cs.since_build );
+        }
+        catch ( const MemError& )
+        {
+            if ( !rec.drop() )
+                throw;
+            contactBuildImpl( s, false, cs.max_disp, cs.since_build );
+        }
+    } );
+}
+} // namespace
+
 // Neighbor::update then the contact pass, storing f (init / computeForce).
 void contactForceStore( pdk_spec_s* s )
 {
     ContactState cs = contactState( s );
-    SpecView v = view( s );
+    PairRecords rec( s );
     if ( *cs.max_disp > cs.extend )
-        specTimed( s, 3, [&] { contactBuildImpl( s, false, cs.max_disp, cs.since_build ); } );
-    v = view( s );
+        rebuildList( s, cs, rec );
+    SpecView v = view( s );
     specTimed( s, 0, [&] {
         launchContactPack( v.dargs, *v.h, *v.cur, v.st );
-        launchContactForce( v.dargs, *v.h, kEpiStoreOnly, v.st );
+        launchContactForce( v.dargs, *v.h, kEpiStoreOnly, *v.cur, v.st );
     } );
+    // the records may be taken back once this returns
+    PDK_HIP( hipStreamSynchronize( v.st ) );
 }
 
 void contactStep( pdk_spec_s* s, int32_t nsteps )
 {
     ContactState cs = contactState( s );
+    PairRecords rec( s );
+    if ( rec.fresh() )
+    {
+        SpecView v = view( s );
+        launchContactPack( v.dargs, *v.h, *v.cur, v.st );
+    }
     for ( int32_t k = 0; k < nsteps; k++ )
     {
+        if ( rec.wanted() )
+            rec.drop();
         SpecView v = view( s );
         const int64_t nb = ( v.n + 255 ) / 256;
         if ( cs.partial->bytes() < static_cast<size_t>( nb ) * sizeof( double ) )
@@ -620,7 +683,7 @@ void contactStep( pdk_spec_s* s, int32_t nsteps )
         const bool periodic = cs.rebuild_every > 0 && *cs.since_build >= cs.rebuild_every;
         auto force = [&] {
             v = view( s );
-            specTimed( s, 0, [&] { launchContactForce( v.dargs, *v.h, kEpiApplyOnly, v.st ); } );
+            specTimed( s, 0, [&] { launchContactForce( v.dargs, *v.h, kEpiApplyOnly, *v.cur, v.st ); } );
         };
         if ( !periodic )
             force();
@@ -629,12 +692,14 @@ void contactStep( pdk_spec_s* s, int32_t nsteps )
         *cs.max_disp = mx;
         if ( mx > cs.extend || periodic )
         {
-            specTimed( s, 3, [&] { contactBuildImpl( s, false, cs.max_disp, cs.since_build ); } );
+            rebuildList( s, cs, rec );
             force();
         }
     }
     SpecView v = view( s );
     specTimed( s, 4, [&] { launchContactFinal( v.dargs, *v.h, v.st ); } );
+    // the records may be taken back once this returns
+    PDK_HIP( hipStreamSynchronize( v.st ) );
 }
 
 } // namespace pdk

@@ -6,6 +6,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <functional>
 #include <stdexcept>
 #include <mutex>
 #include <string>
@@ -45,13 +46,28 @@ struct MemAccount
     uint64_t in_use = 0;
     std::mutex mu;
 
-    void reserve( uint64_t bytes )
+    // Takes back memory that is held only while there is room for it, until
+    // fits() is true; false if it never is.  Called without mu.
+    std::function<bool( const std::function<bool()>& fits )> reclaim;
+
+    bool tryReserve( uint64_t bytes )
     {
         std::lock_guard<std::mutex> g( mu );
         if ( budget && in_use + bytes > budget )
-            throw MemError( "HBM budget exceeded: need " + std::to_string( bytes ) + " B more, " +
-                         std::to_string( budget - in_use ) + " B left" );
+            return false;
         in_use += bytes;
+        return true;
+    }
+    void reserve( uint64_t bytes )
+    {
+        if ( !tryReserve( bytes ) && !( reclaim && reclaim( [&] { return tryReserve( bytes ); } ) ) )
+            throw MemError( "HBM budget exceeded: need " + std::to_string( bytes ) + " B more, " +
+                            std::to_string( left() ) + " B left" );
+    }
+    uint64_t left()
+    {
+        std::lock_guard<std::mutex> g( mu );
+        return budget > in_use ? budget - in_use : 0;
     }
     void unreserve( uint64_t bytes )
     {
@@ -88,7 +104,13 @@ class DevBuf
             return;
         if ( acct )
             acct->reserve( bytes );
-        const hipError_t e = hipMalloc( &ptr_, bytes );
+        hipError_t e = hipMalloc( &ptr_, bytes );
+        if ( e == hipErrorOutOfMemory && acct && acct->reclaim )
+            acct->reclaim( [&] {
+                (void)hipGetLastError();
+                e = hipMalloc( &ptr_, bytes );
+                return e == hipSuccess;
+            } );
         if ( e != hipSuccess )
         {
             ptr_ = nullptr;
@@ -103,6 +125,23 @@ class DevBuf
         }
         bytes_ = bytes;
         acct_ = acct;
+    }
+    // alloc where the budget and the device have room now, else false.
+    bool allocIfRoom( size_t bytes, MemAccount* acct )
+    {
+        release();
+        if ( bytes == 0 || !acct->tryReserve( bytes ) )
+            return false;
+        if ( hipMalloc( &ptr_, bytes ) != hipSuccess )
+        {
+            (void)hipGetLastError();
+            ptr_ = nullptr;
+            acct->unreserve( bytes );
+            return false;
+        }
+        bytes_ = bytes;
+        acct_ = acct;
+        return true;
     }
     void release()
     {
@@ -294,7 +333,8 @@ const char* lpsKernelName( const PDArgs& a );
 const char* energyKernelName( const PDArgs& a );
 
 // ---- contact (pdk_contact.hip) -----------------------------------------------
-void launchContactForce( const PDArgs* args_dev, const PDArgs& a, int32_t epilogue_mode, hipStream_t st );
+void launchContactForce( const PDArgs* args_dev, const PDArgs& a, int32_t epilogue_mode, int32_t parity,
+                         hipStream_t st );
 const char* contactKernelName( const PDArgs& a );
 
 // ---- region outputs (pdk_output.hip) ----------------------------------------

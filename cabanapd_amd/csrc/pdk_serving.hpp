@@ -44,6 +44,27 @@ struct ContactState
     hipEvent_t disp_ready; // recorded after that copy
 };
 ContactState contactState( pdk_spec_s* s );
+
+// The pair records of a contact specimen (96 B a particle) are held only where
+// memory has room for them: an allocation in the context that finds none takes
+// them back (MemAccount::reclaim).  In scope, this specimen's stay until drop;
+// where wanted() says that another thread waits for them, drop soon.
+class PairRecords
+{
+  public:
+    explicit PairRecords( pdk_spec_s* s ); // makes them if there is room
+    ~PairRecords();
+    PairRecords( const PairRecords& ) = delete;
+    PairRecords& operator=( const PairRecords& ) = delete;
+    bool fresh() const { return fresh_; } // made now: positions not packed yet
+    bool wanted() const;
+    bool drop();                          // give them back now; false if there are none
+
+  private:
+    void setArgs();
+    pdk_spec_s* s_;
+    bool fresh_ = false;
+};
 void contactBuildImpl( pdk_spec_s* s, bool initial, double* max_disp, int64_t* since_build );
 
 // Continuous batching over one device: specs submitted with a step count are

@@ -9,6 +9,7 @@ only Coulomb friction (tanh from the device math library vs libm) is
 compared to a tolerance.
 """
 import math
+import threading
 
 import numpy as np
 import pytest
@@ -226,3 +227,103 @@ def test_gpu_crowded_contacts_bitwise(model, polydisperse):
     for fld in ("u", "v", "f"):
         assert np.array_equal(g.get(fld), o.get(fld)), fld
     g.close()
+
+
+def spheres(n_side, seed, polydisperse=True):
+    """Touching spheres that a short run rebuilds its list for."""
+    r = 1e-3
+    a = np.arange(n_side) * 2.02 * r
+    x = np.stack(np.meshgrid(a, a, a, indexing="ij"), axis=-1).reshape(-1, 3)
+    n = x.shape[0]
+    rng = np.random.default_rng(seed)
+    rad = r * rng.uniform(0.95, 1.05, size=n) if polydisperse else np.full(n, r)
+    desc = configs.make_desc("HERTZ_JKR", radius=r, radius_extend=0.05 * r, nu=0.25, E=7e6, restitution=0.5,
+                             gamma=0.05, dt=1e-6, rebuild_every=4, polydisperse=polydisperse)
+    w = configs._base(desc, x, 4.0 / 3.0 * np.pi * rad ** 3, 2600.0, "spheres", r, 8)
+    w["radius"] = rad if polydisperse else None
+    w["v"] = rng.normal(0.0, 0.3, size=(n, 3))
+    return w
+
+
+def made(c, w):
+    s = engine.Spec(c, w["desc"], w["x"].shape[0])
+    configs.upload(s, w)
+    configs.setup(s, w)
+    return s
+
+
+@pytest.mark.parametrize("polydisperse", [False, True])
+def test_gpu_pair_records_only_where_memory_allows(polydisperse):
+    """The pair records (96 B a sphere) are no part of what a contact specimen
+    needs: a budget without room for them is enough, for two specimens in one
+    context as well, and gives the same bits."""
+    ws = [spheres(22, k, polydisperse) for k in range(2)]
+    n = ws[0]["x"].shape[0]
+
+    def run(c):
+        specs, out, names = [], [], []
+        try:
+            for w in ws:
+                specs.append(made(c, w))
+                specs[0].step(5)   # the first one goes on before and after the second is there
+            specs[1].step(10)
+            for s in specs:
+                out += [s.get(f) for f in ("u", "v", "f")]
+                names.append(s.kernel_name(0))
+            return out, names, c.bytes_in_use()
+        finally:
+            for s in specs:
+                s.close()
+
+    with engine.Context(0) as c:
+        ref, names, used = run(c)
+    assert all(name.endswith("true>") for name in names), names
+    say(f"case: polydisperse={polydisperse}, two specimens of {n} spheres: {used} B with records, {192 * n} B of them")
+    for budget, want in ((used + 4096, {True}), (used - 96 * n + 4096, {True, False}), (used - 192 * n + 4096, {False})):
+        with engine.Context(0, budget) as c:
+            out, names, _ = run(c)
+        assert {name.endswith("true>") for name in names} == want, (budget, names)
+        for a, b in zip(out, ref):
+            assert np.array_equal(a, b)
+
+
+def test_gpu_pair_records_taken_back_by_another_thread():
+    """Two threads, two specimens in one context whose budget holds the records
+    of one at most: creation in one thread takes back the records of the other
+    between its calls or between two steps of one; the results stay."""
+    ws = [spheres(16, k) for k in range(2)]
+    n = ws[0]["x"].shape[0]
+    with engine.Context(0) as c:
+        ref, used = [], []
+        for w in ws:
+            s = made(c, w)
+            s.step(40)
+            ref.append([s.get(f) for f in ("u", "v", "f")])
+            used.append(c.bytes_in_use())
+            s.close()
+    bad = []
+
+    def work(c, k, rounds):
+        try:
+            repeat(c, k, rounds)
+        except engine.PdkError as e:
+            bad.append((k, str(e)))
+
+    def repeat(c, k, rounds):
+        for _ in range(rounds):
+            s = made(c, ws[k])
+            for m in (1, 1, 8, 30):
+                s.step(m)
+            for f, r in zip(("u", "v", "f"), ref[k]):
+                if not np.array_equal(s.get(f), r):
+                    bad.append((k, f))
+            s.close()
+
+    with engine.Context(0, used[0] + used[1] - 150 * n) as c:
+        th = [threading.Thread(target=work, args=(c, k, 12)) for k in range(2)]
+        for t in th:
+            t.start()
+        for t in th:
+            t.join()
+    say(f"case: two threads, {n} spheres each, records taken back: {bad}")
+    assert not bad
