@@ -298,6 +298,11 @@ struct pdk_spec_s
         return !gatherOnly() || rowFeaturesSupported( d.model, pair_tables, d.thermal != PDK_TEMP_INDEPENDENT,
                                                       d.mechanics == PDK_MECH_EPP );
     }
+    BondForm bondForm() const
+    {
+        return { slice_ptr.as<int64_t>(), cnt.as<int32_t>(), col.as<int32_t>(),
+                 slot.slots > 0 ? slot.exist.as<uint64_t>() : nullptr, intact.as<uint64_t>(), splas.as<double>() };
+    }
     bool hasPrescribed() const { return pre_u.count > 0 || pre_temp.count > 0; }
     bool dynamicTemp() const { return d.thermal == PDK_TEMP_DYNAMIC; }
     // Work between the initial half step and the force pass of step g:
@@ -1266,9 +1271,12 @@ int pdk_spec_copy_state( pdk_spec dst, pdk_spec src )
         require( dst->d.model == src->d.model && dst->d.fracture == src->d.fracture &&
                      dst->d.mechanics == src->d.mechanics && dst->d.thermal == src->d.thermal,
                  "specs differ in model" );
-        require( dst->slot.slots == src->slot.slots && dst->total_rows == src->total_rows &&
-                     dst->intact.bytes() == src->intact.bytes() && dst->col.bytes() == src->col.bytes(),
-                 "specs differ in bond layout" );
+        const bool same = dst->slot.slots == src->slot.slots && dst->total_rows == src->total_rows &&
+                          dst->intact.bytes() == src->intact.bytes() && dst->col.bytes() == src->col.bytes();
+        // the same layout asked for, but one build had no room for the slot form
+        const bool convert = !same && dst->d.bond_layout == src->d.bond_layout &&
+                             ( dst->slot.slots > 0 ) != ( src->slot.slots > 0 );
+        require( same || convert, "specs differ in bond layout" );
         const size_t v3 = 3 * static_cast<size_t>( src->n ) * sizeof( double );
         const size_t v1 = static_cast<size_t>( src->n ) * sizeof( double );
         // src's stream must be done with its state before dst's copies read it
@@ -1277,10 +1285,19 @@ int pdk_spec_copy_state( pdk_spec dst, pdk_spec src )
             if ( a && b && bytes )
                 PDK_HIP( hipMemcpyAsync( a.as<void>(), b.as<void>(), bytes, hipMemcpyDeviceToDevice, dst->st ) );
         };
+        if ( convert )
+            require( copyBondState( dst->n, dst->bondForm(), dst->total_rows, src->bondForm(), dst->scratch,
+                                    dst->acct(), dst->st ),
+                     "specs differ in bond layout" );
+        else
+        {
+            copy( dst->intact, src->intact, src->intact.bytes() );
+            if ( dst->splas && src->splas && dst->splas.bytes() == src->splas.bytes() )
+                copy( dst->splas, src->splas, src->splas.bytes() );
+        }
         PDK_HIP( hipMemcpyAsync( dst->Ucur(), src->Ucur(), v3, hipMemcpyDeviceToDevice, dst->st ) );
         copy( dst->v, src->v, v3 );
         copy( dst->f, src->f, v3 );
-        copy( dst->intact, src->intact, src->intact.bytes() );
         copy( dst->W, src->W, v1 );
         copy( dst->phi, src->phi, v1 );
         copy( dst->m, src->m, v1 );
@@ -1288,8 +1305,6 @@ int pdk_spec_copy_state( pdk_spec dst, pdk_spec src )
         copy( dst->lpsA, src->lpsA, v1 );
         copy( dst->lpsB, src->lpsB, v1 );
         copy( dst->temp, src->temp, v1 );
-        if ( dst->splas && src->splas && dst->splas.bytes() == src->splas.bytes() )
-            copy( dst->splas, src->splas, src->splas.bytes() );
         dst->steps_done = src->steps_done;
         dst->inited = true;
         PDK_HIP( hipStreamSynchronize( dst->st ) );

@@ -805,6 +805,62 @@ __global__ __launch_bounds__( kThreads ) void kFillHoleSlots( int64_t n, int64_t
     }
 }
 
+// ---- Bond state from one form to the other -----------------------------------
+// The next bond of a particle's row in slot order: compact rows hold bonds
+// only, slot rows one bond or none per slot.
+struct BondWalk
+{
+    const BondForm& F;
+    int64_t row, end;
+    int lane;
+    __device__ BondWalk( const BondForm& f, int64_t p ) : F( f ), lane( static_cast<int>( p % kSlice ) )
+    {
+        row = F.slice_ptr[p / kSlice];
+        end = F.exist ? F.slice_ptr[p / kSlice + 1] : row + F.cnt[p];
+    }
+    __device__ bool next( int64_t& r )
+    {
+        while ( row < end && F.exist && !( ( F.exist[row] >> lane ) & 1ull ) )
+            row++;
+        r = row++;
+        return r < end;
+    }
+};
+__global__ __launch_bounds__( kThreads ) void kCompareBonds( int64_t n, BondForm a, BondForm b,
+                                                             int32_t* __restrict__ flag )
+{
+    const int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if ( p >= n )
+        return;
+    BondWalk wa( a, p ), wb( b, p );
+    int64_t ra, rb;
+    bool more = wa.next( ra ), same = more == wb.next( rb );
+    while ( more && same )
+    {
+        same = a.col[ra * kSlice + wa.lane] == b.col[rb * kSlice + wb.lane];
+        more = wa.next( ra );
+        same = same && more == wb.next( rb );
+    }
+    if ( !same )
+        *flag = 1;
+}
+// (dst's words and stretches are zero before)
+__global__ __launch_bounds__( kThreads ) void kCopyBondState( int64_t n, BondForm dst, BondForm src )
+{
+    const int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if ( p >= n )
+        return;
+    BondWalk wd( dst, p ), ws( src, p );
+    int64_t rd, rs;
+    while ( wd.next( rd ) && ws.next( rs ) )
+    {
+        if ( ( src.intact[rs] >> ws.lane ) & 1ull )
+            atomicOr( reinterpret_cast<unsigned long long*>( dst.intact + rd ), 1ull << wd.lane );
+        if ( dst.splas && src.splas )
+            dst.splas[rd * kSlice + wd.lane] = src.splas[rs * kSlice + ws.lane];
+    }
+}
+
 template <class T>
 void ensure( DevBuf& b, size_t count, MemAccount* acct )
 {
@@ -1578,6 +1634,26 @@ bool buildStencilSlotsDirect( const double* x_dev, int64_t n, const int64_t dims
         return false;
     return finishSlots( n, ( n + kSlice - 1 ) / kSlice, L, es, dent.as<int4>(), h, col, intact, slice_ptr_dev,
                         total_rows, col_capacity_rows, out, acct, st );
+}
+
+bool copyBondState( int64_t n, const BondForm& dst, int64_t dst_rows, const BondForm& src, BuildScratch& s,
+                    MemAccount* acct, hipStream_t st )
+{
+    ensure<int32_t>( s.flag, 1, acct );
+    PDK_HIP( hipMemsetAsync( s.flag.as<int32_t>(), 0, sizeof( int32_t ), st ) );
+    kCompareBonds<<<gridFor( n ), kThreads, 0, st>>>( n, dst, src, s.flag.as<int32_t>() );
+    PDK_HIP( hipGetLastError() );
+    int32_t flag = 0;
+    PDK_HIP( hipMemcpyAsync( &flag, s.flag.as<int32_t>(), sizeof( int32_t ), hipMemcpyDeviceToHost, st ) );
+    PDK_HIP( hipStreamSynchronize( st ) );
+    if ( flag )
+        return false;
+    PDK_HIP( hipMemsetAsync( dst.intact, 0, dst_rows * sizeof( uint64_t ), st ) );
+    if ( dst.splas && src.splas )
+        PDK_HIP( hipMemsetAsync( dst.splas, 0, dst_rows * kSlice * sizeof( double ), st ) );
+    kCopyBondState<<<gridFor( n ), kThreads, 0, st>>>( n, dst, src );
+    PDK_HIP( hipGetLastError() );
+    return true;
 }
 
 void launchPrenotch( const PDArgs& a, int32_t nnotch, const double* notch_dev, hipStream_t st )

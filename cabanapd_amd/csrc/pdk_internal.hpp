@@ -215,6 +215,20 @@ struct SlotForm
     bool hole = false;
     DevBuf hole_win, hole_pos;
 };
+// A specimen's bonds and their state in either form (exist null: compact).
+struct BondForm
+{
+    const int64_t* slice_ptr;
+    const int32_t* cnt;
+    const int32_t* col;
+    const uint64_t* exist;
+    uint64_t* intact;
+    double* splas;
+};
+// dst's intact bits and plastic stretches from src's, bond by bond; false
+// (nothing written) when the bonds differ.
+bool copyBondState( int64_t n, const BondForm& dst, int64_t dst_rows, const BondForm& src, BuildScratch& s,
+                    MemAccount* acct, hipStream_t st );
 bool buildStencilSlots( const PDArgs& a, const int64_t dims[3], const double h[3], double rc,
                         const std::vector<int64_t>& perm_host, DevBuf& col, DevBuf& intact, int64_t* slice_ptr_dev,
                         int64_t& total_rows, int64_t& col_capacity_rows, SlotForm& out, BuildScratch& s,

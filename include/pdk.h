@@ -140,8 +140,10 @@ enum pdk_ordering {
 
 enum pdk_bond_layout {
     PDK_BONDS_AUTO = 0,     /* stencil slots on full lattices (neighbor ids computed, not stored) and on most
-                               lattices with missing sites, else compact */
-    PDK_BONDS_COMPACT = 1   /* always the compact form: one stored neighbor id per bond */
+                               lattices with missing sites, else compact; also compact where the HBM budget
+                               has no room for the slot form beside it during the build */
+    PDK_BONDS_COMPACT = 1   /* always the compact form: one stored neighbor id per bond; the smaller one, by a tenth
+                               on lattices with few sites missing, by far on sparse ones */
 };
 
 /* Derived constants, for inspection and tests. */
@@ -197,7 +199,8 @@ int pdk_spec_set_state(pdk_spec spec, const double* u, const double* v);
  * device.  No counterpart in the reference (a Solver is never forked); it lets
  * one state be advanced in both precision forms.  The specs must share the
  * context, the particle count and device order, the model and the bond
- * layout (same positions, same build); their precision may differ.  dst must
+ * layout asked for (same positions, same build); their precision may differ,
+ * and under PDK_BONDS_AUTO the form that memory left room for.  dst must
  * have its bonds built; it counts as initialised afterwards. */
 int pdk_spec_copy_state(pdk_spec dst, pdk_spec src);
 int pdk_spec_bytes(pdk_spec spec, uint64_t* bytes);

@@ -361,3 +361,53 @@ def test_tight_budgets_hold_the_whole_run(shape, kind):
         seen.add("Rows" in auto[2])
     say(f"case: {shape} {kind}, {n} particles: row windows chosen over the budgets: {sorted(seen)}")
     assert seen == {False, True}
+
+
+@pytest.mark.parametrize("kind", ["pmb", "lps", "epp", "whole horizon"])
+def test_copy_state_between_the_forms_memory_left(kind):
+    """Two identical specimens of which the second finds no room for the slot
+    form: state is copied both ways (broken bonds, plastic stretches), and each
+    goes on with the other's bits.  Layouts asked for differently stay refused."""
+    dims, keep = SHAPES["hole"]
+    w = box("LPS" if kind == "lps" else "PMB", dims, 3 if kind == "whole horizon" else 3.01, True)
+    if kind != "whole horizon":
+        cut(w, dims, keep)
+    d = w["desc"]
+    if kind == "epp":
+        d.mechanics, d.sigma_y = 1, 2.5e7
+    n = w["x"].shape[0]
+
+    def made(c, layout=0):
+        d.bond_layout = layout
+        s = engine.Spec(c, d, n)
+        configs.upload(s, w)
+        configs.setup(s, w)
+        return s
+
+    with engine.Context(0) as c:
+        a = made(c)
+        one = c.bytes_in_use()
+        b = made(c, PDK_BONDS_COMPACT)
+        two = c.bytes_in_use()
+        assert "Rows" in a.kernel_name(0) and "Rows" not in b.kernel_name(0)
+        with pytest.raises(engine.PdkError):
+            b.copy_state_from(a)
+        a.close()
+        b.close()
+    with engine.Context(0, two + 150 * n) as c:
+        a, b = made(c), made(c)
+        say(f"case: {kind}, {n} particles: {one} and {two - one} B; {a.kernel_name(0)} and {b.kernel_name(0)}")
+        assert "Rows" in a.kernel_name(0) and "Rows" not in b.kernel_name(0)
+        for src, dst in ((a, b), (b, a)):
+            src.step(6)
+            dst.copy_state_from(src)
+            for k in range(3):
+                assert np.array_equal(src.bonds()[k], dst.bonds()[k])
+            assert (src.bonds()[2] == 0).any()
+            src.step(5)
+            dst.step(5)
+            for f in ("u", "v", "f"):
+                assert np.array_equal(src.get(f), dst.get(f)), f
+            src.step(2)
+        a.close()
+        b.close()
