@@ -2307,8 +2307,7 @@ int pdk_set_tuning( pdk_spec s, int32_t unroll )
                  "unroll must be 0 (row windows), 1, 2, 4 or 8" );
         require( unroll != 0 || s->rowsCover(),
                  "this combination of materials, EPP and temperature dependence uses the gather variant" );
-        require( unroll != 0 || !s->built || ( s->slot.nrows > 0 && !s->slot.hole ),
-                 "row windows need the stencil-slot layout of a full lattice" );
+        require( unroll != 0 || !s->built || s->slot.nrows > 0, "row windows need the stencil-slot layout of a lattice" );
         s->unroll = unroll;
         if ( s->uploaded )
         {

@@ -424,8 +424,8 @@ int pdk_compute_energy_noalloc(pdk_spec spec, double* total_strain_energy, doubl
 
 /* ---- tuning --------------------------------------------------------------------
  * Force-pass variant: unroll = 1, 2, 4 or 8 gathers the neighbor data of that
- * many bond slots per group; unroll = 0 (full lattices in the stencil-slot
- * layout only; the default on lattices with missing sites in it) stages
+ * many bond slots per group; unroll = 0 (lattices in the stencil-slot form
+ * only, full or with missing sites) stages
  * the neighbor data of each lattice row window in LDS instead (also for
  * several materials, or a temperature-dependent and/or ElasticPerfectlyPlastic
  * PMB; several materials together with either, and the linearized models
@@ -442,8 +442,8 @@ int pdk_set_tuning(pdk_spec spec, int32_t unroll);
  * the stencil-slot form of a full lattice (slot q of every row is stencil
  * entry q, neighbor ids are offsets), 0 for the compact form and for the slot
  * form that lattices with missing sites take where they can (neighbor ids
- * stored; its default force pass is the row-window one too, and pdk_set_tuning
- * selects the gathers over it).  Any pointer may be NULL. */
+ * stored, row windows all the same; pdk_kernel_name tells it from the compact
+ * form).  Any pointer may be NULL. */
 int pdk_spec_layout(pdk_spec spec, int32_t* lattice_rows, int32_t* stencil_entries, int32_t* stencil_slots);
 int pdk_autotune(pdk_spec spec, int32_t launches_per_candidate, int32_t* unroll_out);
 /* enable = 1: pdk_step replays the launches of two consecutive steps as one

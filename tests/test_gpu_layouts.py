@@ -411,3 +411,38 @@ def test_copy_state_between_the_forms_memory_left(kind):
             src.step(2)
         a.close()
         b.close()
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+def test_row_windows_can_be_chosen_on_missing_sites(precision):
+    """Every pass that pdk_autotune may choose can be set, the row windows of a
+    lattice with missing sites as well, before and after the gathers; a
+    specimen in the compact form still refuses them."""
+    dims, keep = SHAPES["hole"]
+    w = cut(box("PMB", dims, 3.01, True), dims, keep)
+    w["desc"].precision = precision
+    out, names = [], []
+    for tune in ((), (4,), (4, 0), (0,)):
+        s = engine.Spec(ctx(), w["desc"], w["x"].shape[0])
+        configs.upload(s, w)
+        configs.setup(s, w)
+        for t in tune:
+            s.set_tuning(t)
+        s.step(6)
+        out.append([s.get(f) for f in ("u", "v", "f")])
+        names.append(s.kernel_name(0))
+        best = s.autotune()
+        s.set_tuning(best)
+        s.close()
+    say(f"case: missing sites, precision {precision}: {names}")
+    assert names[2] == names[3] == names[0] and "Rows" in names[0] and "Rows" not in names[1]
+    for o in out[1:]:
+        for a, b in zip(out[0], o):
+            assert np.array_equal(a, b)
+    w["desc"].bond_layout = PDK_BONDS_COMPACT
+    s = engine.Spec(ctx(), w["desc"], w["x"].shape[0])
+    configs.upload(s, w)
+    configs.setup(s, w)
+    with pytest.raises(engine.PdkError):
+        s.set_tuning(0)
+    s.close()
