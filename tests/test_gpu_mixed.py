@@ -8,7 +8,7 @@ import numpy as np
 import pytest
 
 from cabanapd_amd import configs, engine
-from cabanapd_amd._abi import make_desc
+from cabanapd_amd._abi import PDK_BONDS_COMPACT, make_desc
 from tests.parity import ctx, pair, rel_err, say
 
 pytestmark = pytest.mark.gpu
@@ -282,9 +282,11 @@ def test_holed_lattice_compact_stencil():
     form gathering x_j (Morton order)."""
     say("case: PMB plate 30x60x7 with a hole of radius 6 cells, FP64 vs oracle, mixed vs FP64, 80 steps")
     w = _holed_plate()
+    w["desc"].bond_layout = PDK_BONDS_COMPACT
     g, o = pair(w)
     say(f"  particles {w['x'].shape[0]}, FP64 layout {g.layout()}")
     assert g.layout()["lattice_rows"] and not g.layout()["stencil_slots"]
+    assert g.kernel_name(0).startswith("kForce<")
     g.step(80)
     o.step(80)
     for fld in ("u", "v", "f"):
@@ -303,6 +305,7 @@ def test_holed_lattice_compact_stencil():
         say(f"  mixed {name}: {lay} {s.kernel_name(0)}")
         if order == 2:
             assert lay["stencil_entries"] == 122 and not lay["stencil_slots"]
+            assert s.kernel_name(0).startswith("kForce<")
         s.step(80)
         res[name] = (s.get("u"), s.bonds()[2])
         s.close()
@@ -328,9 +331,11 @@ def test_holed_lps_cube_compact_stencil():
     keep = np.sum((w["x"] - 0.5) ** 2, axis=1) > (4 * dx) ** 2
     for k in ("x", "vol", "rho", "u", "v", "body"):
         w[k] = np.ascontiguousarray(w[k][keep])
+    w["desc"].bond_layout = PDK_BONDS_COMPACT
     g, o = pair(w)
     say(f"  particles {w['x'].shape[0]}, FP64 layout {g.layout()}")
     assert g.layout()["lattice_rows"] and not g.layout()["stencil_slots"]
+    assert g.kernel_name(0).startswith("kForce<") and g.kernel_name(1).startswith("kLpsState<")
     g.step(40)
     o.step(40)
     for fld in ("u", "v", "f", "m", "theta"):
@@ -349,6 +354,7 @@ def test_holed_lps_cube_compact_stencil():
         say(f"  mixed {name}: {lay} {s.kernel_name(0)}")
         if order == 2:
             assert lay["stencil_entries"] > 0 and not lay["stencil_slots"]
+            assert s.kernel_name(0).startswith("kForce<")
         s.step(40)
         res[name] = s.get("u")
         s.close()
