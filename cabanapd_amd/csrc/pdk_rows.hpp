@@ -303,11 +303,13 @@ __device__ __forceinline__ void linearized32g( double xi0, double xi1, double xi
 //     finds every divisor whose low word is all ones.
 // A row in which a lane fails one of them is evaluated again by the general
 // code, from the sums as they were before the row.
-// (checked on the GPU against IEEE results: 1e8 roots and quotients, half of
-// them with mantissas within 16 ulp of a power of two, no difference but for
-// the excluded divisors.  The PMB fracture slot takes 75 VALU instructions;
-// 25 steps of the 1.44M-particle plate with their download 28.2 -> 23.6 ms,
-// 50 steps of a 41^3 cube 4.23 -> 3.52 ms, with the LPS model 8.50 -> 7.48.)
+// (1e8 random roots and quotients, half of them with mantissas within 16 ulp
+// of a power of two, were compared with IEEE results once, with no difference
+// but for the excluded divisors; the extreme-value tests compare specimens whose
+// bonds are of such lengths with the oracle.  The PMB fracture slot takes 75
+// VALU instructions; 25 steps of the 1.44M-particle plate with their download
+// 28.2 -> 23.6 ms, 50 steps of a 41^3 cube 4.23 -> 3.52 ms, with the LPS model
+// 8.50 -> 7.48.)
 // ---------------------------------------------------------------------------
 constexpr int kPlainHigh = 100;  // staged u and T: zero or 2^-plain_low <= |.| < 2^100
 constexpr int kPlainExpAB = 200; // staged lpsA, lpsB: zero or 2^-200 <= |.| < 2^200
@@ -591,9 +593,10 @@ __device__ __forceinline__ double addRound( const SplitTerms<W, ND, NF>& T, int 
 // data from three to twelve scattered loads: 100 mixed steps of a 423k-particle
 // perforated plate 26.5 -> 11.0 ms, 100 FP64 elastic-plastic steps of a 29k
 // dogbone 14.2 -> 5.3 ms (4.3 with slots together).
-// G: slots evaluated together (1: one after the other).  Five in split launches
-// in FP64.  With one wave per slice five gave 47 -> 41 us on small specimens and
-// nothing from 2000 slices on; the mixed form got slower.
+// G: slots evaluated together (1: one after the other).  Five in split
+// launches, in both precisions.  With one wave per slice five gave 47 -> 41 us
+// in FP64 on small specimens and nothing from 2000 slices on; the mixed form got
+// slower.
 template <int MODEL, bool FRAC, int PREC, bool GEN, int W = 1, bool HOLE = false, int G = 1>
 __global__ __launch_bounds__( W == 1 ? kBlock : W * kSlice ) __attribute__( ( amdgpu_waves_per_eu( ( MODEL == 1 || MODEL == 5 || G > 1 ) ? 1 : 6, 8 ) ) ) void
 kForceRows( const PDArgs* __restrict__ specs,
@@ -1193,14 +1196,7 @@ kForceRows( const PDArgs* __restrict__ specs,
                     const double cy = divBy( coeff[g] * b[g].ry, b[g].r, b[g].yr );
                     const double cz = divBy( coeff[g] * b[g].rz, b[g].r, b[g].yr );
                     const bool live = __builtin_amdgcn_inverse_ballot_w64( ww[g] & ~brkm[g] );
-                    if constexpr ( W > 1 )
-                        put( t0 + g, live ? cx : -0.0, live ? cy : -0.0, live ? cz : -0.0 );
-                    else
-                    {
-                        fx += live ? cx : -0.0;
-                        fy += live ? cy : -0.0;
-                        fz += live ? cz : -0.0;
-                    }
+                    put( t0 + g, live ? cx : -0.0, live ? cy : -0.0, live ? cz : -0.0 );
                 }
             }
             else
@@ -1239,18 +1235,8 @@ kForceRows( const PDArgs* __restrict__ specs,
                                  b[g].rinv;
                         }
                         fr = __builtin_amdgcn_inverse_ballot_w64( ww[g] ) ? fr : 0.0f;
-                        if constexpr ( W > 1 )
-                        {
-                            put( t0 + g, r0[g], r1[g], r2[g] );
-                            putFactor( t0 + g, fr );
-                        }
-                        else
-                        {
-                            const double frd = static_cast<double>( fr );
-                            sx = fma( frd, r0[g], sx );
-                            sy = fma( frd, r1[g], sy );
-                            sz = fma( frd, r2[g], sz );
-                        }
+                        put( t0 + g, r0[g], r1[g], r2[g] );
+                        putFactor( t0 + g, fr );
                     }
                 }
             }

@@ -146,3 +146,42 @@ def test_fading_displacements_keep_the_fast_rows(model):
     say(f"case: {model}, {n} particles, force pass {best['full']:.4f} ms, with tails {best['tails']:.4f} ms")
     assert best["tails"] < 1.25 * best["full"]
     s.close()
+
+
+@pytest.mark.parametrize("where", ["current", "reference", "both"])
+@pytest.mark.parametrize("model", ["PMB", "LPS"])
+def test_lengths_near_powers_of_two_match_oracle(model, where):
+    """Bond lengths (current, reference) within 16 ulp of powers of two, where
+    a reciprocal's last bit is the hardest: roots and quotients of 3e6 bonds
+    through the shared reciprocals, the oracle's bits."""
+    n_side = 29
+    ulp = 2.0 ** -58  # of the doubles from 1/64 on; half as much below
+    x, vol, _ = configs.grid_node_centred(n_side, H)
+    n = x.shape[0]
+    rng = np.random.default_rng(11)
+    u = rng.uniform(-1, 1, size=(n, 3)) * 1e-9 * H
+    if where in ("current", "both"):
+        u[:, 0] = rng.integers(-16, 17, size=n) * ulp / 2
+    else:
+        u[:, 0] += rng.uniform(-1, 1, size=n) * 1e-4 * H
+    if where in ("reference", "both"):
+        x[:, 0] += rng.integers(-8, 9, size=n) * np.spacing(np.maximum(x[:, 0], H))
+    kw = dict(horizon=3.01 * H, K=2e9, dt=1e-9)
+    if model == "LPS":
+        kw.update(G=1.1e9, influence=0)
+    w = configs._base(make_desc(model, **kw), x, vol, 1000.0, "near_powers", H, 2)
+    w["u"] = u
+    g, o = pair(w)
+    say(f"case: {model}, {where} lengths near powers of two, {n} particles, {g.bond_stats()[0]} bonds, "
+        f"{g.kernel_name(0)}")
+    assert "Rows" in g.kernel_name(0)
+    for fld in ("f", "W") + (("m", "theta") if model == "LPS" else ()):
+        same(g.get(fld), o.get(fld), fld + " at init")
+    g.compute_stress()
+    o.compute_stress()
+    same(g.get("stress"), o.get("stress"), "stress")
+    g.step(2)
+    o.step(2)
+    for fld in ("u", "v", "f"):
+        same(g.get(fld), o.get(fld), fld)
+    g.close()
