@@ -1319,7 +1319,10 @@ int pdk_spec_bytes( pdk_spec s, uint64_t* bytes )
         for ( const DevBuf* b : { &s->x, &s->U0, &s->U1, &s->v, &s->f, &s->vol, &s->rho, &s->nofail, &s->bcflag,
                                   &s->body, &s->m, &s->theta, &s->lpsA, &s->lpsB, &s->W, &s->phi, &s->perm, &s->inv,
                                   &s->cnt, &s->slice_ptr, &s->col, &s->intact, &s->radius, &s->u_neigh,
-                                  &s->partial, &s->args, &s->sid, &s->stab, &s->stab_xi2d, &s->stab_xiv } )
+                                  &s->partial, &s->args, &s->sid, &s->stab, &s->stab_xi2d, &s->stab_xiv,
+                                  &s->slot.exist, &s->slot.soff, &s->slot.table, &s->slot.xi2d, &s->slot.xiv,
+                                  &s->slot.rows, &s->slot.rowstart, &s->slot.aux, &s->slot.rec, &s->slot.hole_win,
+                                  &s->slot.hole_pos } )
             t += b->bytes();
         t += s->rec_bytes;
         *bytes = t;

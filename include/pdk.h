@@ -142,8 +142,8 @@ enum pdk_bond_layout {
     PDK_BONDS_AUTO = 0,     /* stencil slots on full lattices (neighbor ids computed, not stored) and on most
                                lattices with missing sites, else compact; also compact where the HBM budget
                                has no room for the slot form beside it during the build */
-    PDK_BONDS_COMPACT = 1   /* always the compact form: one stored neighbor id per bond; the smaller one, by a tenth
-                               on lattices with few sites missing, by far on sparse ones */
+    PDK_BONDS_COMPACT = 1   /* always the compact form: one stored neighbor id per bond; in FP64 the smaller one, by a
+                               tenth to a fifth on most specimens, by far on sparse ones */
 };
 
 /* Derived constants, for inspection and tests. */

@@ -446,3 +446,26 @@ def test_row_windows_can_be_chosen_on_missing_sites(precision):
     with pytest.raises(engine.PdkError):
         s.set_tuning(0)
     s.close()
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+def test_spec_bytes_hold_the_forms_tables(precision):
+    """What a specimen reports to hold differs between the forms by what its
+    context has in use."""
+    dims, keep = SHAPES["hole"]
+    for w in (cut(box("PMB", dims, 3.01, True), dims, keep), box("PMB", (40, 31, 6), 3, True)):
+        d = w["desc"]
+        d.precision = precision
+        held, used = [], []
+        for layout in (0, PDK_BONDS_COMPACT):
+            d.bond_layout = layout
+            with engine.Context(0) as c:
+                s = engine.Spec(c, d, w["x"].shape[0])
+                configs.upload(s, w)
+                configs.setup(s, w)
+                held.append(s.bytes())
+                used.append(c.bytes_in_use())
+                s.close()
+        say(f"case: precision {precision}, {w['x'].shape[0]} particles: held {held}, in use {used}")
+        assert held[0] != held[1]
+        assert abs((held[0] - held[1]) - (used[0] - used[1])) <= 4096
