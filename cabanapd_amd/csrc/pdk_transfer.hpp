@@ -15,6 +15,7 @@
 #define PDK_TRANSFER_HPP
 
 #include <atomic>
+#include <chrono>
 #include <condition_variable>
 #include <cstring>
 #include <functional>
@@ -55,12 +56,17 @@ class HostTransfer
     }
 
     // dst (host) <- src (device) after the work queued on st; complete on return.
+    // That work is waited for here, before the context's slots are taken and
+    // before a chunk is queued: a queued copy holds its DMA engine until its
+    // stream gets there, and other specimens' copies with it.  The workers are
+    // woken meanwhile (waiting first made a 34.6 MB copy 20 us longer without).
     void out( void* dst, const void* src, size_t bytes, hipStream_t st )
     {
-        // The work queued on st is waited for here, before the context's
-        // slots are taken: other specimens' copies go on meanwhile.
         if ( bytes >= kDirect )
+        {
+            rouse();
             PDK_HIP( hipStreamSynchronize( st ) );
+        }
         if ( bytes < kDirect || !run( bytes, [=]( Slot& s, size_t off, size_t len ) {
             hipError_t e = hipMemcpyAsync( s.mem, static_cast<const char*>( src ) + off, len, hipMemcpyDeviceToHost, st );
             if ( e == hipSuccess )
@@ -122,17 +128,29 @@ class HostTransfer
     {
         if ( hipSetDevice( device_ ) != hipSuccess )
             return;
-        uint64_t seen = 0;
+        uint64_t seen = 0, roused = 0;
         for ( ;; )
         {
             std::shared_ptr<Job> j;
+            bool soon = false;
             {
                 std::unique_lock<std::mutex> g( job_mu_ );
-                wake_.wait( g, [&] { return stop_ || generation_ != seen; } );
+                wake_.wait( g, [&] { return stop_ || generation_ != seen || roused_ != roused; } );
                 if ( stop_ )
                     return;
-                seen = generation_;
-                j = job_;
+                soon = generation_ == seen;
+                roused = roused_;
+                if ( !soon )
+                {
+                    seen = generation_;
+                    j = job_;
+                }
+            }
+            if ( soon ) // stay awake for it, for 100 us at most
+            {
+                const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds( 100 );
+                while ( generation_ == seen && std::chrono::steady_clock::now() < until )
+                    std::this_thread::yield();
             }
             if ( j )
                 take( *j, slots_[t] );
@@ -162,6 +180,16 @@ class HostTransfer
             }
         }
         return true;
+    }
+
+    // A copy is about to come.
+    void rouse()
+    {
+        {
+            std::lock_guard<std::mutex> g( job_mu_ );
+            roused_++;
+        }
+        wake_.notify_all();
     }
 
     // False, with nothing copied, where there are no slots.
@@ -206,10 +234,11 @@ class HostTransfer
     std::mutex mu_;
     Slot slots_[kSlots];
     std::vector<std::thread> workers_;
-    std::mutex job_mu_; // job_, generation_, stop_ and the jobs' done counts
+    std::mutex job_mu_; // job_, generation_, roused_, stop_ and the jobs' done counts
     std::condition_variable wake_, finished_;
     std::shared_ptr<Job> job_;
-    uint64_t generation_ = 0;
+    std::atomic<uint64_t> generation_{ 0 }; // written under job_mu_
+    uint64_t roused_ = 0;
     bool stop_ = false;
 };
 } // namespace pdk
