@@ -803,7 +803,7 @@ bool pdk_ctx_s::reclaimRecords( const std::function<bool()>& fits )
                 pdk_spec s = rec_holders[k];
                 if ( s->rec_busy.exchange( true ) )
                     continue;
-                // (every call that uses them waits for its launches before it returns)
+                (void)hipStreamSynchronize( s->st ); // what its last call launched
                 s->pair_rec.release();
                 s->rec_bytes = 0;
                 rec_holders.erase( rec_holders.begin() + k );

@@ -639,8 +639,6 @@ void contactForceStore( pdk_spec_s* s )
         launchContactPack( v.dargs, *v.h, *v.cur, v.st );
         launchContactForce( v.dargs, *v.h, kEpiStoreOnly, *v.cur, v.st );
     } );
-    // the records may be taken back once this returns
-    PDK_HIP( hipStreamSynchronize( v.st ) );
 }
 
 void contactStep( pdk_spec_s* s, int32_t nsteps )
@@ -698,8 +696,6 @@ void contactStep( pdk_spec_s* s, int32_t nsteps )
     }
     SpecView v = view( s );
     specTimed( s, 4, [&] { launchContactFinal( v.dargs, *v.h, v.st ); } );
-    // the records may be taken back once this returns
-    PDK_HIP( hipStreamSynchronize( v.st ) );
 }
 
 } // namespace pdk
