@@ -1307,7 +1307,10 @@ __global__ __launch_bounds__( kBlock ) void kStressRows( const PDArgs* __restric
         S.s12 += fy * xi_z;
         S.s21 += fz * xi_y;
     };
-    const int plain_low = kIsLin<MODEL> ? 0 : scalarLoad( &A.plain_low );
+    // (with a plastic stretch the general code is the faster one: its load
+    // and store per slot come behind the longer chain of the shared reciprocals;
+    // 19k particles 94 against 114 us, 373k 283 against 301)
+    const int plain_low = kIsLin<MODEL> || EP ? 0 : scalarLoad( &A.plain_low );
     const bool plain = plain_low != 0;
     int own_lo = 0, own_hi = 0, own_la = 0, own_ha = 0;
     expRange( ui0, own_lo, own_hi );

@@ -1588,7 +1588,7 @@ __global__ __launch_bounds__( W == 1 ? kBlock : W * kSlice ) __attribute__( ( am
     };
 
     // FP64: rows of ordinary values take the shared reciprocals (see kForceRows)
-    constexpr bool FAST = ( PREC == kF64 );
+    constexpr bool FAST = ( PREC == kF64 ) && !( TH && EP && W == 1 );
     const int plain_low = FAST ? scalarLoad( &A.plain_low ) : 0;
     const bool plain = plain_low != 0;
     int own_lo = 0, own_hi = 0;
@@ -2043,29 +2043,32 @@ __global__ __launch_bounds__( W == 1 ? kBlock : W * kSlice ) __attribute__( ( am
         }
         else
         {
-            if ( plain )
+            if constexpr ( FAST )
             {
-                const double fx0 = fx, fy0 = fy, fz0 = fz;
-                uint64_t bad = 0;
-                if constexpr ( W > 1 )
+                if ( plain )
                 {
-                    int t = 0;
-                    for ( ; t + 5 <= R.y; t += 5 )
-                        bad |= groupFast( std::integral_constant<int, 5>{}, t, limit );
-                    for ( ; t + 3 <= R.y; t += 3 )
-                        bad |= groupFast( std::integral_constant<int, 3>{}, t, limit );
-                    for ( ; t < R.y; t++ )
-                        bad |= groupFast( std::integral_constant<int, 1>{}, t, limit );
+                    const double fx0 = fx, fy0 = fy, fz0 = fz;
+                    uint64_t bad = 0;
+                    if constexpr ( W > 1 )
+                    {
+                        int t = 0;
+                        for ( ; t + 5 <= R.y; t += 5 )
+                            bad |= groupFast( std::integral_constant<int, 5>{}, t, limit );
+                        for ( ; t + 3 <= R.y; t += 3 )
+                            bad |= groupFast( std::integral_constant<int, 3>{}, t, limit );
+                        for ( ; t < R.y; t++ )
+                            bad |= groupFast( std::integral_constant<int, 1>{}, t, limit );
+                    }
+                    else
+                        for ( int t = 0; t < R.y; t++ )
+                            bad |= slotFast( t, limit );
+                    if ( __builtin_expect( bad == 0, 1 ) )
+                        return;
+                    fx = fx0;
+                    fy = fy0;
+                    fz = fz0;
+                    pos = pos0;
                 }
-                else
-                    for ( int t = 0; t < R.y; t++ )
-                        bad |= slotFast( t, limit );
-                if ( __builtin_expect( bad == 0, 1 ) )
-                    return;
-                fx = fx0;
-                fy = fy0;
-                fz = fz0;
-                pos = pos0;
             }
             for ( int t = 0; t < R.y; t++ )
                 slot( t );
