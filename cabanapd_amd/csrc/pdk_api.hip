@@ -249,7 +249,7 @@ struct pdk_spec_s
     bool uploaded = false, built = false, inited = false;
     bool lattice_rows = false; // device order is lattice rows (else Morton)
     int32_t unroll = -1;       // force-pass variant (tuning knob): -1 default, 0 row windows, 1/2/4/8 gathers
-    bool coords_plain = false; // every coordinate is zero or within [2^-100, 2^100)
+    bool coords_plain = false; // a lattice, every coordinate zero or within [2^-100, 2^100)
     double vol_min = 0.0, vol_max = 0.0;
     bool vol_uniform = false;  // every particle has volume vol_value
     double vol_value = 0.0;
@@ -420,23 +420,18 @@ struct pdk_spec_s
             return 0;
         const int ev = std::ilogb( vol_min ), eh = std::min( std::ilogb( h_min ), 0 );
         const bool thermal = d.thermal != PDK_TEMP_INDEPENDENT && d.alpha != 0.0;
+        const int ec = lps() ? 0 : std::ilogb( c_min );
+        const int ea = thermal ? std::ilogb( d.alpha ) : 0, et = thermal && d.temp0 != 0.0 ? std::ilogb( d.temp0 ) : 400;
+        const int ey = plastic && k.s_Y != 0.0 ? std::ilogb( k.s_Y ) : 400;
         int low = 400;
         for ( ; low > 0; low-- )
         {
             int es = -55;
             if ( thermal )
-            {
-                es = std::min( -108, std::ilogb( d.alpha ) - low - 56 );
-                if ( d.temp0 != 0.0 )
-                    es = std::min( es, std::ilogb( d.alpha ) + std::ilogb( d.temp0 ) - 54 );
-            }
+                es = std::min( { -108, ea - low - 56, ea + et - 54 } );
             if ( plastic )
-            {
-                es = std::min( -108, es - 53 );
-                if ( k.s_Y != 0.0 )
-                    es = std::min( es, std::ilogb( k.s_Y ) - 54 );
-            }
-            const int ecoeff = lps() ? ev - 364 + 2 * eh : std::ilogb( c_min ) + ev + es - 2;
+                es = std::min( { -108, es - 53, ey - 54 } );
+            const int ecoeff = lps() ? ev - 364 + 2 * eh : ec + ev + es - 2;
             if ( ecoeff - ( low + 54 ) - 102 >= -960 )
                 break;
         }
@@ -1133,25 +1128,12 @@ int pdk_spec_upload( pdk_spec s, const double* x, const double* u, const double*
         // particle spacing (cube root of the mean volume).
         double lo[3] = { x[0], x[1], x[2] };
         double vsum = 0.0;
-        // magnitudes, for the FP64 row passes' arithmetic (plainLow)
-        double cmin = 1.0, cmax = 1.0, vmin = vol[0], vmax = vol[0];
         for ( int64_t i = 0; i < n; i++ )
         {
             for ( int dd = 0; dd < 3; dd++ )
-            {
-                const double c = x[3 * i + dd];
-                lo[dd] = std::min( lo[dd], c );
-                const double a = c == 0.0 ? 1.0 : std::fabs( c );
-                cmin = std::min( cmin, a );
-                cmax = std::max( cmax, a );
-            }
+                lo[dd] = std::min( lo[dd], x[3 * i + dd] );
             vsum += vol[i];
-            vmin = std::min( vmin, vol[i] );
-            vmax = std::max( vmax, vol[i] );
         }
-        s->coords_plain = cmin >= 0x1p-100 && cmax < 0x1p100;
-        s->vol_min = vmin;
-        s->vol_max = vmax;
         double h = std::cbrt( vsum / n );
         if ( !( h > 0 ) || !std::isfinite( h ) )
             h = 1.0;
@@ -1160,14 +1142,22 @@ int pdk_spec_upload( pdk_spec s, const double* x, const double* u, const double*
         // slot.  Other point sets use Morton order.
         std::vector<int64_t> lperm;
         bool lattice = false;
+        double smallest = 0.0, largest = 0.0;
         if ( s->d.ordering != PDK_ORDER_MORTON )
-            lattice = latticeOrder( x, n, lperm, s->lat_lo, s->lat_h, s->lat_dims, &s->lat_dev );
+            lattice = latticeOrder( x, n, lperm, s->lat_lo, s->lat_h, s->lat_dims, &s->lat_dev, &smallest, &largest );
         require( lattice || s->d.ordering != PDK_ORDER_LATTICE_ROWS, "positions do not form a lattice" );
         s->lattice_rows = lattice;
+        s->coords_plain = lattice && smallest >= 0x1p-100 && largest < 0x1p100;
         s->vol_uniform = true;
         s->vol_value = vol[0];
         for ( int64_t i = 1; i < n && s->vol_uniform; i++ )
             s->vol_uniform = vol[i] == vol[0];
+        s->vol_min = s->vol_max = vol[0];
+        for ( int64_t i = 1; i < n && !s->vol_uniform; i++ )
+        {
+            s->vol_min = std::min( s->vol_min, vol[i] );
+            s->vol_max = std::max( s->vol_max, vol[i] );
+        }
         s->any_nofail = false;
         if ( nofail )
             for ( int64_t i = 0; i < n && !s->any_nofail; i++ )

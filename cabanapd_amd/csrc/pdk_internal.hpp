@@ -191,9 +191,10 @@ void launchMortonOrder( const double* x_aos_dev, int64_t n, const double lo[3], 
 // order with x fastest.  dev_out: the largest distance of a position from
 // its site lo + k h along an axis, as a fraction of that axis' spacing, plus
 // the rounding of the site (stencil bond vectors differ from x_j - x_i by at
-// most twice that per axis).
+// most twice that per axis).  smallest_out, largest_out: the smallest nonzero
+// and the largest magnitude of a coordinate.
 bool latticeOrder( const double* x_aos_host, int64_t n, std::vector<int64_t>& perm, double lo_out[3],
-                   double h_out[3], int64_t dims_out[3], double* dev_out );
+                   double h_out[3], int64_t dims_out[3], double* dev_out, double* smallest_out, double* largest_out );
 // Stencil ids of a lattice specimen's bonds (mixed form); false when some
 // bond is not a lattice vector or the stencil has more than 255 entries.
 bool buildStencil( const PDArgs& a, const double h[3], double rc, int64_t total_rows, DevBuf& sid, DevBuf& table,
