@@ -1828,8 +1828,8 @@ ForceFn pickForceRowsFeat( const PDArgs& a )
 //   missing sites (a hole; 185, 510, 1054 and 2201 slices):
 //   FP64 PMB fracture   58/ 20/ 15    58/ 25/ 28    74/ 59/ 67    98/106/127
 //   mixed LPS fracture  82/ 35/ 25    82/ 38/ 38    84/ 84/ 88   104/148/164
-// Eight waves take a CU's LDS once (38 to 140 KB), so they serve up to 256
-// slices, where they won in every form.
+// Eight waves of a force pass take 87 to 140 KB of LDS and fit once on a CU, so
+// they serve up to 256 slices, where they won in every form.
 int splitWaves( const PDArgs& a, int64_t nslices )
 {
     if ( a.row_max > kSplitSlots )
