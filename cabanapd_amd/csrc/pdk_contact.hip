@@ -460,8 +460,8 @@ __global__ __launch_bounds__( kBlock ) void kContact( const PDArgs* __restrict__
 // VelocityVerlet<Contact>::initialHalfStep (CabanaPD_Integrate.hpp:154-193),
 // with FINAL preceded by the final half step of the step before (:128-134):
 // the half kicks, the drift into the other displacement buffer, the pair
-// records and the block maxima of |u - u_build|.
-template <bool FINAL>
+// records (REC) and the block maxima of |u - u_build|.
+template <bool FINAL, bool REC>
 __global__ __launch_bounds__( 256 ) void kContactAdvance( const PDArgs* __restrict__ specs, int32_t parity,
                                                           double* __restrict__ partial )
 {
@@ -491,7 +491,7 @@ __global__ __launch_bounds__( 256 ) void kContactAdvance( const PDArgs* __restri
             dd[d] = uu[d] - A.u_neigh[d * n + p];
         }
         mx = sqrt( dd[0] * dd[0] + dd[1] * dd[1] + dd[2] * dd[2] );
-        if ( A.rec_u )
+        if constexpr ( REC )
         {
             A.rec_u[p] = make_double4( uu[0], uu[1], uu[2], A.rho[p] * A.vol[p] );
             A.rec_v[p] = make_double4( vv[0], vv[1], vv[2], 0.0 );
@@ -662,8 +662,10 @@ void contactStep( pdk_spec_s* s, int32_t nsteps )
         specTimed( s, 4, [&] {
             const dim3 g( static_cast<unsigned>( nb ) );
             // the final half step of the step before rides along
-            hipLaunchKernelGGL( k == 0 ? kContactAdvance<false> : kContactAdvance<true>, g, dim3( 256 ), 0, v.st,
-                                v.dargs, *v.cur, part );
+            const bool records = v.h->rec_x != nullptr;
+            auto advance = k == 0 ? ( records ? kContactAdvance<false, true> : kContactAdvance<false, false> )
+                                  : ( records ? kContactAdvance<true, true> : kContactAdvance<true, false> );
+            hipLaunchKernelGGL( advance, g, dim3( 256 ), 0, v.st, v.dargs, *v.cur, part );
             hipLaunchKernelGGL( kMaxReduce, dim3( 1 ), dim3( 1024 ), 0, v.st, part, nb, cs.disp_dev );
             PDK_HIP( hipGetLastError() );
         } );
