@@ -717,7 +717,10 @@ __global__ __launch_bounds__( kThreads ) void kCheckHoleSlots( PDArgs a, Lattice
 // where the slice's own row has a gap that the neighbouring row fills (the
 // grips of a dogbone): place w holds id w + (w < y ? x : z) of its int4, w its
 // length.  Sets *flag where it is longer than the row passes stage (127 ids;
-// a place may reach one past the end).
+// a place may reach one past the end).  filled_sum: the slots that hold a bond
+// in some lane, as kFilledSums partial sums over the slices (one sum for all
+// would take 30 ns a slice in turn).
+constexpr int kFilledSums = 64, kFilledStride = 8; // 64 bytes apart
 __global__ __launch_bounds__( kThreads ) void kFillHoleSlots( int64_t n, int64_t nslices, LatticeBox L,
                                                               const int4* __restrict__ ent, int32_t S,
                                                               const int4* __restrict__ rows, int32_t nrows,
@@ -725,7 +728,8 @@ __global__ __launch_bounds__( kThreads ) void kFillHoleSlots( int64_t n, int64_t
                                                               const int32_t* __restrict__ id, int32_t* __restrict__ col,
                                                               uint64_t* __restrict__ exist,
                                                               uint64_t* __restrict__ intact, int4* __restrict__ hole_win,
-                                                              uint8_t* __restrict__ hole_pos, int32_t* __restrict__ flag )
+                                                              uint8_t* __restrict__ hole_pos, int32_t* __restrict__ flag,
+                                                              int64_t* __restrict__ filled_sum )
 {
     const int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     const int64_t slice = p / kSlice;
@@ -738,6 +742,7 @@ __global__ __launch_bounds__( kThreads ) void kFillHoleSlots( int64_t n, int64_t
         latticeCoords( site[p], L, ix, iy, iz );
     const int32_t self = static_cast<int32_t>( valid ? p : slice * kSlice );
     constexpr int32_t kNone = 0x7fffffff;
+    int32_t filled = 0; // slots with a bond
     for ( int32_t r = 0; r < nrows; r++ )
     {
         const int4 R = rows[r];
@@ -754,6 +759,7 @@ __global__ __launch_bounds__( kThreads ) void kFillHoleSlots( int64_t n, int64_t
                 exist[slice * S + e] = m;
                 intact[slice * S + e] = m;
             }
+            filled += m != 0 ? 1 : 0;
             if ( ex )
             {
                 first = min( first, j );
@@ -804,6 +810,9 @@ __global__ __launch_bounds__( kThreads ) void kFillHoleSlots( int64_t n, int64_t
         if ( lane == 0 )
             hole_win[slice * nrows + r] = make_int4( g, len1, g2 - len1, len );
     }
+    if ( lane == 0 )
+        atomicAdd( reinterpret_cast<unsigned long long*>( filled_sum + slice % kFilledSums * kFilledStride ),
+                   static_cast<unsigned long long>( filled ) );
 }
 
 // ---- Bond state from one form to the other -----------------------------------
@@ -1353,6 +1362,8 @@ std::vector<int4> slotEntries( const std::vector<SlotEntry>& es )
 // the FP64 |xi|^2 of each entry, and move them into place.
 // With site and id (missing sites) also the windows; false, with nothing
 // moved, when they do not fit the row passes.
+// most_filled: so many slots with a bond per row of the compact form at most,
+// else false as well.
 // With bond_state also one double per bond slot.  keep_room (a compact form is
 // there and would do): MemError, with nothing moved, unless the budget then
 // still has what later calls on this specimen may allocate (stress tensors and
@@ -1361,7 +1372,8 @@ bool finishSlots( int64_t n, int64_t nslices, const LatticeBox& L, const std::ve
                   const int4* dent, const double h[3], DevBuf& col, DevBuf& intact, int64_t* slice_ptr_dev,
                   int64_t& total_rows, int64_t& col_capacity_rows, SlotForm& out, MemAccount* acct,
                   hipStream_t st, const int32_t* site = nullptr, const int32_t* id = nullptr,
-                  int32_t* flag_dev = nullptr, DevBuf* bond_state = nullptr, bool keep_room = false )
+                  int32_t* flag_dev = nullptr, DevBuf* bond_state = nullptr, bool keep_room = false,
+                  double most_filled = 0.0 )
 {
     const int32_t S = static_cast<int32_t>( es.size() );
     const int64_t rows = nslices * S;
@@ -1408,15 +1420,20 @@ bool finishSlots( int64_t n, int64_t nslices, const LatticeBox& L, const std::ve
     {
         nwin.alloc( static_cast<size_t>( nslices ) * nrows * sizeof( int4 ), acct );
         npos.alloc( static_cast<size_t>( nslices ) * nrows * kSlice, acct );
-        PDK_HIP( hipMemsetAsync( flag_dev, 0, sizeof( int32_t ), st ) );
+        // (flag_dev: the sums, and the flag between the first and the second)
+        int64_t sums[kFilledSums * kFilledStride];
+        PDK_HIP( hipMemsetAsync( flag_dev, 0, sizeof sums, st ) );
         kFillHoleSlots<<<gridFor( nslices * kSlice ), kThreads, 0, st>>>(
             n, nslices, L, dent, S, drows.as<int4>(), nrows, site, id, ncol.as<int32_t>(), nexist.as<uint64_t>(),
-            nintact.as<uint64_t>(), nwin.as<int4>(), npos.as<uint8_t>(), flag_dev );
+            nintact.as<uint64_t>(), nwin.as<int4>(), npos.as<uint8_t>(), flag_dev + 2,
+            reinterpret_cast<int64_t*>( flag_dev ) );
         PDK_HIP( hipGetLastError() );
-        int32_t flag = 0;
-        PDK_HIP( hipMemcpyAsync( &flag, flag_dev, sizeof( int32_t ), hipMemcpyDeviceToHost, st ) );
+        PDK_HIP( hipMemcpyAsync( sums, flag_dev, sizeof sums, hipMemcpyDeviceToHost, st ) );
         PDK_HIP( hipStreamSynchronize( st ) );
-        if ( flag )
+        int64_t filled = 0;
+        for ( int i = 0; i < kFilledSums; i++ )
+            filled += sums[i * kFilledStride];
+        if ( sums[1] || static_cast<double>( filled ) > most_filled * static_cast<double>( total_rows ) )
             return false;
     }
     else
@@ -1569,6 +1586,37 @@ bool buildStencilSlots( const PDArgs& a, const int64_t dims[3], const double h[3
                         col_capacity_rows, out, acct, st, nullptr, nullptr, nullptr, bond_state, true );
 }
 
+// Up to how many slots with a bond per row of the compact form the slot form is
+// the faster one: where many sites are missing at random, a wavefront's lanes
+// have their bonds in different slots, and the row passes go through all of them
+// with few lanes live.  Measured, slot form against compact form, boxes with a
+// fraction of the sites filled at random, 122 slots; ratio 3.7 / 2.6 / 2.05 / 1.7 / 1.4:
+//   PMB FP64, 64^3     +48 % /  +13 % / +11 % /  -3 % / -17 %  (materials alike)
+//   PMB mixed          +13   /  -15   / -35   / -41   / -44
+//   LPS FP64           +27   /   -5   / -11   / -23   / -35
+//   LPS mixed          -29   /  -43   / -62   / -64   / -72
+//   plastic FP64       +73   /  +26   / +36   / +25   /  -4
+//   heat every 2 steps +111  /  +63   / +48   / +28   /  +3
+// Up to 384 slices (8 or 4 waves share each) the steps gain at every ratio (PMB
+// FP64 -19 % at 3.7 and 266 slices), heat up to a ratio of 2.
+double mostFilled( const PDArgs& a, bool plastic )
+{
+    const double any = std::numeric_limits<double>::infinity();
+    const bool small = a.nslices <= 384;
+    if ( a.nslices <= 32 )
+        return any;
+    if ( a.cond )
+        return small ? 2.0 : 1.4;
+    if ( small )
+        return any;
+    if ( plastic )
+        return 1.4;
+    const bool mixed = a.precision == PDK_MIXED;
+    if ( a.model == PDK_MODEL_LPS )
+        return mixed ? any : 2.1;
+    return mixed ? 2.4 : 1.75;
+}
+
 bool buildHoleSlots( const PDArgs& a, const int64_t dims[3], const double lo[3], const double h[3], double rc,
                      const std::vector<int64_t>& perm_host, DevBuf& col, DevBuf& intact, int64_t* slice_ptr_dev,
                      int64_t& total_rows, int64_t& col_capacity_rows, SlotForm& out, BuildScratch& s, MemAccount* acct,
@@ -1593,7 +1641,7 @@ bool buildHoleSlots( const PDArgs& a, const int64_t dims[3], const double lo[3],
     dent.alloc( S * sizeof( int4 ), acct );
     site.alloc( n * sizeof( int32_t ), acct );
     id.alloc( box * sizeof( int32_t ), acct );
-    ensure<int32_t>( s.flag, 1, acct );
+    ensure<int64_t>( s.flag, kFilledSums * kFilledStride, acct );
     PDK_HIP( hipMemcpyAsync( dent.as<int4>(), ent.data(), S * sizeof( int4 ), hipMemcpyHostToDevice, st ) );
     PDK_HIP( hipMemsetAsync( s.flag.as<int32_t>(), 0, sizeof( int32_t ), st ) );
     PDK_HIP( hipMemsetAsync( id.as<int32_t>(), 0xff, box * sizeof( int32_t ), st ) );
@@ -1609,7 +1657,7 @@ bool buildHoleSlots( const PDArgs& a, const int64_t dims[3], const double lo[3],
         return false;
     return finishSlots( n, a.nslices, L, es, dent.as<int4>(), h, col, intact, slice_ptr_dev, total_rows,
                         col_capacity_rows, out, acct, st, site.as<int32_t>(), id.as<int32_t>(),
-                        s.flag.as<int32_t>(), bond_state, true );
+                        s.flag.as<int32_t>(), bond_state, true, mostFilled( a, bond_state != nullptr ) );
 }
 
 bool buildStencilSlotsDirect( const double* x_dev, int64_t n, const int64_t dims[3], const double h[3], double rc,

@@ -280,11 +280,12 @@ def test_lines_of_split_launches(kind, short, hole, precision):
     form and the precision: on both sides of each line, the gathers' bits."""
     line = LINES[kind, short, hole][precision]
     for slices, waves in ((line, 4), (line + 1, 1)):
-        # layers of 8 x 8 = 64 particles; the holes' layers have 4 sites more
-        dims = (9, 8, slices) if hole else (8, 8, slices)
+        # layers of 8 x 8 = 64 particles; with a hole wider ones, cut off after
+        # so many particles
+        dims = (33, 32, slices // 14 + 2) if hole else (8, 8, slices)
         w = box("LPS" if kind in ("lps", "materials") else "PMB", dims, 1.5 if short else 3.01, True)
         if hole:
-            cut(w, dims, lambda i, j, k: (i != 4) | (j == 0))
+            cut(w, dims, lambda i, j, k: (i - 16) ** 2 + (j - 15) ** 2 > 36)
             for key in ("x", "vol", "rho", "u", "v"):
                 w[key] = np.ascontiguousarray(w[key][:64 * slices])
         d = w["desc"]
@@ -469,3 +470,48 @@ def test_spec_bytes_hold_the_forms_tables(precision):
         say(f"case: precision {precision}, {w['x'].shape[0]} particles: held {held}, in use {used}")
         assert held[0] != held[1]
         assert abs((held[0] - held[1]) - (used[0] - used[1])) <= 4096
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("kind,most", [("pmb", (1.75, 2.4)), ("lps", (2.1, np.inf)), ("epp", (1.4, 1.4)),
+                                       ("heat", (1.4, 1.4))])
+def test_sparse_lattices_take_the_faster_form(kind, most, precision):
+    """Large boxes with sites missing at random: the slot form where its slots
+    with a bond are at most so many per row of the compact form, the compact
+    form beyond (its row passes would run with few lanes live); the same bits."""
+    dims = (60, 60, 40)
+    seen = set()
+    for fill in (0.2, 0.45, 0.6, 0.75):
+        w = box("LPS" if kind == "lps" else "PMB", dims, 3.01, kind != "heat")
+        cut(w, dims, lambda i, j, k: np.random.default_rng(9).random(i.size) < fill)
+        d = w["desc"]
+        n = w["x"].shape[0]
+        if kind == "epp":
+            d.mechanics, d.sigma_y = 1, 2.5e7
+        if kind == "heat":
+            d.thermal, d.alpha, d.temp0, d.kappa, d.cp, d.thermal_subcycle = 2, 1e-6, 20.0, 10.0, 1.0, 2
+            w["temperature"] = 20.0 + 40.0 * np.random.default_rng(6).random(n)
+        d.precision = precision
+        out = []
+        for layout in (0, PDK_BONDS_COMPACT):
+            d.bond_layout = layout
+            s = engine.Spec(ctx(), d, n)
+            configs.upload(s, w)
+            configs.setup(s, w)
+            s.step(3)
+            out.append(s.bonds() + (s.get("u"), s.kernel_name(0)))
+            s.close()
+        slices = (n + 63) // 64
+        cnt = np.pad(np.diff(out[0][0]), (0, slices * 64 - n)).reshape(slices, 64)
+        ratio = 122 * slices / cnt.max(1).sum()  # every slot has a bond in some lane here
+        rows = "Rows" in out[0][4]
+        say(f"case: {kind} precision {precision} fill {fill}: {slices} slices, {ratio:.2f} slots a row, {out[0][4]}")
+        assert rows == (ratio <= most[precision])
+        seen.add(rows)
+        for b in range(3):
+            assert np.array_equal(out[0][b], out[1][b])
+        if precision == 0:
+            assert np.array_equal(out[0][3], out[1][3])
+        else:
+            assert rel_err(out[0][3], out[1][3]) <= 1e-6
+    assert True in seen
