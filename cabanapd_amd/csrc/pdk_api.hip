@@ -1468,6 +1468,27 @@ int pdk_prenotch( pdk_spec s, int32_t nn, const double* p0, const double* v1, co
     } );
 }
 
+} // extern "C"
+
+namespace
+{
+// A 64 x 64 bit matrix transposed in place: blocks of half the size change
+// places across the diagonal, down to single bits.
+void transposeBits( uint64_t* row )
+{
+    uint64_t low = 0xffffffffull;
+    for ( int half = 32; half; half /= 2, low ^= low << half )
+        for ( int i = 0; i < 64; i++ )
+            if ( !( i & half ) )
+            {
+                const uint64_t swap = ( ( row[i] >> half ) ^ row[i + half] ) & low;
+                row[i] ^= swap << half;
+                row[i + half] ^= swap;
+            }
+}
+} // namespace
+
+extern "C" {
 int pdk_download_bonds( pdk_spec s, int64_t capacity, int64_t* offsets, int64_t* nbr, uint8_t* intact )
 {
     return guarded( [&] {
@@ -1501,6 +1522,19 @@ int pdk_download_bonds( pdk_spec s, int64_t capacity, int64_t* offsets, int64_t*
         for ( int32_t v : c )
             sum += v;
         require( ( !nbr && !intact ) || sum <= capacity, "pdk_download_bonds: capacity is smaller than the bond count" );
+        // Stencil-slot form: each lane's slots with a bond as a bit row, from the
+        // exist words (asking every slot of every particle took up to nine times
+        // as long where many sites are missing).
+        const int64_t words = slots && ns ? ( sp[1] - sp[0] + kSlice - 1 ) / kSlice : 0;
+        std::vector<uint64_t> live( static_cast<size_t>( ns ) * words * kSlice );
+        for ( int64_t slice = 0; slice < ns && slots; slice++ )
+            for ( int64_t w = 0; w < words; w++ )
+            {
+                uint64_t* t = live.data() + ( slice * words + w ) * kSlice;
+                const int64_t row = sp[slice] + w * kSlice;
+                std::copy( ex.begin() + row, ex.begin() + std::min<int64_t>( row + kSlice, sp[slice + 1] ), t );
+                transposeBits( t );
+            }
         int64_t off = 0;
         for ( int64_t cid = 0; cid < n; cid++ )
         {
@@ -1508,22 +1542,23 @@ int pdk_download_bonds( pdk_spec s, int64_t capacity, int64_t* offsets, int64_t*
             const int64_t slice = p / kSlice, lane = p % kSlice;
             if ( offsets )
                 offsets[cid] = off;
-            // compact form: slots [0, cnt); stencil-slot form: every slot of
-            // the row whose exist bit is set, in slot order
-            const int64_t qend = slots ? sp[slice + 1] - sp[slice] : c[p];
             int64_t k = 0;
-            for ( int64_t q = 0; q < qend; q++ )
-            {
-                const int64_t row = sp[slice] + q;
-                if ( slots && !( ( ex[row] >> lane ) & 1ull ) )
-                    continue;
-                require( k < c[p], "pdk_download_bonds: inconsistent bond rows" );
+            const auto put = [&]( int64_t row ) {
                 if ( nbr )
                     nbr[off + k] = s->h_perm[col[row * kSlice + lane]];
                 if ( intact )
                     intact[off + k] = static_cast<uint8_t>( ( bits[row] >> lane ) & 1ull );
                 k++;
-            }
+            };
+            // compact form: slots [0, cnt)
+            while ( !slots && k < c[p] )
+                put( sp[slice] + k );
+            for ( int64_t w = 0; w < words; w++ )
+                for ( uint64_t m = live[( slice * words + w ) * kSlice + lane]; m; m &= m - 1 )
+                {
+                    require( k < c[p], "pdk_download_bonds: inconsistent bond rows" );
+                    put( sp[slice] + w * kSlice + __builtin_ctzll( m ) );
+                }
             require( k == c[p], "pdk_download_bonds: inconsistent bond rows" );
             off += c[p];
         }
