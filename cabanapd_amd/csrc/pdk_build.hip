@@ -718,8 +718,9 @@ __global__ __launch_bounds__( kThreads ) void kCheckHoleSlots( PDArgs a, Lattice
 // grips of a dogbone): place w holds id w + (w < y ? x : z) of its int4, w its
 // length.  Sets *flag where it is longer than the row passes stage (127 ids;
 // a place may reach one past the end).  filled_sum: the slots that hold a bond
-// in some lane, as kFilledSums partial sums over the slices (one sum for all
-// would take 30 ns a slice in turn).
+// in some lane, as kFilledSums partial sums over the slices (so that the
+// slices' atomic adds do not all wait on one address; no difference measured on
+// a specimen of 423 thousand particles).
 constexpr int kFilledSums = 64, kFilledStride = 8; // 64 bytes apart
 __global__ __launch_bounds__( kThreads ) void kFillHoleSlots( int64_t n, int64_t nslices, LatticeBox L,
                                                               const int4* __restrict__ ent, int32_t S,
